@@ -169,17 +169,22 @@ __device__ __forceinline__ double add_xor32(double v) {
 // half of the double-buffered LDS, so the HBM stream has no idle phase
 // between units.
 //
-// rev = 1 runs the same schedule over the units in reverse order (unit u
-// becomes njobs - 1 - u).  The stages of a step alternate directions, so
-// each launch starts on the part of the store the previous launch read
-// last, which the device's 256 MB memory-side cache still holds; the
-// loads are ordinary (cache-allocating) loads for that reason.  Every unit
-// writes its own partial slots, so the order changes no result bit.
-// Measured per launch, against non-temporal loads in one direction: He
-// 4 x 4000 (384 MB) 64.6 us against 65.7 us, 4 x 3500 (294 MB) 48.7 us
-// against 52.3 us, the He_test.yaml shape (194 MB) 32.2 us against
-// 33.4 us.  Ordinary loads without the alternation lose on the 384 MB
-// store (71.9 us): each launch then evicts what the next one needs first.
+// rev = 1 runs the workgroup's own units last to first, and the row groups
+// of each unit bottom to top.  The stages of a step alternate directions, so
+// each launch starts on the bytes the previous launch read last, and on the
+// same workgroup, hence (workgroups go to the 8 XCDs round-robin) on the
+// same XCD, whose 4 MB L2 still holds them.  Reads that miss L2 run at
+// 6.9 TB/s at most here, whether the 256 MB memory-side cache or HBM serves
+// them (streaming probe, 96 to 768 MiB), so only L2 hits save time: the
+// same probe reads 24 MiB in 2.6 us with this order, 4.9 us when the
+// reversed sweep mirrors the units over the whole grid (another XCD each
+// time), 96 MiB in 11.6 against 15.1 us, 384 MiB in 57.2 against 61.9 us.
+// This kernel, per launch, against the mirrored order: He 4 x 4000
+// (384 MB) 64.5 against 65.3 us, the He_test.yaml shape (194 MB) 31.6
+// against 32.1 us, 4 x 2000 (96 MB) 18.2 against 19.5 us, 4 x 1500 (54 MB)
+// 11.2-11.9 against 13.1 us.  Ordinary (cache-allocating) loads, as the
+// retained bytes have to be.  Every unit writes its own partial slots; a
+// unit's column sums run over its rows in the sweep's direction.
 // ---------------------------------------------------------------------
 namespace {
 struct UnitGeo {
@@ -209,11 +214,15 @@ __global__ __launch_bounds__(kGvThreads) void k_gemv_tile(
     const Ctl *__restrict__ ctl, int rev) {
   const SysDesc &d = *dp;
   if (ctl[0].done) return;
-  // store position of the workgroup's sweep unit x (x < njobs)
-  auto phys = [&](int x) { return rev ? njobs - 1 - x : x; };
   const int G = gridDim.x;
-  int u = blockIdx.x;
-  if (u >= njobs) return;
+  if ((int)blockIdx.x >= njobs) return;
+  // the workgroup's units blockIdx.x, blockIdx.x + G, ... in sweep order
+  const int nu = (njobs - (int)blockIdx.x + G - 1) / G;
+  auto unit = [&](int k) {
+    return (int)blockIdx.x + (rev ? nu - 1 - k : k) * G;
+  };
+  // row group visited i-th in a unit of nI groups
+  auto group = [&](int i, int nI) { return rev ? nI - 1 - i : i; };
   const int t = threadIdx.x;
   const int tr = t & 15, g = t >> 4, lane = t & 63, w = t >> 6;
 
@@ -256,16 +265,17 @@ __global__ __launch_bounds__(kGvThreads) void k_gemv_tile(
           (q.col0 + c < q.sL1) ? x1[q.col0 + c] : make_double2(0.0, 0.0);
   };
 
-  UnitGeo q = unit_geo(jobs, phys(u), d);
+  int u = unit(0);
+  UnitGeo q = unit_geo(jobs, u, d);
   dv2 cur[kGvColPairIter], nxt[kGvColPairIter];
-  load_group(phys(u), 0, q.nrows, q.col0, q.sL1, cur);
+  load_group(u, group(0, q.nI), q.nrows, q.col0, q.sL1, cur);
   stage_x(q, 0);
   __syncthreads();
   int b = 0;
-  for (;;) {
-    const int un = u + G;
-    const bool more = un < njobs;  // uniform over the workgroup
-    const UnitGeo qn = more ? unit_geo(jobs, phys(un), d) : q;
+  for (int k = 0;; ++k) {
+    const bool more = k + 1 < nu;  // uniform over the workgroup
+    const int un = more ? unit(k + 1) : u;
+    const UnitGeo qn = more ? unit_geo(jobs, un, d) : q;
     // Stage the next unit's x into the other LDS half now: its loads are
     // waited for together with this unit's first row group, which the
     // first iteration needs anyway.  That half was last read before the
@@ -304,18 +314,17 @@ __global__ __launch_bounds__(kGvThreads) void k_gemv_tile(
     };
     // groups 0 .. nI-2: the next group of this unit is in flight meanwhile
     for (int i = 0; i + 1 < q.nI; ++i) {
-      load_group(phys(u), i + 1, q.nrows, q.col0, q.sL1, nxt);
-      consume(i, cur);
+      load_group(u, group(i + 1, q.nI), q.nrows, q.col0, q.sL1, nxt);
+      consume(group(i, q.nI), cur);
 #pragma unroll
       for (int j = 0; j < kGvColPairIter; ++j) cur[j] = nxt[j];
     }
     // last group: the next unit's first group goes into flight (after the
     // workgroup's last unit, this group again: a cache hit) and stays in
     // flight through the epilogue
-    load_group(phys(more ? un : u), more ? 0 : q.nI - 1,
-               more ? qn.nrows : q.nrows, more ? qn.col0 : q.col0,
-               more ? qn.sL1 : q.sL1, nxt);
-    consume(q.nI - 1, cur);
+    load_group(un, group(more ? 0 : q.nI - 1, qn.nI), qn.nrows, qn.col0,
+               qn.sL1, nxt);
+    consume(group(q.nI - 1, q.nI), cur);
 
     // ---- epilogue of unit u (the next unit's first group is in flight)
     // column partials: sum over the 16 row lanes (lane bits 0..3)
