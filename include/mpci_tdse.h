@@ -252,8 +252,16 @@ int mpci_prop_observables(mpci_prop *prop, int electrons, double threshold,
                           double *out);
 
 /* Launch the 13-stage step as one captured hipGraph (1, default) or as
- * individual launches (0). */
+ * individual launches (0).  With 1, one pulse on a system whose dipoles take
+ * at most 24 MiB runs its attempts inside one cooperative launch instead,
+ * with the bits of the fused small-system stages (below). */
 int mpci_prop_set_graph(mpci_prop *prop, int enable);
+/* The workgroups of that launch wait for one another; a wait is given up
+ * after `ms` milliseconds (0: the default of 20000; negative: at once), for
+ * instance when other work holds part of the device for that long.  The run
+ * then goes back to where the launch began and goes on with one launch per
+ * stage. */
+int mpci_prop_set_wait_limit(mpci_prop *prop, int ms);
 /* One pulse on a small system: each stage as one fused launch (coupling
  * from row-major copies of D_L and D_L^T, one wave per row, then the stage
  * algebra) instead of the GEMV tile kernel and the stage kernel.  mode -1

@@ -69,6 +69,30 @@ constexpr int kPrR = 256;
 constexpr int kPrTK = 16;
 constexpr int kPrTN = 32;
 
+// ---- row form (one pulse): every row of the operator owned by one place --
+// Rows are taken four at a time (a quad).  The row store Dq holds, per quad,
+// the concatenated columns [D_{L-1}^T | D_L] of its four rows in chunks of
+// 64 columns (each of the two parts padded with zeros to whole chunks):
+// element (chunk c, row r, column j) sits at ((c * 2 + r / 2) * 64 + j) * 2
+// + r % 2, so one 16-byte load per lane carries two rows of one column.
+constexpr int kRwQuad = 4;
+constexpr int kRwThreads = 512;  // persistent form: eight waves,
+constexpr int kRwCompute = 4;    // four compute, four poll
+constexpr int kRwReg = 16;       // chunks of a wave's first quad in registers
+constexpr int kRwMaxRows = 64;   // rows of a workgroup
+
+struct RowDesc {
+  long long q_off[kMaxBlocks];  // block L's first quad in Dq (doubles)
+  int quad0[kMaxBlocks + 1];    // block L's first quad in the quad order
+};
+
+// One workgroup of the persistent row kernel: rows row0 .. row0 + nrows - 1
+// of block L, its first quad's number, and how many chunks of each quad it
+// keeps in LDS.
+struct RowWg {
+  int L, row0, nrows, quad0, nlds, pad;
+};
+
 // Per-propagator description of the blocks and the partial-sum buffers.
 struct SysDesc {
   int nb;

@@ -100,12 +100,10 @@ struct mpci_system {
   DevBuf<double> Dr;
   DevBuf<long long> dr_off;
   std::vector<int> dr_ld;  // even row stride of each block in Dr
-  DevBuf<int> dr_ld_d;     // the same on the device
-  // row-major D_L^T (s_{L+1} x s_L) of every pair, for the single-pulse
-  // small-system path, built with it
-  DevBuf<double> DrT;
-  DevBuf<long long> drt_off;
-  DevBuf<int> drt_ld_d;
+  // row store of the single-pulse row form (RowDesc), built on its first use
+  DevBuf<double> Dq;
+  DevBuf<RowDesc> drow;
+  RowDesc hrow{};
   std::vector<std::vector<double>> hostD;
   // the energies as given, for the observable weights (pes's masks)
   std::vector<std::vector<double>> hostE;
@@ -130,7 +128,15 @@ struct mpci_prop {
   // one pulse on a small system: one fused launch per stage
   // (k_small_stage, four rows per workgroup) instead of GEMV tile + stage
   bool small = false;
-  int nblk_small = 0;
+  int nblk_small = 0;  // quads: partials of its step control
+  // one pulse, whole runs in one cooperative launch (k_rows_run)
+  bool rows = false;
+  int rows_wg = 0;       // workgroups
+  size_t rows_lds = 0;   // dynamic LDS bytes
+  int rows_kq = 1;       // quads per computing wave
+  int wait_limit_ms = 0; // time limit of one wait inside the launch
+  DevBuf<RowWg> rwg;
+  DevBuf<double2> xb, rb;  // exchange buffers
   DevBuf<double2> X, Xs, K, Y, part;
   DevBuf<double2> xstage;  // one pulse's contiguous state (set/get_state)
   DevBuf<double2> Xs2;  // second stage-input buffer of the fused path
@@ -540,9 +546,6 @@ static int ensure_rowmajor(mpci_system *sys) {
   }
   TRY(sys->Dr.alloc(tot));
   TRY(sys->dr_off.alloc(off.size()));
-  TRY(sys->dr_ld_d.alloc(off.size()));
-  HIPCHK(hipMemcpy(sys->dr_ld_d.p, sys->dr_ld.data(),
-                   sizeof(int) * off.size(), hipMemcpyHostToDevice));
   HIPCHK(hipMemset(sys->Dr.p, 0, sizeof(double) * tot));
   HIPCHK(hipMemcpy(sys->dr_off.p, off.data(), sizeof(long long) * off.size(),
                    hipMemcpyHostToDevice));
@@ -555,34 +558,42 @@ static int ensure_rowmajor(mpci_system *sys) {
   return MPCI_OK;
 }
 
-// Row-major D_L^T of every pair (row stride s_L) for k_small_stage.
-static int ensure_transposed(mpci_system *sys) {
-  if (sys->DrT.p || sys->nb < 2) return MPCI_OK;
-  std::vector<long long> off(sys->nb - 1);
-  std::vector<int> ld(sys->nb - 1);
+// Columns of block L's rows in the row store, in chunks of 64 (its lower and
+// its upper neighbour padded separately).
+static int row_chunks(const mpci_system *sys, int L) {
+  const int n0 = L > 0 ? sys->s[L - 1] : 0;
+  const int n1 = L + 1 < sys->nb ? sys->s[L + 1] : 0;
+  return (n0 + 63) / 64 + (n1 + 63) / 64;
+}
+
+// The row store (RowDesc), built on the device from the GEMV store.
+static int ensure_rows(mpci_system *sys) {
+  if (sys->Dq.p || sys->nb < 2) return MPCI_OK;
+  RowDesc r{};
   long long tot = 0;
-  for (int L = 0; L + 1 < sys->nb; ++L) {
-    ld[L] = sys->s[L];
-    off[L] = tot;
-    tot += (long long)sys->s[L + 1] * sys->s[L];
+  for (int L = 0; L < sys->nb; ++L) {
+    const int nq = (sys->s[L] + kRwQuad - 1) / kRwQuad;
+    r.q_off[L] = tot;
+    r.quad0[L + 1] = r.quad0[L] + nq;
+    tot += (long long)nq * row_chunks(sys, L) * 64 * kRwQuad;
   }
-  std::vector<double> h((size_t)tot);
-  for (int L = 0; L + 1 < sys->nb; ++L) {
-    const int a = sys->s[L], b = sys->s[L + 1];
-    const double *D = sys->hostD[L].data();
-    double *T = h.data() + off[L];
-    for (int i = 0; i < a; ++i)
-      for (int j = 0; j < b; ++j) T[(size_t)j * a + i] = D[(size_t)i * b + j];
+  DevBuf<RowDesc> dr;
+  DevBuf<double> q;
+  TRY(dr.alloc(1));
+  TRY(q.alloc((size_t)tot));
+  HIPCHK(hipMemcpy(dr.p, &r, sizeof(r), hipMemcpyHostToDevice));
+  for (int L = 0; L < sys->nb; ++L) {
+    const long long n =
+        (L + 1 < sys->nb ? r.q_off[L + 1] : tot) - r.q_off[L];
+    hipLaunchKernelGGL(k_relayout_rows, dim3((unsigned)((n + 255) / 256)),
+                       dim3(256), 0, 0, sys->Dg.p, sys->ddesc1.p, dr.p,
+                       (int)sys->jobs.size(), L, n, q.p);
+    HIPCHK(hipGetLastError());
   }
-  TRY(sys->DrT.alloc(tot));
-  TRY(sys->drt_off.alloc(off.size()));
-  TRY(sys->drt_ld_d.alloc(ld.size()));
-  HIPCHK(hipMemcpy(sys->DrT.p, h.data(), sizeof(double) * tot,
-                   hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(sys->drt_off.p, off.data(), sizeof(long long) * off.size(),
-                   hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(sys->drt_ld_d.p, ld.data(), sizeof(int) * ld.size(),
-                   hipMemcpyHostToDevice));
+  HIPCHK(hipDeviceSynchronize());
+  sys->hrow = r;
+  sys->drow.swap(dr);
+  sys->Dq.swap(q);
   return MPCI_OK;
 }
 
@@ -914,21 +925,105 @@ static int autotune_gemm(mpci_prop *pr) {
 // on four equal blocks: 1.95x the tile path at 0.9 MB of dipoles, 1.30x at
 // 8.6 MB, even at 15 MB, 0.85x at 24 MB.
 constexpr long long kSmallPathBytes = 12LL << 20;
+// The same for whole runs in one persistent launch (k_rows_run): past it the
+// row store no longer stays on the chip (registers and LDS of the workgroups,
+// then L2).  Per attempt against the tile path, four equal blocks: 0.9 MB
+// 31.6 against 83 us, 6 MB 37.9 against 116 us, 19.4 MB 78 against 164 us,
+// 31.7 MB and beyond see the table in k_rows_run's comment.
+constexpr long long kRowsBytes = 24LL << 20;
+constexpr int kWaitLimitMs = 20000;  // time limit of one wait in k_rows_run
+
+// The workgroups of the persistent row kernel: at most one per compute unit,
+// each inside one block, 16 rows (one pass of its four quads) while that
+// fits the device, else dealt to the blocks by the elements of their rows.
+// Returns false when the form does not apply to the system.
+static bool plan_rows(const mpci_prop *pr, std::vector<RowWg> &wg,
+                      size_t *lds, int *kq) {
+  const mpci_system *sys = pr->sys;
+  wg.clear();
+  if (pr->P != 1 || sys->nb < 2 || 64LL * sys->N >= (1LL << 31)) return false;
+  int coop = 0, lds_max = 0;
+  if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch,
+                            sys->device) != hipSuccess || !coop)
+    return false;
+  if (hipDeviceGetAttribute(&lds_max,
+                            hipDeviceAttributeMaxSharedMemoryPerBlock,
+                            sys->device) != hipSuccess)
+    return false;
+  // the kernel's static LDS: the control record and the reduction arrays
+  const long long room = (long long)lds_max - 4096 - 2048;
+  std::vector<int> rpw(sys->nb);
+  long long n16 = 0, cost = 0;
+  for (int L = 0; L < sys->nb; ++L) {
+    n16 += (sys->s[L] + 15) / 16;
+    cost += (long long)sys->s[L] * row_chunks(sys, L);
+  }
+  for (int L = 0; L < sys->nb; ++L) {
+    rpw[L] = 16;
+    if (n16 > sys->ncu) {
+      const double share = (double)(sys->ncu - sys->nb) *
+                           ((double)sys->s[L] * row_chunks(sys, L)) /
+                           (double)cost;
+      rpw[L] = (int)std::ceil(sys->s[L] / std::max(share, 1.0));
+      rpw[L] = (rpw[L] + kRwQuad - 1) / kRwQuad * kRwQuad;
+    }
+    if (rpw[L] > kRwMaxRows) return false;
+  }
+  const int rmax = *std::max_element(rpw.begin(), rpw.end());
+  *kq = rmax <= 16 ? 1 : rmax <= 32 ? 2 : 4;
+  const int reg = *kq == 1 ? kRwReg : 0;
+  *lds = 0;
+  for (int L = 0; L < sys->nb; ++L) {
+    const int nch = row_chunks(sys, L);
+    for (int r = 0; r < sys->s[L]; r += rpw[L]) {
+      RowWg g{};
+      g.L = L;
+      g.row0 = r;
+      g.nrows = std::min(rpw[L], sys->s[L] - r);
+      g.quad0 = sys->hrow.quad0[L] + r / kRwQuad;
+      const int nq = (g.nrows + kRwQuad - 1) / kRwQuad;
+      const long long base = 2LL * ((nch + 3) / 4 * 4) * 64 * 16 +
+                             kStages * nq * kRwQuad * 16LL;
+      if (base > room) return false;
+      g.nlds = (int)std::min<long long>(std::max(nch - reg, 0),
+                                        (room - base) / (nq * 2048LL));
+      *lds = std::max<size_t>(*lds, base + g.nlds * nq * 2048LL);
+      wg.push_back(g);
+    }
+  }
+  return (int)wg.size() <= sys->ncu;
+}
 
 // mode -1: automatic (one pulse, more than one block, 8 S within
 // kSmallPathBytes); 0: off; 1: on wherever it applies (one pulse, more
 // than one block).
 static int apply_small_path(mpci_prop *pr, int mode) {
   mpci_system *sys = pr->sys;
-  bool on = false;
-  if (pr->P == 1 && sys->nb > 1)
+  bool on = false, rows = false;
+  if (pr->P == 1 && sys->nb > 1) {
     on = mode == 1 || (mode < 0 && 8 * sys->S <= kSmallPathBytes);
-  if (on) {
-    TRY(ensure_rowmajor(sys));
-    TRY(ensure_transposed(sys));
-    if (!pr->Xs2.p) TRY(pr->Xs2.alloc(pr->NP));
+    rows = mode == 1 || (mode < 0 && 8 * sys->S <= kRowsBytes);
+  }
+  if (on || rows) {
+    TRY(ensure_rows(sys));
+    pr->nblk_small = sys->hrow.quad0[sys->nb];
+  }
+  if (on && !pr->Xs2.p) TRY(pr->Xs2.alloc(pr->NP));
+  if (rows && !pr->rwg.p) {
+    std::vector<RowWg> wg;
+    rows = plan_rows(pr, wg, &pr->rows_lds, &pr->rows_kq);
+    if (rows) {
+      TRY(pr->xb.alloc(4 * (size_t)sys->N));
+      TRY(pr->rb.alloc(3 * (size_t)sys->hrow.quad0[sys->nb]));
+      DevBuf<RowWg> d;
+      TRY(d.alloc(wg.size()));
+      TRY(h2d(pr, d.p, wg.data(), sizeof(RowWg) * wg.size()));
+      pr->rwg.swap(d);
+      pr->rows_wg = (int)wg.size();
+    }
   }
   pr->small = on;
+  pr->rows = rows;
   return MPCI_OK;
 }
 
@@ -941,6 +1036,7 @@ extern "C" int mpci_prop_create(mpci_system *sys, int P, mpci_prop **out) {
   if (!pr) return fail(MPCI_ERR_HIP, "host allocation failed");
   pr->sys = sys;
   pr->P = P;
+  pr->wait_limit_ms = kWaitLimitMs;
   HIPCHK(hipSetDevice(sys->device));
   HIPCHK(hipStreamCreateWithFlags(&pr->stream, hipStreamNonBlocking));
   pr->NP = (long long)sys->N * P;
@@ -952,20 +1048,24 @@ extern "C" int mpci_prop_create(mpci_system *sys, int P, mpci_prop **out) {
   TRY(pr->Xs.alloc(pr->NP));
   TRY(pr->Y.alloc(pr->NP));
   TRY(pr->K.alloc(pr->NP * kStages));
-  pr->nblk_small = (sys->N + 3) / 4;
+  int quads = 0;
+  for (int L = 0; L < sys->nb; ++L)
+    quads += (sys->s[L] + kRwQuad - 1) / kRwQuad;
   TRY(pr->red.alloc(
-      (size_t)std::max({pr->nblk, pr->nblk_stage, pr->nblk_small}) * P * 2));
-  TRY(pr->ctl.alloc(P));
+      (size_t)std::max({pr->nblk, pr->nblk_stage, quads}) * P * 2));
+  // behind the pulses' records: the one saved by k_rows_begin, and one whose
+  // status is k_rows_run's abort flag
+  TRY(pr->ctl.alloc(P + 2));
   TRY(pr->pulses.alloc(P));
   TRY(pr->log.alloc((size_t)pr->logcap * P));
   HIPCHK(hipMemsetAsync(pr->X.p, 0, sizeof(double2) * pr->NP, pr->stream));
   HIPCHK(hipMemsetAsync(pr->part.p, 0, sizeof(double2) * pr->part.n,
                         pr->stream));
   HIPCHK(hipStreamSynchronize(pr->stream));
-  std::vector<Ctl> c(P);
-  std::memset(c.data(), 0, sizeof(Ctl) * P);
+  std::vector<Ctl> c(P + 2);
+  std::memset(c.data(), 0, sizeof(Ctl) * c.size());
   for (auto &x : c) x.done = 1;
-  TRY(h2d(pr.get(), pr->ctl.p, c.data(), sizeof(Ctl) * P));
+  TRY(h2d(pr.get(), pr->ctl.p, c.data(), sizeof(Ctl) * c.size()));
   pr->hpulses.assign(P, PulseDev{});
   pr->henv.assign(P, {});
   if (P > 1 && sys->nb > 1) {
@@ -1151,17 +1251,13 @@ static int launch_small_stage(mpci_prop *pr, const StageArgs &a, int s) {
     e0 = pr->ev[pr->ev_base + 2 * s];
     e1 = pr->ev[pr->ev_base + 2 * s + 1];
   }
-  const dim3 grid(pr->nblk_small), block(256);
+  const dim3 grid((pr->nblk_small + 3) / 4), block(256);
   if (a.s == kStages - 1)
     hipExtLaunchKernelGGL((k_small_stage<true>), grid, block, 0, pr->stream,
-                          e0, e1, 0, a, pr->ddesc.p, sys->Dr.p, sys->dr_off.p,
-                          sys->dr_ld_d.p, sys->DrT.p, sys->drt_off.p,
-                          sys->drt_ld_d.p);
+                          e0, e1, 0, a, pr->ddesc.p, sys->drow.p, sys->Dq.p);
   else
     hipExtLaunchKernelGGL((k_small_stage<false>), grid, block, 0, pr->stream,
-                          e0, e1, 0, a, pr->ddesc.p, sys->Dr.p, sys->dr_off.p,
-                          sys->dr_ld_d.p, sys->DrT.p, sys->drt_off.p,
-                          sys->drt_ld_d.p);
+                          e0, e1, 0, a, pr->ddesc.p, sys->drow.p, sys->Dq.p);
   HIPCHK(hipGetLastError());
   return MPCI_OK;
 }
@@ -1263,8 +1359,59 @@ static int run_attempts_instrumented(mpci_prop *pr, int n) {
   return MPCI_OK;
 }
 
+// Attempts until the pulse has finished (or the log is full) in one
+// cooperative launch (k_rows_run); read_ctl undoes and switches off a launch
+// that gave up.  Returns false when the device does not take the launch.
+static bool run_attempts_rows(mpci_prop *pr) {
+  mpci_system *sys = pr->sys;
+  RowRun a{};
+  a.wg = pr->rwg.p;
+  a.X = pr->X.p;
+  a.E = sys->E.p;
+  a.xb = pr->xb.p;
+  a.rb = pr->rb.p;
+  a.ctl = pr->ctl.p;
+  a.abort_flag = &pr->ctl.p[pr->P + 1].status;
+  a.hs = pr->hs.p;
+  a.Ftab = pr->Ftab.p;
+  a.pulses = pr->pulses.p;
+  a.env = pr->env.p;
+  a.log = pr->log.p;
+  a.logcap = pr->logcap;
+  a.track = pr->track;
+  a.N = sys->N;
+  a.nquad = sys->hrow.quad0[sys->nb];
+  a.attempts = pr->logcap;
+  a.limit_ms = pr->wait_limit_ms;
+  const unsigned nb = (unsigned)((4LL * sys->N + 255) / 256);
+  hipLaunchKernelGGL(k_rows_begin, dim3(nb), dim3(256), 0, pr->stream, a,
+                     pr->Y.p, pr->ctl.p + pr->P);
+  if (hipGetLastError() != hipSuccess) return false;
+  const SysDesc *d = pr->ddesc.p;
+  const RowDesc *rd = sys->drow.p;
+  const double *dq = sys->Dq.p;
+  void *args[] = {&a, &d, &rd, &dq};
+  const void *fn = pr->rows_kq == 1
+                       ? reinterpret_cast<const void *>(k_rows_run<1>)
+                   : pr->rows_kq == 2
+                       ? reinterpret_cast<const void *>(k_rows_run<2>)
+                       : reinterpret_cast<const void *>(k_rows_run<4>);
+  if (hipLaunchCooperativeKernel(fn, dim3((unsigned)pr->rows_wg),
+                                 dim3(kRwThreads), args,
+                                 (unsigned)pr->rows_lds,
+                                 pr->stream) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 static int run_attempts(mpci_prop *pr, int n) {
   if (pr->instrument) return run_attempts_instrumented(pr, n);
+  if (pr->rows && pr->use_graph && !pr->store.xs && !pr->store.xn &&
+      !pr->store.nrm && !pr->store.ckpt) {
+    if (run_attempts_rows(pr)) return MPCI_OK;
+    pr->rows = false;
+  }
   if (pr->use_graph) {
     TRY(ensure_graph(pr));
     for (int i = 0; i < n; ++i) HIPCHK(hipGraphLaunch(pr->gexec, pr->stream));
@@ -1275,9 +1422,21 @@ static int run_attempts(mpci_prop *pr, int n) {
 }
 
 static int read_ctl(mpci_prop *pr, std::vector<Ctl> &c) {
-  c.resize(pr->P);
+  const int P = pr->P;
+  c.resize(pr->rows ? P + 2 : P);
   HIPCHK(hipStreamSynchronize(pr->stream));
-  TRY(d2h(pr, c.data(), pr->ctl.p, sizeof(Ctl) * pr->P));
+  TRY(d2h(pr, c.data(), pr->ctl.p, sizeof(Ctl) * c.size()));
+  if (pr->rows && c[P + 1].status) {
+    // the persistent launch gave up waiting (the device was held by others
+    // for longer than its time limit): back to where it began, and from now
+    // on one launch per stage
+    pr->rows = false;
+    HIPCHK(hipMemcpyAsync(pr->X.p, pr->Y.p, sizeof(double2) * pr->NP,
+                          hipMemcpyDeviceToDevice, pr->stream));
+    c[0] = c[P];
+    TRY(h2d(pr, pr->ctl.p, c.data(), sizeof(Ctl)));
+  }
+  c.resize(P);
   return MPCI_OK;
 }
 
@@ -1444,6 +1603,8 @@ extern "C" int mpci_system_rhs_noalloc(const mpci_system *sys, double F,
   return MPCI_OK;
 }
 
+static int plan_chunk(const mpci_prop *pr, const std::vector<Ctl> &c);
+
 extern "C" int mpci_prop_fixed(mpci_prop *pr, double t0, double dt, int steps,
                                const double *F, int track, double *pop) {
   if (!pr || !F || steps < 0) return fail(MPCI_ERR_ARG, "bad argument");
@@ -1468,13 +1629,10 @@ extern "C" int mpci_prop_fixed(mpci_prop *pr, double t0, double dt, int steps,
   }
   TRY(start_ctl(pr, c));
   std::vector<std::vector<LogEnt>> acc(pr->P);
-  int left = steps;
-  while (left > 0) {
-    const int n = std::min(left, pr->logcap);
+  for (int n; (n = plan_chunk(pr, c)) > 0;) {
     TRY(run_attempts(pr, n));
     TRY(read_ctl(pr, c));
     TRY(drain_log(pr, c, acc));
-    left -= n;
   }
   if (pop)
     for (int p = 0; p < pr->P; ++p)
@@ -2421,6 +2579,12 @@ extern "C" int mpci_prop_set_small_path(mpci_prop *pr, int mode,
   drop_graph(pr);  // the captured step holds the other path's kernels
   TRY(apply_small_path(pr, mode));
   if (active) *active = pr->small ? 1 : 0;
+  return MPCI_OK;
+}
+
+extern "C" int mpci_prop_set_wait_limit(mpci_prop *pr, int ms) {
+  if (!pr) return fail(MPCI_ERR_ARG, "NULL argument");
+  pr->wait_limit_ms = ms == 0 ? kWaitLimitMs : ms;
   return MPCI_OK;
 }
 

@@ -46,6 +46,25 @@ struct AdjArgs {
   int pad;
 };
 
+// The persistent row kernel: `attempts` attempts of one pulse in one
+// cooperative launch.
+struct RowRun {
+  const RowWg *wg;
+  double2 *X;            // committed state (N)
+  const double *E;
+  double2 *xb;           // stage inputs in exchange: 4 x N
+  double2 *rb;           // per-quad (error max, |y|^2) in exchange: 3 x nquad
+  Ctl *ctl;              // the pulse's control record
+  int *abort_flag;       // set when a wait ran into its time limit
+  const double *hs;
+  const double *Ftab;
+  const PulseDev *pulses;
+  const double *env;
+  LogEnt *log;
+  int logcap, track, N, nquad, attempts;
+  int limit_ms;          // time limit of one wait
+};
+
 // The coupling operands of every member of a grouped GEMM launch, passed
 // in the kernel arguments (so the compiler may reload them at will instead
 // of holding them in registers across the K loop).
@@ -116,10 +135,15 @@ __global__ void k_apply_g(const GroupMember *m, int nm);
 template <bool LAST>
 __global__ void k_stage1(StageArgs a, const SysDesc *d);
 template <bool LAST>
-__global__ void k_small_stage(StageArgs a, const SysDesc *d, const double *Dr,
-                              const long long *dr_off, const int *dr_ld,
-                              const double *DrT, const long long *drt_off,
-                              const int *drt_ld);
+__global__ void k_small_stage(StageArgs a, const SysDesc *d, const RowDesc *rd,
+                              const double *Dq);
+__global__ void k_relayout_rows(const double *Dg, const SysDesc *d,
+                                const RowDesc *rd, int njobs, int L,
+                                long long nelem, double *Dq);
+__global__ void k_rows_begin(RowRun a, double2 *Xsave, Ctl *ctl_save);
+template <int kQ>
+__global__ void k_rows_run(RowRun a, const SysDesc *d, const RowDesc *rd,
+                           const double *Dq);
 __global__ void k_finalize(Ctl *ctl, const double *red, int nblk, int P,
                            const double *hs, const double *Ftab,
                            const PulseDev *pulses, const double *env);

@@ -108,6 +108,7 @@ _SIGS = [
                                     _dp, C.c_int, _ip, _dp, C.c_int,
                                     C.POINTER(MpciAdjointStats)]),
     ("mpci_prop_set_graph", C.c_int, [_vp, C.c_int]),
+    ("mpci_prop_set_wait_limit", C.c_int, [_vp, C.c_int]),
     ("mpci_prop_set_instrument", C.c_int, [_vp, C.c_int]),
     ("mpci_prop_kernel_time", C.c_int, [_vp, _dp, C.POINTER(C.c_longlong),
                                         C.POINTER(C.c_longlong),

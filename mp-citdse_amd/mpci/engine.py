@@ -232,6 +232,10 @@ class Propagator:
     def set_graph(self, on: bool):
         check(_lib.tdse_lib().mpci_prop_set_graph(self.h, int(on)))
 
+    def set_wait_limit(self, ms: int = 0):
+        """Time limit of one wait inside a persistent launch (0: default)."""
+        check(_lib.tdse_lib().mpci_prop_set_wait_limit(self.h, int(ms)))
+
     def set_instrument(self, on: bool):
         check(_lib.tdse_lib().mpci_prop_set_instrument(self.h, int(on)))
 

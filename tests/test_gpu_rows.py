@@ -1,0 +1,115 @@
+"""The persistent row kernel (one pulse, whole runs in one cooperative
+launch) against the same run with one launch per stage, which sums in the
+same order, so the two agree bit for bit; and its way back when a launch
+gives up waiting.  The shapes sit at the kernel's edges: single states, row
+counts around the quads of 4 and workgroups of 16, neighbour columns around
+the 64-column chunks and the 16 chunks held in registers, chunks in LDS and
+past it, and more than 16 and 32 rows a workgroup."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [[1, 1], [3, 2, 4], [17, 64, 65, 5], [63, 129, 1, 16],
+          [300, 257, 513], [511, 513, 40], [1025, 30, 1100],
+          [2300, 9, 2600, 3], [4100, 8, 2100], [9000, 2, 3]]
+
+
+@pytest.fixture(scope="module")
+def mpci():
+    import mpci as m
+    assert m.device_count() >= 1
+    return m
+
+
+def state(n, seed):
+    x = np.random.default_rng(seed).standard_normal(2 * n)
+    return x / np.linalg.norm(x)
+
+
+def make(mpci, g, x0, graph, gauge):
+    prop = mpci.Propagator(g)
+    assert prop.set_small_path(1)
+    prop.set_graph(graph)
+    prop.set_state(x0)
+    prop.set_pulse(mpci.Pulse.sine(0.04 ** 2, 0.7, 2, gauge))
+    return prop
+
+
+@pytest.mark.parametrize("gauge", ["v", "l"])
+@pytest.mark.parametrize("s", SHAPES)
+def test_persistent_equals_stage_launches(mpci, s, gauge):
+    from mpci import synth
+    E, D = synth.system_arrays(s, seed=sum(s))
+    g = mpci.System(E, D, gauge=gauge)
+    x0 = state(g.N, len(s))
+    F = 0.05 * np.sin(np.arange(9.0))[None]
+    runs = []
+    for graph in (True, False):
+        prop = make(mpci, g, x0, graph, gauge)
+        # the first trial steps of 2 a.u. are rejected
+        st, log = prop.prop_adaptive(3.0, 7.0, 2.0, 1e-9, 1e-9, track=g.N - 1,
+                                     log_cap=400)
+        xa = prop.get_state()
+        pop = prop.prop_fixed(0.0, 0.1, F, track=g.N // 2)
+        prop.prop_schedule(1.0, [[0.1, 0.2, 0.05]])
+        runs.append((st[0].accepted, st[0].rejected, st[0].t, st[0].h, log,
+                     xa, pop, prop.get_state()))
+        prop.close()
+    assert runs[0][1] >= 1
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+
+
+def test_gives_up_and_goes_on(mpci):
+    """A launch that may not wait leaves at once; the run goes on with one
+    launch per stage from where it began, and so do later runs."""
+    from mpci import synth
+    E, D = synth.system_arrays([60, 75, 33], seed=3)
+    g = mpci.System(E, D)
+    x0 = state(g.N, 1)
+    out = []
+    for ms in (0, -1):
+        prop = make(mpci, g, x0, True, "v")
+        prop.set_wait_limit(ms)
+        st, _ = prop.prop_adaptive(0.0, 5.0, 0.1, 1e-10, 1e-10)
+        pop = prop.prop_fixed(0.0, 0.1, np.full((1, 30), 0.02))
+        out.append((st[0].accepted, pop, prop.get_state()))
+        prop.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+def test_nan_state_does_not_wait(mpci):
+    """A state that holds the exchange's marker bits (a signalling NaN no
+    arithmetic produces) propagates like any other NaN."""
+    from mpci import synth
+    E, D = synth.system_arrays([20, 30], seed=4)
+    g = mpci.System(E, D)
+    x0 = state(g.N, 2)
+    x0.view(np.uint64)[5] = 0x7FF4C0DEFACE0FF5
+    prop = make(mpci, g, x0, True, "v")
+    prop.prop_fixed(0.0, 0.1, np.full((1, 3), 0.02))
+    assert np.isnan(prop.get_state()).all()
+
+
+def test_concurrent_members(mpci):
+    """Several one-pulse propagators at once, each with its own persistent
+    launches, equal separate runs bit for bit."""
+    from mpci import synth
+    members = []
+    for i, s in enumerate(([198] * 4, [300, 257, 513], [40, 30])):
+        E, D = synth.system_arrays(s, seed=i)
+        g = mpci.System(E, D)
+        members.append((g, state(g.N, i)))
+    ref, props = [], []
+    for g, x0 in members:
+        prop = make(mpci, g, x0, True, "v")
+        prop.prop_adaptive(0.0, 9.0, 0.05, 1e-10, 1e-10)
+        ref.append(prop.get_state())
+        prop.set_state(x0)
+        props.append(prop)
+    n = len(props)
+    mpci.multi_adaptive(props, [0.0] * n, [9.0] * n, [0.05] * n, 1e-10, 1e-10)
+    for prop, r in zip(props, ref):
+        assert np.array_equal(prop.get_state(), r)
