@@ -252,9 +252,13 @@ int mpci_prop_observables(mpci_prop *prop, int electrons, double threshold,
                           double *out);
 
 /* Launch the 13-stage step as one captured hipGraph (1, default) or as
- * individual launches (0).  With 1, one pulse on a system whose dipoles take
- * at most 24 MiB runs its attempts inside one cooperative launch instead,
- * with the bits of the fused small-system stages (below). */
+ * individual launches (0).  With 1, one pulse on a system of more than one
+ * block runs its attempts inside one cooperative launch instead: where the
+ * dipoles take at most 24 MiB and a compute unit's share is at most 16 rows,
+ * with the bits of the fused small-system stages (below), otherwise with the
+ * coupling sums in an order of its own (equal to rounding, and the same from
+ * run to run).  A process that is refused cooperative launches, because
+ * another one on the device holds them, makes an ordinary launch of it. */
 int mpci_prop_set_graph(mpci_prop *prop, int enable);
 /* The workgroups of that launch wait for one another; a wait is given up
  * after `ms` milliseconds (0: the default of 20000; negative: at once), for
@@ -267,7 +271,8 @@ int mpci_prop_set_wait_limit(mpci_prop *prop, int ms);
  * algebra) instead of the GEMV tile kernel and the stage kernel.  mode -1
  * (default): on when P = 1, the system has more than one block and its
  * dipoles take at most 12 MiB; 0: off; 1: on whenever P = 1 and there is
- * more than one block.  active (may be NULL) reports the outcome.  Both
+ * more than one block (also inside the cooperative launch, whatever the
+ * size).  active (may be NULL) reports the outcome.  Both
  * paths give the same result to rounding (the coupling sums in another
  * order). */
 int mpci_prop_set_small_path(mpci_prop *prop, int mode, int *active);

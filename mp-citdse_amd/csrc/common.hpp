@@ -93,6 +93,34 @@ struct RowWg {
   int L, row0, nrows, quad0, nlds, pad;
 };
 
+// ---- persistent tile form (one pulse, larger systems) ------------------
+// The GEMV store is taken in groups of 16 rows x 256 columns (a row group of
+// one unit).  A segment is a run of groups down one column block of a pair;
+// a workgroup owns a run of groups, cut into segments, and some rows.
+constexpr int kTlReg = 4;     // groups of a workgroup kept in registers
+constexpr int kTlRing = 2;    // streamed groups in flight
+constexpr int kTlMaxRows = 256;  // rows owned by a workgroup
+struct TileSeg {
+  int L, cb;       // pair, column block
+  int g0, ng;      // row groups [g0, g0 + ng) of block L
+  int slot;        // partial slot of D^T x_L for this column block
+  int job0, ncb;   // first unit of the pair, its column blocks
+  int pad;
+};
+struct TileWg {
+  int seg0, nseg;      // its segments
+  int ngroups, nlds;   // groups in all, groups kept in LDS
+  int L, row0, nrows;  // its rows: of block L (nrows may be 0)
+  int nrs, ncs;        // partials per row: D x_{L+1}, D^T x_{L-1} (at most)
+  int pad;
+};
+struct TileDesc {
+  int part_n;                  // partials of one exchange copy
+  int rp_off[kMaxBlocks];      // pair L: D x_{L+1}, [column block][row]
+  int cp_off[kMaxBlocks];      // pair L: D^T x_L, [slot][column]
+  int cs_off[kMaxBlocks];      // pair L: where its slot counts begin
+};
+
 // Per-propagator description of the blocks and the partial-sum buffers.
 struct SysDesc {
   int nb;

@@ -135,8 +135,18 @@ struct mpci_prop {
   size_t rows_lds = 0;   // dynamic LDS bytes
   int rows_kq = 1;       // quads per computing wave
   int wait_limit_ms = 0; // time limit of one wait inside the launch
+  bool coop_refused = false;  // another process holds cooperative launching
   DevBuf<RowWg> rwg;
-  DevBuf<double2> xb, rb;  // exchange buffers
+  // the same for larger systems (k_tiles_run)
+  bool tiles = false;
+  int tiles_wg = 0, tiles_xrows = 0, tiles_xsegs = 0, tiles_xpieces = 0,
+      tiles_part = 0;
+  size_t tiles_lds = 0;
+  DevBuf<TileWg> twg;
+  DevBuf<TileSeg> tseg;
+  DevBuf<TileDesc> tdesc;
+  DevBuf<int> tslot;
+  DevBuf<double2> xb, pb, rb;  // exchange buffers
   DevBuf<double2> X, Xs, K, Y, part;
   DevBuf<double2> xstage;  // one pulse's contiguous state (set/get_state)
   DevBuf<double2> Xs2;  // second stage-input buffer of the fused path
@@ -925,13 +935,19 @@ static int autotune_gemm(mpci_prop *pr) {
 // on four equal blocks: 1.95x the tile path at 0.9 MB of dipoles, 1.30x at
 // 8.6 MB, even at 15 MB, 0.85x at 24 MB.
 constexpr long long kSmallPathBytes = 12LL << 20;
-// The same for whole runs in one persistent launch (k_rows_run): past it the
-// row store no longer stays on the chip (registers and LDS of the workgroups,
-// then L2).  Per attempt against the tile path, four equal blocks: 0.9 MB
-// 31.6 against 83 us, 6 MB 37.9 against 116 us, 19.4 MB 78 against 164 us,
-// 31.7 MB and beyond see the table in k_rows_run's comment.
+// The same for whole runs in one persistent launch: the row form
+// (k_rows_run) up to here, the tile form (k_tiles_run) past it, where the
+// row store, which holds every dipole twice, outgrows registers and LDS.  Per
+// attempt, row against tile form: 6 x 300 (3.6 MB) 34.9 against 72 us, 4 x
+// 700 (12 MB) 51 against 100 us, 4 x 1000 (24 MB) 87 against 104 us, 4 x 1150
+// (32 MB) 186 against 113 us.  The launches these replace took 105 us (6 x
+// 300), 164 us (4 x 900), 200 us (4 x 1500), 474 us (He_test.yaml shape),
+// 910 us (He 4 x 4000); the tile form takes 127, 355 and 763 us there.
 constexpr long long kRowsBytes = 24LL << 20;
-constexpr int kWaitLimitMs = 20000;  // time limit of one wait in k_rows_run
+constexpr int kWaitLimitMs = 20000;  // time limit of one wait in them
+// Time limit of the start of an ordinary launch: two processes' launches
+// that hold half the device each let go of it after this.
+constexpr int kStartLimitMs = 200;
 
 // The workgroups of the persistent row kernel: at most one per compute unit,
 // each inside one block, 16 rows (one pass of its four quads) while that
@@ -994,15 +1010,183 @@ static bool plan_rows(const mpci_prop *pr, std::vector<RowWg> &wg,
   return (int)wg.size() <= sys->ncu;
 }
 
-// mode -1: automatic (one pulse, more than one block, 8 S within
-// kSmallPathBytes); 0: off; 1: on wherever it applies (one pulse, more
-// than one block).
+struct TilePlan {
+  std::vector<TileWg> wg;
+  std::vector<TileSeg> seg;
+  std::vector<int> nslot;
+  TileDesc desc{};
+  int xrows = 0, xsegs = 0, xpieces = 0;
+  size_t lds = 0;
+};
+
+// The workgroups of the persistent tile kernel: the row groups of all units
+// in the order (pair, column block, row), cut into as many runs of equal
+// bytes as there are compute units, and the rows dealt out evenly.  Returns
+// false when the form does not apply to the system.
+static bool plan_tiles(const mpci_prop *pr, TilePlan &pl) {
+  const mpci_system *sys = pr->sys;
+  if (pr->P != 1 || sys->nb < 2 || 48LL * sys->N >= (1LL << 31)) return false;
+  int coop = 0, lds_max = 0;
+  if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch,
+                            sys->device) != hipSuccess || !coop)
+    return false;
+  if (hipDeviceGetAttribute(&lds_max,
+                            hipDeviceAttributeMaxSharedMemoryPerBlock,
+                            sys->device) != hipSuccess)
+    return false;
+  const int np = sys->nb - 1;
+  // a group's weight: a group of a narrow last column block takes nearly the
+  // time of a full one (He 4 x 4000 per attempt: weight by columns with a
+  // share of 32 for the rest 971 us, 256 845 us, 1000 778 us, 2000 763 us)
+  auto weight = [&](int L, int cb) {
+    return 2000.0 + std::min(kGvTC, sys->s[L + 1] - cb * kGvTC);
+  };
+  double total = 0.0;
+  long long groups = 0;
+  for (int L = 0; L < np; ++L) {
+    const int ng = (sys->s[L] + 15) / 16;
+    for (int cb = 0; cb < sys->ncb[L]; ++cb) total += ng * weight(L, cb);
+    groups += (long long)ng * sys->ncb[L];
+  }
+  const int W = (int)std::min<long long>({(long long)sys->ncu, groups, 256LL});
+  std::vector<int> cs0(np);
+  int nc = 0;
+  for (int L = 0; L < np; ++L) {
+    cs0[L] = nc;
+    nc += sys->ncb[L];
+  }
+  pl.nslot.assign(nc, 0);
+  pl.wg.assign(W, TileWg{});
+  double done = 0.0;
+  int w = 0, job0 = 0;
+  for (int L = 0; L < np; ++L) {
+    const int ng = (sys->s[L] + 15) / 16;
+    for (int cb = 0; cb < sys->ncb[L]; ++cb)
+      for (int g = 0; g < ng; ++g) {
+        // the group goes to the workgroup its middle falls to
+        const double mid = done + 0.5 * weight(L, cb);
+        done += weight(L, cb);
+        const int to = std::min(W - 1, (int)(mid / total * W));
+        const bool cut = to != w || g == 0 || pl.seg.empty();
+        if (to != w) w = to;
+        TileWg &q = pl.wg[w];
+        if (cut) {
+          TileSeg sg{};
+          sg.L = L;
+          sg.cb = cb;
+          sg.g0 = g;
+          sg.slot = pl.nslot[cs0[L] + cb]++;
+          sg.job0 = job0;
+          sg.ncb = sys->ncb[L];
+          if (q.nseg == 0) q.seg0 = (int)pl.seg.size();
+          ++q.nseg;
+          pl.seg.push_back(sg);
+        }
+        ++pl.seg.back().ng;
+        ++q.ngroups;
+      }
+    job0 += sys->nrb[L] * sys->ncb[L];
+  }
+  // partials
+  long long o = 0;
+  std::vector<int> slots(np, 0);
+  for (int L = 0; L < np; ++L) {
+    for (int cb = 0; cb < sys->ncb[L]; ++cb)
+      slots[L] = std::max(slots[L], pl.nslot[cs0[L] + cb]);
+    pl.desc.cs_off[L] = cs0[L];
+    pl.desc.rp_off[L] = (int)o;
+    o += (long long)sys->ncb[L] * sys->s[L];
+    pl.desc.cp_off[L] = (int)o;
+    o += (long long)slots[L] * sys->s[L + 1];
+    if (48 * o >= (1LL << 31)) return false;
+  }
+  pl.desc.part_n = (int)o;
+  // rows
+  int rpw = (sys->N + W - 1) / W;
+  for (;; ++rpw) {
+    int n = 0;
+    for (int L = 0; L < sys->nb; ++L) n += (sys->s[L] + rpw - 1) / rpw;
+    if (n <= W) break;
+    if (rpw > kTlMaxRows) return false;
+  }
+  if (rpw > kTlMaxRows) return false;
+  w = 0;
+  for (int L = 0; L < sys->nb; ++L)
+    for (int r = 0; r < sys->s[L]; r += rpw) {
+      TileWg &q = pl.wg[w++];
+      q.L = L;
+      q.row0 = r;
+      q.nrows = std::min(rpw, sys->s[L] - r);
+      q.nrs = L < np ? sys->ncb[L] : 0;
+      q.ncs = L > 0 ? slots[L - 1] : 0;
+    }
+  // LDS
+  for (const TileWg &q : pl.wg) {
+    pl.xrows = std::max(pl.xrows, q.ngroups * 16);
+    pl.xsegs = std::max(pl.xsegs, q.nseg);
+    int n = 0;
+    for (int k = 0; k < q.nseg; ++k) n += (pl.seg[q.seg0 + k].ng + 3) / 4 + 4;
+    pl.xpieces = std::max(pl.xpieces, n);
+  }
+  const long long room = (long long)lds_max - 8192;  // the static part
+  const long long group = 16LL * kGvTC * 8;
+  for (TileWg &q : pl.wg) {
+    const long long base =
+        16LL * (pl.xrows + (long long)pl.xsegs * kGvTC +
+                2LL * (kGvThreads / 64) * kGvTR +
+                (long long)(kGvThreads / 64 + kStages) * q.nrows + q.ngroups +
+                pl.xpieces + 2 * pl.xsegs);
+    if (base > room) return false;
+    q.nlds = (int)std::min<long long>(std::max(q.ngroups - kTlReg, 0),
+                                      (room - base) / group);
+    pl.lds = std::max<size_t>(pl.lds, base + q.nlds * group);
+  }
+  // one workgroup per compute unit at a time, whatever its size
+  pl.lds = std::max<size_t>(pl.lds, lds_max / 2 + 1024);
+  return true;
+}
+
+static int setup_tiles(mpci_prop *pr, bool *ok) {
+  TilePlan pl;
+  *ok = plan_tiles(pr, pl);
+  if (!*ok) return MPCI_OK;
+  const int N = pr->sys->N, W = (int)pl.wg.size();
+  TRY(pr->xb.alloc(3 * (size_t)N));
+  TRY(pr->pb.alloc(3 * (size_t)pl.desc.part_n));
+  TRY(pr->rb.alloc(3 * (size_t)W));
+  TRY(pr->tseg.alloc(pl.seg.size()));
+  TRY(pr->tdesc.alloc(1));
+  TRY(pr->tslot.alloc(std::max<size_t>(pl.nslot.size(), 1)));
+  TRY(h2d(pr, pr->tseg.p, pl.seg.data(), sizeof(TileSeg) * pl.seg.size()));
+  TRY(h2d(pr, pr->tdesc.p, &pl.desc, sizeof(TileDesc)));
+  TRY(h2d(pr, pr->tslot.p, pl.nslot.data(), sizeof(int) * pl.nslot.size()));
+  TRY(pr->twg.alloc(W));
+  TRY(h2d(pr, pr->twg.p, pl.wg.data(), sizeof(TileWg) * W));
+  pr->tiles_wg = W;
+  pr->tiles_xrows = pl.xrows;
+  pr->tiles_xsegs = pl.xsegs;
+  pr->tiles_xpieces = pl.xpieces;
+  pr->tiles_part = pl.desc.part_n;
+  pr->tiles_lds = pl.lds;
+  return MPCI_OK;
+}
+
+// The forms of one pulse on more than one block: fused stages from the row
+// store (small), and the persistent launches (rows, tiles).  mode -1:
+// automatic; 0: none of them; 1: the row store wherever it applies.
 static int apply_small_path(mpci_prop *pr, int mode) {
   mpci_system *sys = pr->sys;
-  bool on = false, rows = false;
+  bool on = false, rows = false, tiles = false;
   if (pr->P == 1 && sys->nb > 1) {
     on = mode == 1 || (mode < 0 && 8 * sys->S <= kSmallPathBytes);
-    rows = mode == 1 || (mode < 0 && 8 * sys->S <= kRowsBytes);
+    // the row form by default only where a wave has one quad: with more rows
+    // than that the tile form is faster (12 x 500 96 against 120 us per
+    // attempt, 30 x 250 89 against 200 us)
+    int n16 = 0;
+    for (int L = 0; L < sys->nb; ++L) n16 += (sys->s[L] + 15) / 16;
+    rows = mode == 1 ||
+           (mode < 0 && 8 * sys->S <= kRowsBytes && n16 <= sys->ncu);
+    tiles = mode < 0 && !rows;
   }
   if (on || rows) {
     TRY(ensure_rows(sys));
@@ -1022,8 +1206,10 @@ static int apply_small_path(mpci_prop *pr, int mode) {
       pr->rows_wg = (int)wg.size();
     }
   }
+  if (tiles && !pr->twg.p) TRY(setup_tiles(pr, &tiles));
   pr->small = on;
   pr->rows = rows;
+  pr->tiles = tiles;
   return MPCI_OK;
 }
 
@@ -1360,57 +1546,104 @@ static int run_attempts_instrumented(mpci_prop *pr, int n) {
 }
 
 // Attempts until the pulse has finished (or the log is full) in one
-// cooperative launch (k_rows_run); read_ctl undoes and switches off a launch
-// that gave up.  Returns false when the device does not take the launch.
-static bool run_attempts_rows(mpci_prop *pr) {
+// cooperative launch (k_rows_run, k_tiles_run); read_ctl undoes and switches
+// off a launch that gave up.  Returns false when the device does not take
+// the launch.
+static bool run_attempts_persistent(mpci_prop *pr) {
   mpci_system *sys = pr->sys;
-  RowRun a{};
-  a.wg = pr->rwg.p;
-  a.X = pr->X.p;
-  a.E = sys->E.p;
-  a.xb = pr->xb.p;
-  a.rb = pr->rb.p;
-  a.ctl = pr->ctl.p;
-  a.abort_flag = &pr->ctl.p[pr->P + 1].status;
-  a.hs = pr->hs.p;
-  a.Ftab = pr->Ftab.p;
-  a.pulses = pr->pulses.p;
-  a.env = pr->env.p;
-  a.log = pr->log.p;
-  a.logcap = pr->logcap;
-  a.track = pr->track;
-  a.N = sys->N;
-  a.nquad = sys->hrow.quad0[sys->nb];
-  a.attempts = pr->logcap;
-  a.limit_ms = pr->wait_limit_ms;
-  const unsigned nb = (unsigned)((4LL * sys->N + 255) / 256);
-  hipLaunchKernelGGL(k_rows_begin, dim3(nb), dim3(256), 0, pr->stream, a,
-                     pr->Y.p, pr->ctl.p + pr->P);
+  const int nxb = (pr->rows ? 4 : 3) * sys->N;
+  const int npb = pr->rows ? 0 : 3 * pr->tiles_part;
+  const int nrb = 3 * (pr->rows ? sys->hrow.quad0[sys->nb] : pr->tiles_wg);
+  int *flag = &pr->ctl.p[pr->P + 1].status;
+  int *arrived = &pr->ctl.p[pr->P + 1].nlog;
+  const unsigned nb = (unsigned)((std::max(nxb, npb) + 255) / 256);
+  hipLaunchKernelGGL(k_rows_begin, dim3(nb), dim3(256), 0, pr->stream,
+                     pr->xb.p, nxb, pr->pb.p, npb, pr->rb.p, nrb, pr->X.p,
+                     sys->N, pr->Y.p, pr->ctl.p, pr->ctl.p + pr->P, flag,
+                     arrived);
   if (hipGetLastError() != hipSuccess) return false;
+  auto common = [&](auto &a) {
+    a.X = pr->X.p;
+    a.E = sys->E.p;
+    a.xb = pr->xb.p;
+    a.rb = pr->rb.p;
+    a.ctl = pr->ctl.p;
+    a.abort_flag = flag;
+    a.hs = pr->hs.p;
+    a.Ftab = pr->Ftab.p;
+    a.pulses = pr->pulses.p;
+    a.env = pr->env.p;
+    a.log = pr->log.p;
+    a.logcap = pr->logcap;
+    a.track = pr->track;
+    a.N = sys->N;
+    a.attempts = pr->logcap;
+    a.limit_ms = pr->wait_limit_ms;
+    a.arrived = arrived;
+    a.start_ms = pr->coop_refused ? kStartLimitMs : 0;
+  };
   const SysDesc *d = pr->ddesc.p;
-  const RowDesc *rd = sys->drow.p;
-  const double *dq = sys->Dq.p;
-  void *args[] = {&a, &d, &rd, &dq};
-  const void *fn = pr->rows_kq == 1
-                       ? reinterpret_cast<const void *>(k_rows_run<1>)
-                   : pr->rows_kq == 2
-                       ? reinterpret_cast<const void *>(k_rows_run<2>)
-                       : reinterpret_cast<const void *>(k_rows_run<4>);
-  if (hipLaunchCooperativeKernel(fn, dim3((unsigned)pr->rows_wg),
-                                 dim3(kRwThreads), args,
-                                 (unsigned)pr->rows_lds,
-                                 pr->stream) == hipSuccess)
-    return true;
+  // A second process on the device is refused cooperative launches
+  // (hipErrorIllegalState) for as long as the first holds them.  It launches
+  // the ordinary way: on an idle device every workgroup is resident all the
+  // same, and where one is not after kStartLimitMs the launch gives up.
+  auto launch = [&](const void *fn, int wgs, int threads, void **args,
+                    int *start_ms, size_t lds) {
+    const dim3 g((unsigned)wgs), b((unsigned)threads);
+    if (!pr->coop_refused) {
+      const hipError_t rc = hipLaunchCooperativeKernel(
+          fn, g, b, args, (unsigned)lds, pr->stream);
+      if (rc != hipErrorIllegalState) return rc;
+      (void)hipGetLastError();
+      pr->coop_refused = true;
+      *start_ms = kStartLimitMs;
+    }
+    return hipLaunchKernel(fn, g, b, args, lds, pr->stream);
+  };
+  hipError_t e;
+  if (pr->rows) {
+    RowRun a{};
+    common(a);
+    a.wg = pr->rwg.p;
+    a.nquad = sys->hrow.quad0[sys->nb];
+    const RowDesc *rd = sys->drow.p;
+    const double *dq = sys->Dq.p;
+    void *args[] = {&a, &d, &rd, &dq};
+    const void *fn = pr->rows_kq == 1
+                         ? reinterpret_cast<const void *>(k_rows_run<1>)
+                     : pr->rows_kq == 2
+                         ? reinterpret_cast<const void *>(k_rows_run<2>)
+                         : reinterpret_cast<const void *>(k_rows_run<4>);
+    e = launch(fn, pr->rows_wg, kRwThreads, args, &a.start_ms, pr->rows_lds);
+  } else {
+    TileRun a{};
+    common(a);
+    a.wg = pr->twg.p;
+    a.seg = pr->tseg.p;
+    a.nslot = pr->tslot.p;
+    a.Dg = sys->Dg.p;
+    a.pb = pr->pb.p;
+    a.nwg = pr->tiles_wg;
+    a.njobs = (int)sys->jobs.size();
+    a.xs_rows = pr->tiles_xrows;
+    a.xs_segs = pr->tiles_xsegs;
+    a.xs_pieces = pr->tiles_xpieces;
+    const TileDesc *td = pr->tdesc.p;
+    void *args[] = {&a, &d, &td};
+    e = launch(reinterpret_cast<const void *>(k_tiles_run), pr->tiles_wg,
+               kGvThreads, args, &a.start_ms, pr->tiles_lds);
+  }
+  if (e == hipSuccess) return true;
   (void)hipGetLastError();
   return false;
 }
 
 static int run_attempts(mpci_prop *pr, int n) {
   if (pr->instrument) return run_attempts_instrumented(pr, n);
-  if (pr->rows && pr->use_graph && !pr->store.xs && !pr->store.xn &&
-      !pr->store.nrm && !pr->store.ckpt) {
-    if (run_attempts_rows(pr)) return MPCI_OK;
-    pr->rows = false;
+  if ((pr->rows || pr->tiles) && pr->use_graph && !pr->store.xs &&
+      !pr->store.xn && !pr->store.nrm && !pr->store.ckpt) {
+    if (run_attempts_persistent(pr)) return MPCI_OK;
+    pr->rows = pr->tiles = false;
   }
   if (pr->use_graph) {
     TRY(ensure_graph(pr));
@@ -1423,14 +1656,15 @@ static int run_attempts(mpci_prop *pr, int n) {
 
 static int read_ctl(mpci_prop *pr, std::vector<Ctl> &c) {
   const int P = pr->P;
-  c.resize(pr->rows ? P + 2 : P);
+  const bool persistent = pr->rows || pr->tiles;
+  c.resize(persistent ? P + 2 : P);
   HIPCHK(hipStreamSynchronize(pr->stream));
   TRY(d2h(pr, c.data(), pr->ctl.p, sizeof(Ctl) * c.size()));
-  if (pr->rows && c[P + 1].status) {
+  if (persistent && c[P + 1].status) {
     // the persistent launch gave up waiting (the device was held by others
     // for longer than its time limit): back to where it began, and from now
     // on one launch per stage
-    pr->rows = false;
+    pr->rows = pr->tiles = false;
     HIPCHK(hipMemcpyAsync(pr->X.p, pr->Y.p, sizeof(double2) * pr->NP,
                           hipMemcpyDeviceToDevice, pr->stream));
     c[0] = c[P];

@@ -14,76 +14,11 @@
 //   k_stage1         the same for one pulse, 16 lanes per row, every load
 //                    in one round.
 //   k_small_stage    coupling and stage of one pulse on a small system.
-//   k_rows_run       whole attempts of it in one cooperative launch.
 //   k_finalize       per-pulse reduction + on-device accept/reject control.
 //   k_apply          accepted: x = y / ||y|| (tdse.cpp:194-198) + log entry.
-#include "kernels.hpp"
+#include "device.hpp"
 
 namespace mpci {
-
-// Fehlberg 7(8) tableau (NASA TR R-287, 1968), the coefficients of
-// boost::odeint runge_kutta_fehlberg78.
-__constant__ double cA[kStages][kStages] = {
-    {0},
-    {2.0 / 27.0},
-    {1.0 / 36.0, 1.0 / 12.0},
-    {1.0 / 24.0, 0.0, 1.0 / 8.0},
-    {5.0 / 12.0, 0.0, -25.0 / 16.0, 25.0 / 16.0},
-    {1.0 / 20.0, 0.0, 0.0, 1.0 / 4.0, 1.0 / 5.0},
-    {-25.0 / 108.0, 0.0, 0.0, 125.0 / 108.0, -65.0 / 27.0, 125.0 / 54.0},
-    {31.0 / 300.0, 0.0, 0.0, 0.0, 61.0 / 225.0, -2.0 / 9.0, 13.0 / 900.0},
-    {2.0, 0.0, 0.0, -53.0 / 6.0, 704.0 / 45.0, -107.0 / 9.0, 67.0 / 90.0, 3.0},
-    {-91.0 / 108.0, 0.0, 0.0, 23.0 / 108.0, -976.0 / 135.0, 311.0 / 54.0,
-     -19.0 / 60.0, 17.0 / 6.0, -1.0 / 12.0},
-    {2383.0 / 4100.0, 0.0, 0.0, -341.0 / 164.0, 4496.0 / 1025.0,
-     -301.0 / 82.0, 2133.0 / 4100.0, 45.0 / 82.0, 45.0 / 164.0, 18.0 / 41.0},
-    {3.0 / 205.0, 0.0, 0.0, 0.0, 0.0, -6.0 / 41.0, -3.0 / 205.0, -3.0 / 41.0,
-     3.0 / 41.0, 6.0 / 41.0, 0.0},
-    {-1777.0 / 4100.0, 0.0, 0.0, -341.0 / 164.0, 4496.0 / 1025.0,
-     -289.0 / 82.0, 2193.0 / 4100.0, 51.0 / 82.0, 33.0 / 164.0, 12.0 / 41.0,
-     0.0, 1.0},
-};
-__constant__ double cB[kStages] = {0, 0, 0, 0, 0, 34.0 / 105.0, 9.0 / 35.0,
-                                   9.0 / 35.0, 9.0 / 280.0, 9.0 / 280.0, 0,
-                                   41.0 / 840.0, 41.0 / 840.0};
-// b - bhat: the embedded error weights.
-__constant__ double cDB[kStages] = {-41.0 / 840.0, 0, 0, 0, 0, 0, 0, 0, 0, 0,
-                                    -41.0 / 840.0, 41.0 / 840.0,
-                                    41.0 / 840.0};
-__constant__ double cC[kStages] = {0, 2.0 / 27.0, 1.0 / 9.0, 1.0 / 6.0,
-                                   5.0 / 12.0, 0.5, 5.0 / 6.0, 1.0 / 6.0,
-                                   2.0 / 3.0, 1.0 / 3.0, 1.0, 0, 1.0};
-
-// ---------------------------------------------------------------------
-// Laser field, src/tdse/pulse.cpp:34-39 (gauss), 52-56 (sineAA), 93-97
-// (sineEE), plus the piecewise-linear envelope extension.
-// Always inlined: hipcc (ROCm 7.2) emitted this as a call from inside a
-// divergent branch and copied the saved thread id under the branch's exec
-// mask, so lanes outside the branch lost threadIdx.x across the call.
-// ---------------------------------------------------------------------
-__device__ __forceinline__ double field_at(const PulseDev &p,
-                                           const double *env, double t) {
-  if (p.kind == kSine2) {
-    double sinWt = sin(p.a * t);
-    return (double)(t >= 0.0 && t <= M_PI / p.a) * p.Eo * sinWt * sinWt *
-           sin(p.w * t + p.cepd);
-  }
-  if (p.kind == kGauss) {
-    double t_diff = t - 0.5 * p.b;
-    return (double)(t >= 0.0 && t <= p.b) * p.Eo *
-           exp(-t_diff * t_diff / (p.a * p.a)) * sin(p.w * t + p.cepd);
-  }
-  if (!(t >= 0.0 && t <= p.t_end) || p.n_env < 2) return 0.0;
-  const double *e = env + p.env_off;
-  double dx = p.t_end / (p.n_env - 1);
-  double u = t / dx;
-  int k = (int)floor(u);
-  if (k > p.n_env - 2) k = p.n_env - 2;
-  if (k < 0) k = 0;
-  double f = u - k;
-  double en = (1.0 - f) * e[k] + f * e[k + 1];
-  return p.scale * en * sin(p.w * t + p.cepd);
-}
 
 // ---------------------------------------------------------------------
 // One-time dipole re-layout into the GEMV store.  Row group i of every
@@ -115,49 +50,6 @@ __global__ void k_relayout_gemv(const double *__restrict__ D, int sL, int sL1,
       ((((long long)i * njobs + job) * kGvColPairIter + j) * kGvThreads + t) *
           2 + el;
   out[dst] = (row < sL && col < sL1) ? D[(long long)row * sL1 + col] : 0.0;
-}
-
-// ---------------------------------------------------------------------
-// Cross-lane sums on the VALU (DPP and the gfx950 lane swaps), no LDS.
-// ---------------------------------------------------------------------
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF,
-                                             0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF,
-                                             0xF, false);
-  return __hiloint2double(hi, lo);
-}
-
-// Sum over the 16 lanes of a row: quad_perm [1,0,3,2], quad_perm [2,3,0,1],
-// row_half_mirror, row_mirror.  Each step adds two operands, which commute
-// exactly, so every lane of the row ends with the same bits.
-__device__ __forceinline__ double sum16(double v) {
-  v += dpp_d<0xB1>(v);
-  v += dpp_d<0x4E>(v);
-  v += dpp_d<0x141>(v);
-  v += dpp_d<0x140>(v);
-  return v;
-}
-
-// v[l] + v[l ^ 16]: v_permlane16_swap of v with itself leaves the even rows
-// in the first result and the odd rows in the second, so lane l holds both
-// operands; l and l ^ 16 add them in the same order.
-__device__ __forceinline__ double add_xor16(double v) {
-  const unsigned lo = __double2loint(v), hi = __double2hiint(v);
-  const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-  const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-  return __hiloint2double((int)h[0], (int)l[0]) +
-         __hiloint2double((int)h[1], (int)l[1]);
-}
-
-// v[l] + v[l ^ 32], likewise with v_permlane32_swap (wave halves).
-__device__ __forceinline__ double add_xor32(double v) {
-  const unsigned lo = __double2loint(v), hi = __double2hiint(v);
-  const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-  const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-  return __hiloint2double((int)h[0], (int)l[0]) +
-         __hiloint2double((int)h[1], (int)l[1]);
 }
 
 // ---------------------------------------------------------------------
@@ -1264,30 +1156,6 @@ __device__ __forceinline__ void sum_both(const double2 *cb, int nc,
   }
 }
 
-// k_s of one (row, pulse) from the coupling sums cs = D^T x_{L-1} and
-// rs = D x_{L+1}, the stage input xs, the energy e and the stage field F
-// (MatVecV / MatVecL, src/tdse/tdse.cpp:14-143).  The fma is written out:
-// left to the compiler, which of the two products it fuses may differ from
-// one kernel to another, and with it the last bit.
-__device__ __forceinline__ double2 stage_deriv(int gauge, double e, double2 xs,
-                                               double F, double2 cs,
-                                               double2 rs) {
-  double2 k;
-  if (gauge == 0) {  // velocity: -iE x + F (D^T x_{L-1} - D x_{L+1})
-    k.x = fma(F, cs.x - rs.x, e * xs.y);
-    k.y = fma(F, cs.y - rs.y, -e * xs.x);
-  } else {           // length: -i (E x + F (D^T x_{L-1} + D x_{L+1}))
-    k.x = fma(F, cs.y + rs.y, e * xs.y);
-    k.y = fma(-F, cs.x + rs.x, -e * xs.x);
-  }
-  return k;
-}
-
-// |v|^2, likewise.
-__device__ __forceinline__ double abs2(double x, double y) {
-  return fma(x, x, y * y);
-}
-
 // The per-row end of a stage, shared by k_stage and k_small_stage: from
 // the coupling sums cs = D^T x_{L-1} and rs = D x_{L+1} of (row, pulse p)
 // it forms k_s, stores it, and forms the next stage input, or on the
@@ -1467,92 +1335,6 @@ __global__ __launch_bounds__(256) void k_stage_g(
 }
 template __global__ void k_stage_g<false>(const GroupMember *, int, int);
 template __global__ void k_stage_g<true>(const GroupMember *, int, int);
-// ---------------------------------------------------------------------
-// Row form (one pulse): a wave forms the coupling sums of four rows (a quad)
-// from the row store (RowDesc), its lanes taking the columns of each
-// 64-column chunk of [D_{L-1}^T | D_L] in turn.  The stage input enters the
-// second part with the sign of the gauge's formula, so one sum per component
-// holds D^T x_{L-1} - D x_{L+1} (velocity) or the plus form (length).
-// ---------------------------------------------------------------------
-__device__ __forceinline__ void quad_fma(double2 (&acc)[4], double2 d01,
-                                         double2 d23, double2 x) {
-  acc[0].x = fma(d01.x, x.x, acc[0].x);
-  acc[0].y = fma(d01.x, x.y, acc[0].y);
-  acc[1].x = fma(d01.y, x.x, acc[1].x);
-  acc[1].y = fma(d01.y, x.y, acc[1].y);
-  acc[2].x = fma(d23.x, x.x, acc[2].x);
-  acc[2].y = fma(d23.x, x.y, acc[2].y);
-  acc[3].x = fma(d23.y, x.x, acc[3].x);
-  acc[3].y = fma(d23.y, x.y, acc[3].y);
-}
-
-// Lane-swap sum of two values: the lower wave half (HALF) or the even rows
-// of 16 lanes keep the sum of a, the others that of b.
-template <bool HALF>
-__device__ __forceinline__ double pair_sum(double a, double b) {
-  const unsigned al = __double2loint(a), ah = __double2hiint(a);
-  const unsigned bl = __double2loint(b), bh = __double2hiint(b);
-  if constexpr (HALF) {
-    const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
-    const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
-    return __hiloint2double((int)h[0], (int)l[0]) +
-           __hiloint2double((int)h[1], (int)l[1]);
-  } else {
-    const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
-    const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
-    return __hiloint2double((int)h[0], (int)l[0]) +
-           __hiloint2double((int)h[1], (int)l[1]);
-  }
-}
-
-// dpp_d for controls under which every lane reads a lane of its row.
-template <int CTRL>
-__device__ __forceinline__ double dpp_perm(double v) {
-  const int lo =
-      __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
-  const int hi =
-      __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
-  return __hiloint2double(hi, lo);
-}
-
-// The eight sums of a wave over its 64 lanes in ten additions (a wave64
-// instruction takes four cycles, so their number counts): every lane l
-// returns both parts of row l >> 4.
-__device__ __forceinline__ double2 quad_reduce(const double2 (&acc)[4],
-                                               int lane) {
-  // halves: rows 0, 1 | 2, 3; then rows of 16 lanes: 0 | 1 | 2 | 3
-  const double re = pair_sum<false>(pair_sum<true>(acc[0].x, acc[2].x),
-                                    pair_sum<true>(acc[1].x, acc[3].x));
-  const double im = pair_sum<false>(pair_sum<true>(acc[0].y, acc[2].y),
-                                    pair_sum<true>(acc[1].y, acc[3].y));
-  // the lower eight lanes of a row go on with the real part
-  const bool up = (lane & 8) != 0;
-  double v = up ? im : re;
-  v += dpp_perm<0x128>(up ? re : im);  // row_ror:8, the other half's share
-  v += dpp_perm<0xB1>(v);
-  v += dpp_perm<0x4E>(v);
-  v += dpp_perm<0x141>(v);
-  const double o = dpp_perm<0x128>(v);
-  return up ? make_double2(o, v) : make_double2(v, o);
-}
-
-// (error max, |y|^2) of a quad's rows in order, from lanes 0, 16, 32, 48.
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  return __hiloint2double(
-      __builtin_amdgcn_readlane(__double2hiint(v), lane),
-      __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-__device__ __forceinline__ double2 quad_norms(double errv, double nrm2) {
-  double em = 0.0, ns = 0.0;
-#pragma unroll
-  for (int r = 0; r < kRwQuad; ++r) {
-    const double e = lane_value(errv, 16 * r), m = lane_value(nrm2, 16 * r);
-    em = e > em ? e : em;
-    ns += m;
-  }
-  return make_double2(em, ns);
-}
-
 // One-time build of block L's part of the row store from the GEMV store.
 __global__ __launch_bounds__(256) void k_relayout_rows(
     const double *__restrict__ Dg, const SysDesc *__restrict__ dp,
@@ -1669,77 +1451,6 @@ template __global__ void k_small_stage<true>(StageArgs, const SysDesc *,
 
 template __global__ void k_stage<1, false>(StageArgs, const SysDesc *);
 template __global__ void k_stage<1, true>(StageArgs, const SysDesc *);
-
-// The field at stage time s of pulse p's current attempt: the frozen
-// per-step value of the fixed mode (src/tdse/tdse.cpp:187), the pulse at
-// t + c_s h (adaptive and schedule modes) or a constant.
-__device__ __forceinline__ double stage_field(const Ctl &c, int s, int p,
-                                              const double *__restrict__ Ftab,
-                                              const PulseDev *__restrict__ pulses,
-                                              const double *__restrict__ env) {
-  if (c.fmode == kFieldTable) return Ftab[(long long)p * c.hstride + c.step];
-  if (c.fmode == kFieldPulse)
-    return field_at(pulses[p], env, c.t + cC[s] * c.hc);
-  return c.Fc;
-}
-
-// The step control of one attempt from its error ratio E and |y|^2:
-// accept / reject, the next step size (adaptive), or the next step of a
-// fixed or schedule run.
-__device__ __forceinline__ Ctl control_step(Ctl c, double E, double n2, int p,
-                                            const double *__restrict__ hs) {
-  c.nrm = sqrt(n2);
-  c.err = E;
-  c.attempts++;
-  if (c.mode == kModeAdaptive) {
-    const double hh = c.hc;
-    if (E > 1.0) {
-      // reject: h *= max(0.9 E^(-1/(q-1)), 1/5), error order q = 7
-      const double f = 0.9 / cbrt(sqrt(E));
-      c.h = hh * (f > 0.2 ? f : 0.2);
-      c.rejected++;
-      c.accept = 0;
-    } else {
-      c.accept = 1;
-      c.accepted++;
-      c.hacc = hh;
-      c.nlog++;
-      if (c.last) {
-        c.t = c.t_end;
-        c.done = 1;
-      } else {
-        c.t += hh;
-        if (E < 0.5) {
-          // increase: h *= 0.9 max(E, 5^-8)^(-1/8), stepper order 8
-          const double Em = E > 1.0 / 390625.0 ? E : 1.0 / 390625.0;
-          c.h = hh * (0.9 / sqrt(sqrt(sqrt(Em))));
-        } else {
-          c.h = hh;
-        }
-      }
-    }
-    if (!c.done && c.attempts >= c.max_attempts) {
-      c.done = 1;
-      c.status = -1;
-    }
-    if (!c.done) {
-      c.last = (c.t + c.h >= c.t_end);
-      c.hc = c.last ? (c.t_end - c.t) : c.h;
-    }
-  } else {
-    c.accept = 1;
-    c.accepted++;
-    c.hacc = c.hc;
-    c.nlog++;
-    c.t += c.hc;
-    c.step++;
-    if (c.step >= c.nsteps)
-      c.done = 1;
-    else if (c.mode == kModeSchedule)
-      c.hc = hs[(long long)p * c.hstride + c.step];
-  }
-  return c;
-}
 
 // Reduction of pulse p's per-workgroup (error max, |y|^2) partials in a
 // fixed order and the step control (accept / reject, next step size).  Run
@@ -2002,493 +1713,6 @@ __global__ __launch_bounds__(256) void k_stage1(StageArgs a, const SysDesc *__re
 }
 template __global__ void k_stage1<false>(StageArgs, const SysDesc *);
 template __global__ void k_stage1<true>(StageArgs, const SysDesc *);
-
-// ---------------------------------------------------------------------
-// Persistent row kernel: whole attempts of one pulse in one cooperative
-// launch (every workgroup resident, one per compute unit).  A workgroup owns
-// up to 64 rows of one block.  Four waves compute, a quad each (two or four
-// when a workgroup has more rows): the first kRwReg chunks of a quad's part
-// of the row store stay in registers for the whole launch, further ones in
-// LDS, the rest comes from L2; the rows' 13 stage derivatives stay in LDS.
-// The other four waves poll the neighbour blocks' stage input into one of
-// two LDS copies, so a stage has one workgroup barrier and one exchange.
-//
-// What bounds it: latency.  Per stage (4 x 198, clock64): about 0.9 us from
-// a store to its reader, 0.4 us for the coupling sums and their lane
-// reduction, 0.3 us for the stage algebra; a launch per stage took 5.7 us.
-// Whole attempts 83 -> 31.6 us (4 x 198), 105 -> 34.9 us (6 x 300), 165 ->
-// 72 us (blocks 1201, 1333, 997, where the neighbours' 2198 rows of 16
-// bytes per workgroup weigh as much as the dipoles).  Tried: coupling sums
-// split over all eight waves with a second barrier and an LDS sum (42 and
-// 49 us; a wave64 instruction takes four cycles, and eight waves reducing 32
-// sums each issue more of them than four waves reducing eight), every wave
-// polling and storing (47 us: a poll waits for the acknowledgement of the
-// stores before it), 16 waves (register spills).
-//
-// Exchange.  xb holds four copies of the state; stage g (counted over the
-// launch) uses copy g % 4.  An unset component holds kUnset, a signalling
-// NaN that no arithmetic produces (a raw copy of it is quieted).  The owner
-// of a row stores its stage input with device-scope (write-through) stores;
-// a reader polls the rows it needs with device-scope loads, 16 bytes at a
-// time, until both components are set, so the data is its own flag.  A
-// workgroup that has read every neighbour row of stage g knows that all its
-// readers have finished with copy (g + 3) % 4 (they published stage g after
-// reading stage g - 1), and unsets its own rows there; those stores have
-// landed before it publishes stage g + 2, ahead of any poll of that copy for
-// stage g + 3.  The step control needs every row's error and norm: quads
-// exchange them the same way (rb, three copies by attempt), every workgroup
-// reduces them in k_finalize's order and runs the controller on its own,
-// with the same bits everywhere.
-//
-// Every wait is bounded: past limit_ms a workgroup sets abort_flag and
-// leaves, the others see the flag; the host then restores the state saved
-// by k_rows_begin and runs the attempts with one launch per stage.
-// ---------------------------------------------------------------------
-constexpr unsigned long long kUnset = 0x7FF4C0DEFACE0FF5ull;
-template <int V>
-struct Int {
-  static constexpr int value = V;
-};
-constexpr int kXbCopies = 4;   // copies of the state in exchange
-constexpr int kScDevice = 16;  // sc1: device-scope load / store
-
-typedef unsigned uv4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ bool is_unset(double v) {
-  return (unsigned long long)__double_as_longlong(v) == kUnset;
-}
-
-__device__ __forceinline__ double2 dev_load(__amdgpu_buffer_rsrc_t r,
-                                            unsigned byte) {
-  const uv4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte, 0,
-                                                      kScDevice);
-  return make_double2(__hiloint2double((int)v.y, (int)v.x),
-                      __hiloint2double((int)v.w, (int)v.z));
-}
-
-__device__ __forceinline__ void dev_store(__amdgpu_buffer_rsrc_t r,
-                                          unsigned byte, double2 x) {
-  const uv4 v = {(unsigned)__double2loint(x.x), (unsigned)__double2hiint(x.x),
-                 (unsigned)__double2loint(x.y), (unsigned)__double2hiint(x.y)};
-  __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)byte, 0, kScDevice);
-}
-
-// a value as published: never kUnset
-__device__ __forceinline__ double2 publishable(double2 v) {
-  const double q = __longlong_as_double((long long)(kUnset | (1ull << 51)));
-  return make_double2(is_unset(v.x) ? q : v.x, is_unset(v.y) ? q : v.y);
-}
-
-// Unsets the exchange buffers and saves the state and the control record.
-__global__ __launch_bounds__(256) void k_rows_begin(RowRun a, double2 *Xsave,
-                                                    Ctl *ctl_save) {
-  const double u = __longlong_as_double((long long)kUnset);
-  const double2 unset = make_double2(u, u);
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < kXbCopies * a.N) a.xb[i] = unset;
-  if (i < 3 * a.nquad) a.rb[i] = unset;
-  if (i < a.N) Xsave[i] = a.X[i];
-  if (i == 0) {
-    *ctl_save = *a.ctl;
-    *a.abort_flag = 0;
-  }
-}
-
-template <int kQ>
-__global__ __launch_bounds__(kRwThreads) void k_rows_run(
-    RowRun a, const SysDesc *__restrict__ dp, const RowDesc *__restrict__ rp,
-    const double *__restrict__ Dq) {
-  // chunks of a quad kept in registers: one quad a wave leaves room for them
-  constexpr int kReg = kQ == 1 ? kRwReg : 0;
-  const SysDesc &d = *dp;
-  const RowWg g = a.wg[blockIdx.x];
-  const int t = threadIdx.x, lane = t & 63;
-  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int L = g.L, gauge = d.gauge;
-  const int n0 = L > 0 ? d.off[L] - d.off[L - 1] : 0;
-  const int n1 = L + 1 < d.nb ? d.off[L + 2] - d.off[L + 1] : 0;
-  const int nch0 = (n0 + 63) >> 6, nch = nch0 + ((n1 + 63) >> 6);
-  const int nchp = (nch + 3) & ~3;  // whole groups of four chunks
-  const int nx = n0 + n1;
-  const int nq = (g.nrows + kRwQuad - 1) / kRwQuad, nr4 = nq * kRwQuad;
-
-  // LDS: two copies of the neighbours' stage input (zero padded to whole
-  // groups of chunks), the 13 stage derivatives of the own rows, the
-  // resident chunks of the row store ([quad][chunk])
-  extern __shared__ __align__(16) unsigned char smem[];
-  double2 *xs0 = reinterpret_cast<double2 *>(smem);
-  double2 *Ks = xs0 + 2 * nchp * 64;
-  double2 *Dl = Ks + kStages * nr4;
-  __shared__ Ctl cl;
-  __shared__ double se[256], sn[256];
-  __shared__ int stop;
-  // row s < 12: a_{s+1,j}; rows 12, 13: b, b - bhat
-  __shared__ double coef[kStages + 1][kStages];
-
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)a.xb, (short)0, (int)(kXbCopies * (unsigned)a.N * 16u), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)a.rb, (short)0, (int)(3u * (unsigned)a.nquad * 16u), 0x00020000);
-  constexpr unsigned kOut = 0x80000000u;  // beyond any buffer range
-  const unsigned N = (unsigned)a.N, NQ = (unsigned)a.nquad;
-  const double u_ = __longlong_as_double((long long)kUnset);
-  const double2 unset = make_double2(u_, u_);
-
-  if (t == 0) {
-    cl = a.ctl[0];
-    stop = 0;
-    if (a.limit_ms < 0) {  // no wait at all
-      stop = 1;
-      __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  if (t < (kStages + 1) * kStages) {
-    const int s = t / kStages, j = t - s * kStages;
-    coef[s][j] = s < kStages - 1 ? cA[s + 1][j] : s == kStages - 1 ? cB[j] : cDB[j];
-  }
-  for (int i = t; i < 2 * nchp * 64; i += kRwThreads)
-    xs0[i] = make_double2(0.0, 0.0);
-  const double2 *D2 = reinterpret_cast<const double2 *>(Dq + rp->q_off[L]) +
-                      (long long)(g.row0 / kRwQuad) * nch * 128;
-  for (int i = t; i < nq * g.nlds * 128; i += kRwThreads) {
-    const int qc = i >> 7, q = qc / g.nlds, c = qc - q * g.nlds;
-    const int ch = kReg + c;
-    if (ch < nch) Dl[i] = D2[((long long)q * nch + ch) * 128 + (i & 127)];
-  }
-  __syncthreads();
-
-  if (stop) return;  // uniform
-
-  // true once the wait has to be given up (looked at now and then)
-  long long t_wait = 0;
-  auto give_up = [&](int tries) -> bool {
-    if ((tries & 63) != 0) return false;
-    const long long now = wall_clock64();
-    if (tries == 64) t_wait = now;
-    const bool late = now - t_wait > (long long)a.limit_ms * 100000;
-    if (late)
-      __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    return late || __hip_atomic_load(a.abort_flag, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT) != 0;
-  };
-
-  unsigned buf = 0, rbuf = 0;  // exchange copies of the coming stage, reduction
-  int par = 0;                 // LDS copy of the coming stage's input
-  if (w >= kRwCompute) {
-    // ================= the polling waves =================
-    const int tp = t - 64 * kRwCompute;
-    constexpr int kPoll = kRwThreads - 64 * kRwCompute;
-    const int row_lo = L > 0 ? d.off[L - 1] : 0;
-    const int row_up = L + 1 < d.nb ? d.off[L + 1] : 0;
-    const bool negate = gauge == 0;
-    // U rows per thread, from slot u0 on, of exchange copy b into xs, all
-    // in flight, polled until set
-    auto poll = [&](unsigned b, double2 *xs, int u0, auto width) {
-      constexpr int U = decltype(width)::value;
-      unsigned miss = 0, off[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = (u0 + u) * kPoll + tp;
-        if (i < nx) miss |= 1u << u;
-        off[u] =
-            (b * N + (unsigned)(i < n0 ? row_lo + i : row_up + i - n0)) * 16u;
-      }
-      for (int tries = 1; miss; ++tries) {
-        double2 r[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          r[u] = dev_load(rx, (miss >> u) & 1u ? off[u] : kOut);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (((miss >> u) & 1u) && !is_unset(r[u].x) && !is_unset(r[u].y)) {
-            const int i = (u0 + u) * kPoll + tp;
-            const bool up = i >= n0;
-            xs[up ? nch0 * 64 + i - n0 : i] =
-                up && negate ? make_double2(-r[u].x, -r[u].y) : r[u];
-            miss &= ~(1u << u);
-          }
-        }
-        asm volatile("" ::: "memory");
-        if (miss && give_up(tries)) {
-          stop = 1;
-          break;
-        }
-      }
-    };
-    const int nslots = (nx + kPoll - 1) / kPoll;
-    for (int n = 0; n < a.attempts && !cl.done; ++n) {
-      for (int s = 0; s < kStages; ++s) {
-        double2 *xs = xs0 + par * nchp * 64;
-        if (nslots <= 1) {
-          poll(buf, xs, 0, Int<1>());
-        } else if (nslots <= 2) {
-          poll(buf, xs, 0, Int<2>());
-        } else if (nslots <= 4) {
-          poll(buf, xs, 0, Int<4>());
-        } else {
-          // one row first: while it is not there, the others are not asked for
-          poll(buf, xs, 0, Int<1>());
-          for (int u = 1; u < nslots; u += 8) poll(buf, xs, u, Int<8>());
-        }
-        __syncthreads();
-        if (stop) return;  // uniform over the workgroup
-        buf = (buf + 1) % kXbCopies;
-        par ^= 1;
-      }
-      // ---- step control: every quad's (error max, |y|^2)
-      double em = 0.0, ns = 0.0;
-      for (int i0 = tp; i0 < (int)NQ; i0 += 4 * 256) {
-        double2 p[4];
-        unsigned miss = 0;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (i0 + u * 256 < (int)NQ) miss |= 1u << u;
-        for (int tries = 1; miss; ++tries) {
-          double2 q[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            q[u] = dev_load(
-                rr, (miss >> u) & 1u ? (rbuf * NQ + i0 + u * 256) * 16u : kOut);
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (((miss >> u) & 1u) && !is_unset(q[u].x) && !is_unset(q[u].y)) {
-              p[u] = q[u];
-              miss &= ~(1u << u);
-            }
-          asm volatile("" ::: "memory");
-          if (miss && give_up(tries)) {
-            stop = 1;
-            break;
-          }
-        }
-        if (miss) break;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (i0 + u * 256 < (int)NQ) {
-            em = p[u].x > em ? p[u].x : em;
-            ns += p[u].y;
-          }
-      }
-      se[tp] = em;
-      sn[tp] = ns;
-      __syncthreads();
-      if (stop) return;
-      if (w == kRwCompute) {
-        // k_finalize's tree: halves of 128, 64, then 32 .. 1 across the wave
-        auto mx = [](double p, double q) { return p > q ? p : q; };
-        em = mx(mx(se[lane], se[lane + 128]), mx(se[lane + 64], se[lane + 192]));
-        ns = (sn[lane] + sn[lane + 128]) + (sn[lane + 64] + sn[lane + 192]);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          em = mx(em, __shfl_xor(em, o));
-          ns += __shfl_xor(ns, o);
-        }
-        if (lane == 0) cl = control_step(cl, em, ns, 0, a.hs);
-        // the record is in LDS before the wave's other lanes read it
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_wave_barrier();
-        if (lane < kStages && !cl.done)
-          cl.Fs[lane] = stage_field(cl, lane, 0, a.Ftab, a.pulses, a.env);
-      }
-      rbuf = rbuf == 2 ? 0 : rbuf + 1;
-      __syncthreads();
-    }
-    if (blockIdx.x == 0 && tp == 0) a.ctl[0] = cl;
-    return;
-  }
-
-  // ================= the computing waves =================
-  // wave w owns quads w, w + 4, .. of the workgroup, lanes 0, 16, 32, 48
-  // their rows
-  bool own[kQ];
-  int lr[kQ];
-  unsigned row[kQ];
-  double2 x[kQ], v[kQ], xin[kQ];
-  double e[kQ];
-#pragma unroll
-  for (int m = 0; m < kQ; ++m) {
-    lr[m] = (w + m * kRwCompute) * kRwQuad + (lane >> 4);
-    own[m] = (lane & 15) == 0 && lr[m] < g.nrows;
-    row[m] = (unsigned)(d.off[L] + g.row0 + lr[m]);
-    x[m] = make_double2(0.0, 0.0);
-    e[m] = 0.0;
-    if (own[m]) {
-      x[m] = a.X[row[m]];
-      e[m] = a.E[row[m]];
-    }
-  }
-  // the first quad's first chunks (zeros beyond the last)
-  double2 R[kReg + 1][2];
-#pragma unroll
-  for (int c = 0; c < kReg; ++c)
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-      R[c][p] = c < nch && w < nq
-                    ? D2[((long long)w * nch + c) * 128 + p * 64 + lane]
-                    : make_double2(0.0, 0.0);
-  for (int n = 0; n < a.attempts && !cl.done; ++n) {
-    const double h = cl.hc;
-    const unsigned rnext = rbuf == 2 ? 0 : rbuf + 1;
-    double errv[kQ] = {}, nrm2[kQ] = {};
-#pragma unroll
-    for (int m = 0; m < kQ; ++m) {
-      xin[m] = x[m];
-      if (own[m])
-        dev_store(rx, (buf * N + row[m]) * 16u, publishable(x[m]));
-      // the reduction's copy last read two attempts ago, whose results every
-      // workgroup has used since
-      if (lane == 0 && own[m])
-        dev_store(rr, (rnext * NQ + g.quad0 + w + m * kRwCompute) * 16u, unset);
-    }
-    for (int s = 0; s < kStages; ++s) {
-      const unsigned b1 = (buf + 1) % kXbCopies, b3 = (buf + 3) % kXbCopies;
-      const bool last = s == kStages - 1;
-      const double2 *xs = xs0 + par * nchp * 64 + lane;
-      // while the stage input arrives: the tableau sums of the next one but
-      // for k_s (stage_row's terms in stage_row's order)
-      const double F = cl.Fs[s];
-      const double co = h * coef[s][s];
-      double2 err[kQ] = {};
-#pragma unroll
-      for (int m = 0; m < kQ; ++m) {
-        if (!own[m]) continue;
-        v[m] = x[m];
-        if (!last) {
-#pragma unroll 4
-          for (int j = 0; j < s; ++j) {
-            const double cj = h * coef[s][j];
-            const double2 kj = Ks[j * nr4 + lr[m]];
-            v[m].x = fma(cj, kj.x, v[m].x);
-            v[m].y = fma(cj, kj.y, v[m].y);
-          }
-        } else {
-#pragma unroll 4
-          for (int j = 0; j < kStages - 1; ++j) {
-            const double cb = h * coef[kStages - 1][j], cd = h * coef[kStages][j];
-            const double2 kj = Ks[j * nr4 + lr[m]];
-            v[m].x = fma(cb, kj.x, v[m].x);
-            v[m].y = fma(cb, kj.y, v[m].y);
-            err[m].x = fma(cd, kj.x, err[m].x);
-            err[m].y = fma(cd, kj.y, err[m].y);
-          }
-        }
-      }
-      __syncthreads();
-      if (stop) return;  // uniform over the workgroup
-#pragma unroll
-      for (int m = 0; m < kQ; ++m) {
-        const int q = w + m * kRwCompute;
-        if (q >= nq) continue;  // uniform over the wave
-        double2 acc[4] = {};
-        // every x is read a group of four chunks ahead (past the last group
-        // that stays inside the LDS buffer and is not used)
-        double2 xn[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) xn[u] = xs[u * 64];
-#pragma unroll
-        for (int c0 = 0; c0 < kReg; c0 += 4) {
-          if (c0 < nch) {
-            double2 xc[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              xc[u] = xn[u];
-              xn[u] = xs[(c0 + 4 + u) * 64];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-              quad_fma(acc, R[c0 + u][0], R[c0 + u][1], xc[u]);
-          }
-        }
-        int c = kReg;
-        const int cl1 = min(c + g.nlds, nch);
-        const double2 *Dr = Dl + ((long long)q * g.nlds - c) * 128 + lane;
-#pragma unroll 4
-        for (; c < cl1; ++c)
-          quad_fma(acc, Dr[c * 128], Dr[c * 128 + 64], xs[c * 64]);
-        if (c < nch) {
-          // the chunks past the LDS share
-          const double2 *Dg = D2 + (long long)q * nch * 128 + lane;
-#pragma unroll 4
-          for (; c < nch; ++c)
-            quad_fma(acc, Dg[c * 128], Dg[c * 128 + 64], xs[c * 64]);
-        }
-        const double2 cs = quad_reduce(acc, lane);
-        if (!own[m]) continue;
-        const double2 k =
-            stage_deriv(gauge, e[m], xin[m], F, cs, make_double2(0.0, 0.0));
-        if (!last) {
-          v[m].x = fma(co, k.x, v[m].x);
-          v[m].y = fma(co, k.y, v[m].y);
-          xin[m] = v[m];
-          // the rows unset a stage ago have landed
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          dev_store(rx, (b1 * N + row[m]) * 16u, publishable(v[m]));
-        } else {
-          const double cb = h * cB[kStages - 1], cd = h * cDB[kStages - 1];
-          v[m].x = fma(cb, k.x, v[m].x);
-          v[m].y = fma(cb, k.y, v[m].y);
-          err[m].x = fma(cd, k.x, err[m].x);
-          err[m].y = fma(cd, k.y, err[m].y);
-          const double2 k1 = Ks[lr[m]];
-          const double ex = fabs(err[m].x) / (cl.atol + cl.rtol * (fabs(x[m].x) +
-                                                         h * fabs(k1.x)));
-          const double ey = fabs(err[m].y) / (cl.atol + cl.rtol * (fabs(x[m].y) +
-                                                         h * fabs(k1.y)));
-          errv[m] = ex > ey ? ex : ey;
-          nrm2[m] = abs2(v[m].x, v[m].y);
-        }
-        Ks[s * nr4 + lr[m]] = k;
-      }
-      // copy b3 (stage g - 1's) has been read by all its readers
-#pragma unroll
-      for (int m = 0; m < kQ; ++m)
-        if (own[m]) dev_store(rx, (b3 * N + row[m]) * 16u, unset);
-      buf = b1;
-      par ^= 1;
-    }
-    // ---- step control
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int m = 0; m < kQ; ++m) {
-      const int q = w + m * kRwCompute;
-      if (q >= nq) continue;
-      const double2 en = quad_norms(errv[m], nrm2[m]);
-      if (lane == 0)
-        dev_store(rr, (rbuf * NQ + g.quad0 + q) * 16u, publishable(en));
-    }
-    __syncthreads();
-    if (stop) return;
-    __syncthreads();
-    if (cl.accept) {
-#pragma unroll
-      for (int m = 0; m < kQ; ++m) {
-        if (!own[m]) continue;
-        x[m] = make_double2(v[m].x / cl.nrm, v[m].y / cl.nrm);
-        if ((int)row[m] == a.track && cl.nlog >= 1 && cl.nlog <= a.logcap) {
-          LogEnt le;
-          le.t = cl.t;
-          le.h = cl.hacc;
-          le.pop = abs2(x[m].x, x[m].y);
-          a.log[cl.nlog - 1] = le;
-        }
-      }
-    }
-    rbuf = rnext;
-  }
-#pragma unroll
-  for (int m = 0; m < kQ; ++m)
-    if (own[m]) a.X[row[m]] = x[m];
-}
-
-template __global__ void k_rows_run<1>(RowRun, const SysDesc *,
-                                        const RowDesc *, const double *);
-template __global__ void k_rows_run<2>(RowRun, const SysDesc *,
-                                        const RowDesc *, const double *);
-template __global__ void k_rows_run<4>(RowRun, const SysDesc *,
-                                        const RowDesc *, const double *);
-
 // The rows of workgroup blk of k_apply (also its grouped form).
 __device__ __forceinline__ void apply_block(double2 *__restrict__ X,
                                             const double2 *__restrict__ Y,

@@ -63,6 +63,34 @@ struct RowRun {
   LogEnt *log;
   int logcap, track, N, nquad, attempts;
   int limit_ms;          // time limit of one wait
+  int start_ms;          // > 0: not cooperative, wait for all workgroups
+  int *arrived;          // workgroups that run
+};
+
+// The persistent tile kernel, likewise.
+struct TileRun {
+  const TileWg *wg;
+  const TileSeg *seg;
+  const int *nslot;      // D^T x_L slots per column block of every pair
+  const double *Dg;
+  double2 *X;
+  const double *E;
+  double2 *xb;           // stage inputs in exchange: 3 x N
+  double2 *pb;           // coupling partials in exchange: 3 x part_n
+  double2 *rb;           // per-workgroup (error max, |y|^2): 3 x workgroups
+  Ctl *ctl;
+  int *abort_flag;
+  const double *hs;
+  const double *Ftab;
+  const PulseDev *pulses;
+  const double *env;
+  LogEnt *log;
+  int logcap, track, N, nwg, njobs, attempts;
+  int limit_ms, start_ms;
+  int *arrived;
+  int xs_rows;           // LDS rows of the stage input (row part)
+  int xs_segs;           // LDS column blocks of the stage input
+  int xs_pieces;         // pieces of 64 rows it is fetched in, at most
 };
 
 // The coupling operands of every member of a grouped GEMM launch, passed
@@ -140,7 +168,12 @@ __global__ void k_small_stage(StageArgs a, const SysDesc *d, const RowDesc *rd,
 __global__ void k_relayout_rows(const double *Dg, const SysDesc *d,
                                 const RowDesc *rd, int njobs, int L,
                                 long long nelem, double *Dq);
-__global__ void k_rows_begin(RowRun a, double2 *Xsave, Ctl *ctl_save);
+// Unsets the exchange buffers and saves the state and the control record.
+__global__ void k_rows_begin(double2 *xb, int nxb, double2 *pb, int npb,
+                             double2 *rb, int nrb, const double2 *X, int N,
+                             double2 *Xsave, const Ctl *ctl, Ctl *ctl_save,
+                             int *abort_flag, int *arrived);
+__global__ void k_tiles_run(TileRun a, const SysDesc *d, const TileDesc *td);
 template <int kQ>
 __global__ void k_rows_run(RowRun a, const SysDesc *d, const RowDesc *rd,
                            const double *Dq);

@@ -61,6 +61,94 @@ def test_persistent_equals_stage_launches(mpci, s, gauge):
         assert np.array_equal(a, b)
 
 
+# around the units of 128 x 256, the 16-row groups, one and two segments a
+# workgroup, groups in registers, in LDS and streamed, narrow column blocks
+TILE_SHAPES = [[1777, 1801], [2049, 1800, 16], [40, 13000, 257],
+               [300, 6200, 1100], [2400, 2500, 1300], [1, 4200, 3],
+               [9] * 28 + [1300, 2500]]
+
+
+@pytest.mark.parametrize("gauge", ["v", "l"])
+@pytest.mark.parametrize("s", TILE_SHAPES)
+def test_persistent_tiles_against_oracle(mpci, oracle, s, gauge):
+    """The persistent tile kernel (larger systems): two frozen-field steps
+    against the oracle within 1e-12, the run split in two calls bit for bit,
+    the adaptive mode's counts against stage launches (another summation
+    order: the state within 1e-11), and the way back when a launch gives up."""
+    from mpci import synth
+    E, D = synth.system_arrays(s, seed=sum(s))
+    g, o = mpci.System(E, D, gauge=gauge), oracle.System(E, D, gauge=gauge)
+    # past the row form's range
+    assert 8 * g.dipole_elements > 24 << 20 or sum(-(-n // 16) for n in s) > 256
+    x0 = state(g.N, 7)
+    F = np.array([[0.04, -0.03, 0.02]])
+
+    def prop(graph=True):
+        p = mpci.Propagator(g)
+        p.set_graph(graph)
+        p.set_state(x0)
+        p.set_pulse(mpci.Pulse.sine(0.04 ** 2, 0.7, 2, gauge))
+        return p
+
+    a = prop()
+    a.prop_fixed(0.0, 0.1, F)
+    xr = x0.copy()
+    for k in range(3):
+        xr = o.step(F[0, k], xr, 0.1)
+        xr /= np.sqrt(xr @ xr)
+    assert np.abs(a.get_state() - xr).max() < 1e-12
+    b = prop()
+    b.prop_fixed(0.0, 0.1, F[:, :1])
+    b.prop_fixed(0.1, 0.1, F[:, 1:])
+    assert np.array_equal(a.get_state(), b.get_state())
+    b.set_state(x0)
+    b.set_wait_limit(-1)
+    b.prop_fixed(0.0, 0.1, F)
+    assert np.abs(a.get_state() - b.get_state()).max() < 1e-14
+    c = prop(False)
+    a.set_state(x0)
+    st = [p.prop_adaptive(3.0, 6.0, 1.5, 1e-9, 1e-9)[0][0] for p in (a, c)]
+    assert st[0].accepted == st[1].accepted and st[0].rejected >= 1
+    assert st[0].rejected == st[1].rejected
+    assert np.abs(a.get_state() - c.get_state()).max() < 1e-11
+
+
+CHILD = """
+import sys
+import numpy as np
+sys.path[:0] = [%r, %r]
+import mpci
+from mpci import synth
+from test_gpu_rows import state
+E, D = synth.system_arrays(%r, seed=9)
+g = mpci.System(E, D)
+p = mpci.Propagator(g)
+p.set_state(state(g.N, 3))
+p.prop_fixed(0.0, 0.1, np.full((1, 20), 0.02))
+np.save(%r, p.get_state())
+"""
+
+
+@pytest.mark.parametrize("s", [[300, 257, 513], [1777, 1801]])
+def test_second_process(mpci, tmp_path, s):
+    """A second process is refused cooperative launches while this one holds
+    them; its ordinary launch gives the same bits."""
+    import os
+    import subprocess
+    import sys
+    from mpci import synth
+    E, D = synth.system_arrays(s, seed=9)
+    g = mpci.System(E, D)
+    p = mpci.Propagator(g)
+    p.set_state(state(g.N, 3))
+    p.prop_fixed(0.0, 0.1, np.full((1, 20), 0.02))
+    out = str(tmp_path / "x.npy")
+    code = CHILD % (os.path.dirname(os.path.dirname(mpci.__file__)),
+                    os.path.dirname(os.path.abspath(__file__)), s, out)
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=100)
+    assert np.array_equal(np.load(out), p.get_state())
+
+
 def test_gives_up_and_goes_on(mpci):
     """A launch that may not wait leaves at once; the run goes on with one
     launch per stage from where it began, and so do later runs."""
