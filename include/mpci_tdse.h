@@ -205,7 +205,8 @@ int mpci_prop_schedule(mpci_prop *prop, const double *t0, int n,
  * mpci_prop_adaptive from the current states, keeping the state after every
  * ckpt_every accepted steps, then sweeps backward through the same discrete
  * map (accepted steps only, schedule frozen, renormalisation included),
- * recomputing each checkpoint segment.  Objective per pulse:
+ * recomputing each checkpoint segment but the last, whose steps the forward
+ * pass keeps.  Objective per pulse:
  * J[p] = sum_k W[k] |c_{k,p}(t1[p])|^2 (e.g. the ground-state population or
  * the yield mask of pes::genPES2e, src/pes/pes.cpp:199-213).  Output:
  * grad[p * grad_stride + k] = dJ[p] / d env_p[k]; nsteps[p] and hlog

@@ -180,11 +180,13 @@ struct Ctl {
                        // set on the device when the attempt is set up
 };
 
-// Optional stores written while stepping (adjoint support).
+// Optional stores written while stepping (adjoint support).  Step n of a
+// pulse goes to slot n % cap.
 struct StepStore {
-  double2 *xs;      // stage inputs 1..12 of every step: [step][12][N x P]
-  double2 *xn;      // normalised states after every step: [step + 1][N x P]
-  double *nrm;      // ||y|| of every step: [step][P]
+  double2 *xs;      // stage inputs 1..12 of a step: [slot][12][N x P]
+  double2 *xn;      // normalised state after a step: [slot + 1][N x P]
+  double *nrm;      // ||y|| of a step: [slot][P]
+  int cap;
   double2 *ckpt;    // adaptive mode: state after every ckpt_every accepted
   int ckpt_every;   //   steps, slot accepted / ckpt_every, ckpt_cap slots
   int ckpt_cap;

@@ -1423,6 +1423,7 @@ static StageArgs stage_args(mpci_prop *pr, int s) {
   a.red = pr->red.p;
   a.ctl = pr->ctl.p;
   a.xs_store = pr->store.xs;
+  a.store_cap = pr->store.cap;
   a.NP = pr->NP;
   a.s = s;
   return a;
@@ -2386,13 +2387,36 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
       return fail(MPCI_ERR_ARG, "grad_stride smaller than n_env");
   }
   const int K = ckpt_every;
-  DevBuf<double2> ckpt, xs_store, xn_store, mu, lam, lamx, xfinal;
+  DevBuf<double2> ckpt, xs_store, xn_store, mu, nu, ly, lam, lamx, xfinal;
   DevBuf<double> nrm_store, tn_tab, hn_tab, gdev, red2, dotv, Wd;
   // device bytes held by the adjoint's own buffers, and their peak
   long long held = 0, peak = 0;
   auto hold = [&](long long bytes) {
     held += bytes;
     peak = std::max(peak, held);
+  };
+  // What the sweep needs of a segment's K steps.  The forward pass keeps it
+  // too, so the steps of the last segment are not propagated again (all of
+  // them, for a run of up to K steps: 16 pulses on 4000 x 4, 7 steps, 44.5 ->
+  // 31.7 ms); without room for it beside the checkpoints they are.
+  bool kept = false;
+  auto alloc_segment = [&]() -> int {
+    TRY(xs_store.alloc((size_t)K * (kStages - 1) * NP));
+    TRY(xn_store.alloc((size_t)(K + 1) * NP));
+    TRY(nrm_store.alloc((size_t)K * P));
+    hold((long long)(xs_store.bytes() + xn_store.bytes() + nrm_store.bytes()));
+    return MPCI_OK;
+  };
+  auto drop_segment = [&]() {
+    if (kept)
+      held -= (long long)(xs_store.bytes() + xn_store.bytes() +
+                          nrm_store.bytes());
+    (void)xs_store.alloc(0);
+    (void)xn_store.alloc(0);
+    (void)nrm_store.alloc(0);
+    kept = false;
+    pr->store.xs = pr->store.xn = nullptr;
+    pr->store.nrm = nullptr;
   };
   // Checkpoint slot j holds the state after j K accepted steps.  The store
   // grows with the forward pass, which runs in chunks of at most logcap
@@ -2403,7 +2427,13 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
     if (need <= ckcap) return MPCI_OK;
     const int cap = std::max(need, ckcap + ckcap / 2);
     DevBuf<double2> bigger;
-    TRY(bigger.alloc((size_t)cap * NP));
+    if (bigger.alloc((size_t)cap * NP) != MPCI_OK) {
+      if (!kept) return MPCI_ERR_HIP;
+      (void)hipGetLastError();
+      HIPCHK(hipStreamSynchronize(pr->stream));
+      drop_segment();
+      TRY(bigger.alloc((size_t)cap * NP));
+    }
     hold((long long)bigger.bytes());
     if (ckcap > 0)
       HIPCHK(hipMemcpyAsync(bigger.p, ckpt.p, ckpt.bytes(),
@@ -2438,7 +2468,17 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
   auto tf = std::chrono::steady_clock::now();
   pr->store = StepStore{};
   pr->store.ckpt_every = K;
+  pr->store.cap = K;
   TRY(grow_ckpt(2));
+  kept = alloc_segment() == MPCI_OK;
+  if (kept) {
+    pr->store.xs = xs_store.p;
+    pr->store.xn = xn_store.p;
+    pr->store.nrm = nrm_store.p;
+  } else {
+    (void)hipGetLastError();
+    drop_segment();
+  }
   HIPCHK(hipMemcpyAsync(ckpt.p, pr->X.p, sizeof(double2) * NP,
                         hipMemcpyDeviceToDevice, pr->stream));
   std::vector<Ctl> c;
@@ -2489,7 +2529,7 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
     hipLaunchKernelGGL(k_adj_seed, dim3(nb), dim3(256), 0, pr->stream,
                        pr->X.p, Wd.p, N, P, lam.p);
     HIPCHK(hipGetLastError());
-    TRY(red2.alloc((size_t)pr->nblk * P));
+    TRY(red2.alloc((size_t)kStages * pr->nblk * P));
     TRY(dotv.alloc(P));
     // J_p = <x, W x>: reuse the dot kernels on (x, x * W) = (x, lam) / 2
     hipLaunchKernelGGL(k_dot_partial, dim3(pr->nblk), dim3(256), 0,
@@ -2504,16 +2544,15 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
   }
 
   // ---- backward, one checkpoint segment at a time ----------------------
-  TRY(xs_store.alloc((size_t)K * (kStages - 1) * NP));
-  TRY(xn_store.alloc((size_t)(K + 1) * NP));
-  TRY(nrm_store.alloc((size_t)K * P));
-  TRY(mu.alloc((size_t)kStages * NP));
+  if (!xs_store.p) TRY(alloc_segment());
+  TRY(mu.alloc(NP));
+  TRY(nu.alloc((size_t)kStages * NP));
+  TRY(ly.alloc(NP));
   TRY(tn_tab.alloc((size_t)K * P));
   TRY(hn_tab.alloc((size_t)K * P));
   TRY(gdev.alloc((size_t)K * kStages * P));
   hold((long long)(lam.bytes() + lamx.bytes() + red2.bytes() + dotv.bytes() +
-                   xs_store.bytes() + xn_store.bytes() + nrm_store.bytes() +
-                   mu.bytes() + tn_tab.bytes() + hn_tab.bytes() +
+                   mu.bytes() + nu.bytes() + ly.bytes() + tn_tab.bytes() + hn_tab.bytes() +
                    gdev.bytes()));
   for (int p = 0; p < P; ++p)
     for (int k = 0; k < grad_stride; ++k) grad[(size_t)p * grad_stride + k] = 0;
@@ -2530,11 +2569,11 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
     }
     if (kmax == 0) continue;
     // recompute the segment from checkpoint j, storing what the sweep needs
-    HIPCHK(hipMemcpyAsync(pr->X.p, ckpt.p + (size_t)j * NP,
+    // (the last one's is there from the forward pass)
+    const bool stored = kept && j == nseg - 1;
+    HIPCHK(hipMemcpyAsync(xn_store.p, ckpt.p + (size_t)j * NP,
                           sizeof(double2) * NP, hipMemcpyDeviceToDevice,
                           pr->stream));
-    HIPCHK(hipMemcpyAsync(xn_store.p, pr->X.p, sizeof(double2) * NP,
-                          hipMemcpyDeviceToDevice, pr->stream));
     std::fill(hs.begin(), hs.end(), 0.0);
     std::fill(hn.begin(), hn.end(), 0.0);
     std::fill(tn.begin(), tn.end(), 0.0);
@@ -2548,11 +2587,16 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
       }
     }
     pr->store = StepStore{};
-    pr->store.xs = xs_store.p;
-    pr->store.xn = xn_store.p;
-    pr->store.nrm = nrm_store.p;
-    TRY(run_schedule(pr, ts.data(), nloc.data(), K, hs.data()));
-    pr->store = StepStore{};
+    if (!stored) {
+      HIPCHK(hipMemcpyAsync(pr->X.p, xn_store.p, sizeof(double2) * NP,
+                            hipMemcpyDeviceToDevice, pr->stream));
+      pr->store.xs = xs_store.p;
+      pr->store.xn = xn_store.p;
+      pr->store.nrm = nrm_store.p;
+      pr->store.cap = K;
+      TRY(run_schedule(pr, ts.data(), nloc.data(), K, hs.data()));
+      pr->store = StepStore{};
+    }
     TRY(h2d(pr, tn_tab.p, tn.data(), sizeof(double) * K * P));
     TRY(h2d(pr, hn_tab.p, hn.data(), sizeof(double) * K * P));
     // coupling kernels skip finished pulses: mark all live for the sweep
@@ -2567,6 +2611,8 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
       a.pulses = pr->pulses.p;
       a.env = pr->env.p;
       a.mu = mu.p;
+      a.nu = nu.p;
+      a.ly = ly.p;
       a.lam = lam.p;
       a.lamx = lamx.p;
       a.x1 = xn_store.p + (size_t)(k + 1) * NP;
@@ -2576,7 +2622,6 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
       a.nrm = nrm_store.p + (size_t)k * P;
       a.tn = tn_tab.p + (size_t)k * P;
       a.hn = hn_tab.p + (size_t)k * P;
-      a.red = red2.p;
       a.NP = NP;
       hipLaunchKernelGGL(k_dot_partial, dim3(pr->nblk), dim3(256), 0,
                          pr->stream, a.x1, lam.p, N, P, red2.p);
@@ -2586,15 +2631,17 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
                          pr->stream, a, pr->ddesc.p);
       HIPCHK(hipGetLastError());
       for (int st = kStages - 1; st >= 0; --st) {
-        TRY(enqueue_tile(pr, mu.p + (size_t)st * NP, st));
+        TRY(enqueue_tile(pr, mu.p, st));
         a.s = st;
+        a.red = red2.p + (size_t)st * pr->nblk * P;
         hipLaunchKernelGGL(k_adj_stage, dim3(pr->nblk), dim3(256), 0,
                            pr->stream, a, pr->ddesc.p);
-        hipLaunchKernelGGL(k_reduce_final, dim3(P), dim3(256), 0, pr->stream,
-                           red2.p, pr->nblk, P,
-                           gdev.p + ((size_t)k * kStages + st) * P);
         HIPCHK(hipGetLastError());
       }
+      hipLaunchKernelGGL(k_reduce_final, dim3(P, kStages), dim3(256), 0,
+                         pr->stream, red2.p, pr->nblk, P,
+                         gdev.p + (size_t)k * kStages * P);
+      HIPCHK(hipGetLastError());
       std::swap(lam.p, lamx.p);
     }
     HIPCHK(hipStreamSynchronize(pr->stream));

@@ -18,7 +18,8 @@ struct StageArgs {
   const double *E;       // energies (N)
   double *red;           // per-block (error max, |y|^2) partials
   Ctl *ctl;              // per-pulse control (P), with the stage fields
-  double2 *xs_store;     // optional: stage inputs of every step
+  double2 *xs_store;     // optional: stage inputs (StepStore::xs)
+  int store_cap;
   long long NP;
   int s;                 // stage 0..12
   int pad;
@@ -30,7 +31,9 @@ struct AdjArgs {
   const double *E;
   const PulseDev *pulses;
   const double *env;
-  double2 *mu;           // 13 stage adjoints, stride NP
+  double2 *mu;           // mu_s; after stage s mu_{s-1}
+  double2 *nu;           // nu_s, stride NP
+  double2 *ly;           // lam_y
   double2 *lam;          // adjoint of the state after the step (input)
   double2 *lamx;         // adjoint of the state before the step (output)
   const double2 *x1;     // normalised state after the step
@@ -191,6 +194,7 @@ __global__ void k_adj_seed(const double2 *X, const double *W, int N, int P,
                            double2 *lam);
 __global__ void k_dot_partial(const double2 *a, const double2 *b, int N, int P,
                               double *red);
+// grid (P, sets): set y from red + y nblk P to out + y P
 __global__ void k_reduce_final(const double *red, int nblk, int P,
                                double *out);
 __global__ void k_adj_init(AdjArgs a, const SysDesc *d);

@@ -195,3 +195,39 @@ def test_checkpoint_store_sized_by_the_run(mpci):
     # the slots a chunk can fill, at most one chunk of attempts ahead
     assert st.ckpt_slots <= (nst[0] + 4096) // K + 2
     assert st.peak_bytes >= st.ckpt_slots * g.N * 16
+
+
+@pytest.mark.parametrize("P", [1, 3])
+def test_gradient_does_not_depend_on_the_segments(mpci, P):
+    """The last segment's steps come from the forward pass, the others are
+    propagated again: one step a segment, segments that end with the run,
+    before it and after it, and pulses whose last steps lie in different
+    segments give one gradient (sums of the same terms, grouped differently:
+    1e-12)."""
+    from mpci import synth
+    E, D = synth.system_arrays([20, 33, 17], seed=23)
+    g = mpci.System(E, D)
+    W = np.zeros(g.N)
+    W[:5] = 1.0
+    w, T = 0.7, 12.0
+    t1 = np.linspace(4.0, T, P)
+
+    def run(K):
+        prop = mpci.Propagator(g, P=P)
+        for p in range(P):
+            prop.set_state(synth.ground_state(g.N), p)
+            prop.set_pulse(mpci.Pulse.pwl(synth.uniform(9, 10 * p, 8, 0.0,
+                                                        0.04), w, T), p)
+        J, grad, nst, _, st = prop.adjoint(0.0, t1, 0.05, W, ckpt_every=K,
+                                           atol=1e-7, rtol=1e-7)
+        assert st.segments == math.ceil(nst.max() / K)
+        return J, grad, nst, prop.get_state(P - 1)
+
+    J, grad, nst, x = run(1000)
+    n = int(nst.max())
+    assert n >= 6 and np.linalg.norm(grad[0]) > 0
+    for K in (1, 3, n - 1, n, n + 1):
+        Jk, gk, nk, xk = run(K)
+        assert np.array_equal(nk, nst) and np.array_equal(xk, x)
+        assert np.array_equal(Jk, J)
+        assert rel(gk, grad) < 1e-12
