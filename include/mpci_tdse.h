@@ -254,11 +254,12 @@ int mpci_prop_observables(mpci_prop *prop, int electrons, double threshold,
 
 /* Launch the 13-stage step as one captured hipGraph (1, default) or as
  * individual launches (0).  With 1, one pulse on a system of more than one
- * block runs its attempts inside one cooperative launch instead: where the
- * dipoles take at most 24 MiB and a compute unit's share is at most 16 rows,
- * with the bits of the fused small-system stages (below), otherwise with the
- * coupling sums in an order of its own (equal to rounding, and the same from
- * run to run).  A process that is refused cooperative launches, because
+ * block runs its attempts inside one cooperative launch instead: where a
+ * compute unit's share is at most 16 rows, with the bits of the fused
+ * small-system stages (below), otherwise with the coupling sums in an order
+ * of its own (equal to rounding, and the same from run to run).  So does a
+ * batch of few pulses on such a small system, every pulse with the bits of
+ * its run alone. A process that is refused cooperative launches, because
  * another one on the device holds them, makes an ordinary launch of it. */
 int mpci_prop_set_graph(mpci_prop *prop, int enable);
 /* The workgroups of that launch wait for one another; a wait is given up
@@ -300,7 +301,7 @@ int mpci_prop_gemm_config(mpci_prop *prop, int *wm, int *wn, int *ks,
                           double *ms, int *kind, int *tk, int *fm, int *fn);
 /* The autotuner's candidate tiles: their number, and pinning one of them
  * (0 <= index < count) on a batched propagator in place of the autotuned
- * choice (it is timed as the autotuner times it; mpci_prop_gemm_config
+ * choice, and of the cooperative launch (it is timed as the autotuner times it; mpci_prop_gemm_config
  * then reports it).  For tests and tuning studies; the pin holds for this
  * propagator only. */
 int mpci_prop_gemm_candidates(int *count);

@@ -80,6 +80,7 @@ constexpr int kRwThreads = 512;  // persistent form: eight waves,
 constexpr int kRwCompute = 4;    // four compute, four poll
 constexpr int kRwReg = 16;       // chunks of a wave's first quad in registers
 constexpr int kRwMaxRows = 64;   // rows of a workgroup
+constexpr int kRwSlots = 8;      // pulses a workgroup holds at a time
 
 struct RowDesc {
   long long q_off[kMaxBlocks];  // block L's first quad in Dq (doubles)

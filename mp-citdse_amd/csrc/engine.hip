@@ -129,9 +129,11 @@ struct mpci_prop {
   // (k_small_stage, four rows per workgroup) instead of GEMV tile + stage
   bool small = false;
   int nblk_small = 0;  // quads: partials of its step control
-  // one pulse, whole runs in one cooperative launch (k_rows_run)
+  // whole runs in one cooperative launch (k_rows_run)
   bool rows = false;
-  int rows_wg = 0;       // workgroups
+  int rows_wg = 0;       // workgroups of a pulse
+  int rows_grp = 1;      // groups of workgroups
+  int rows_slots = 1;    // pulses a group runs at a time
   size_t rows_lds = 0;   // dynamic LDS bytes
   int rows_kq = 1;       // quads per computing wave
   int wait_limit_ms = 0; // time limit of one wait inside the launch
@@ -936,28 +938,36 @@ static int autotune_gemm(mpci_prop *pr) {
 // 8.6 MB, even at 15 MB, 0.85x at 24 MB.
 constexpr long long kSmallPathBytes = 12LL << 20;
 // The same for whole runs in one persistent launch: the row form
-// (k_rows_run) up to here, the tile form (k_tiles_run) past it, where the
-// row store, which holds every dipole twice, outgrows registers and LDS.  Per
+// (k_rows_run) while a compute unit's share is at most 16 rows (a quad a
+// wave, its chunks in registers), the tile form (k_tiles_run) past it.  Per
 // attempt, row against tile form: 6 x 300 (3.6 MB) 34.9 against 72 us, 4 x
-// 700 (12 MB) 51 against 100 us, 4 x 1000 (24 MB) 87 against 104 us, 4 x 1150
-// (32 MB) 186 against 113 us.  The launches these replace took 105 us (6 x
-// 300), 164 us (4 x 900), 200 us (4 x 1500), 474 us (He_test.yaml shape),
-// 910 us (He 4 x 4000); the tile form takes 127, 355 and 763 us there.
-constexpr long long kRowsBytes = 24LL << 20;
+// 700 (12 MB) 51 against 100 us, 4 x 1000 (24 MB) 87 against 104 us, 2 x 2048
+// (34 MB) 82 against 103 us; with more rows, 4 x 1150 (32 MB) 186 against 113
+// us, 12 x 500 (22 MB) 120 against 96 us, 30 x 250 (15 MB) 200 against 89
+// us.  The launches these replace took 105 us (6 x 300), 164 us (4 x 900),
+// 200 us (4 x 1500), 474 us (He_test.yaml shape), 910 us (He 4 x 4000); the
+// tile form takes 127, 355 and 763 us there.
 constexpr int kWaitLimitMs = 20000;  // time limit of one wait in them
 // Time limit of the start of an ordinary launch: two processes' launches
 // that hold half the device each let go of it after this.
 constexpr int kStartLimitMs = 200;
 
+// Workgroups of 16 rows of one block that hold all rows.
+static int row_groups(const mpci_system *sys) {
+  int n = 0;
+  for (int L = 0; L < sys->nb; ++L) n += (sys->s[L] + 15) / 16;
+  return n;
+}
+
 // The workgroups of the persistent row kernel: at most one per compute unit,
 // each inside one block, 16 rows (one pass of its four quads) while that
 // fits the device, else dealt to the blocks by the elements of their rows.
 // Returns false when the form does not apply to the system.
-static bool plan_rows(const mpci_prop *pr, std::vector<RowWg> &wg,
+static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
                       size_t *lds, int *kq) {
   const mpci_system *sys = pr->sys;
   wg.clear();
-  if (pr->P != 1 || sys->nb < 2 || 64LL * sys->N >= (1LL << 31)) return false;
+  if (sys->nb < 2 || 64LL * nslot * sys->N >= (1LL << 31)) return false;
   int coop = 0, lds_max = 0;
   if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch,
                             sys->device) != hipSuccess || !coop)
@@ -999,7 +1009,7 @@ static bool plan_rows(const mpci_prop *pr, std::vector<RowWg> &wg,
       g.quad0 = sys->hrow.quad0[L] + r / kRwQuad;
       const int nq = (g.nrows + kRwQuad - 1) / kRwQuad;
       const long long base = 2LL * ((nch + 3) / 4 * 4) * 64 * 16 +
-                             kStages * nq * kRwQuad * 16LL;
+                             nslot * (kStages + 2LL) * nq * kRwQuad * 16;
       if (base > room) return false;
       g.nlds = (int)std::min<long long>(std::max(nch - reg, 0),
                                         (room - base) / (nq * 2048LL));
@@ -1008,6 +1018,34 @@ static bool plan_rows(const mpci_prop *pr, std::vector<RowWg> &wg,
     }
   }
   return (int)wg.size() <= sys->ncu;
+}
+
+// Whether a batch runs in the persistent row form: pulses are independent, so
+// groups of workgroups take some each and a group runs a stage of each of its
+// pulses in turn, which hides one's exchange behind the others'.  A pulse
+// then costs its group about 20 us an attempt while the rows' chunks fit in
+// registers, and more past that; the batched launches cost 110 to 300 us an
+// attempt at any P.  Measured, row form against batched launches, in us per
+// attempt: 60 x 8, P = 5 28 / 128, P = 40 97 / 139, P = 64 151 / 148; 198 x
+// 4, P = 5 45 / 148, P = 16 81 / 158, P = 40 197 / 168; 300 x 6, P = 5 66 /
+// 171, P = 16 159 / 194, P = 40 392 / 250; 800 x 5, P = 3 93 / 270, P = 8
+// 275 / 276; 2000 x 2, P = 2 105 / 314, P = 8 456 / 342; 1500, 1000, 1500,
+// P = 3 257 / 304, P = 5 420 / 312.
+static bool rows_pay(const mpci_prop *pr) {
+  const mpci_system *sys = pr->sys;
+  const int n16 = row_groups(sys);
+  int chunks = 0, smax = 0;
+  for (int L = 0; L < sys->nb; ++L) {
+    chunks = std::max(chunks, row_chunks(sys, L));
+    smax = std::max(smax, sys->s[L]);
+  }
+  if (n16 > sys->ncu) return false;
+  const int groups = std::min(pr->P, sys->ncu / n16);
+  const int each = (pr->P + groups - 1) / groups;
+  const double pulse = 20.0 + 2.4 * std::max(chunks - kRwReg, 0);
+  const double batched = 110.0 + 0.15 * std::min(smax, 1000) +
+                         2.5e-6 * (double)sys->S * pr->P;
+  return each * pulse < 0.95 * batched;
 }
 
 struct TilePlan {
@@ -1173,21 +1211,17 @@ static int setup_tiles(mpci_prop *pr, bool *ok) {
 
 // The forms of one pulse on more than one block: fused stages from the row
 // store (small), and the persistent launches (rows, tiles).  mode -1:
-// automatic; 0: none of them; 1: the row store wherever it applies.
+// automatic; 0: none of them; 1: the row store wherever it applies.  A batch
+// has the persistent row form, where it pays, unless mode is 0.
 static int apply_small_path(mpci_prop *pr, int mode) {
   mpci_system *sys = pr->sys;
   bool on = false, rows = false, tiles = false;
   if (pr->P == 1 && sys->nb > 1) {
     on = mode == 1 || (mode < 0 && 8 * sys->S <= kSmallPathBytes);
-    // the row form by default only where a wave has one quad: with more rows
-    // than that the tile form is faster (12 x 500 96 against 120 us per
-    // attempt, 30 x 250 89 against 200 us)
-    int n16 = 0;
-    for (int L = 0; L < sys->nb; ++L) n16 += (sys->s[L] + 15) / 16;
-    rows = mode == 1 ||
-           (mode < 0 && 8 * sys->S <= kRowsBytes && n16 <= sys->ncu);
+    rows = mode == 1 || (mode < 0 && row_groups(sys) <= sys->ncu);
     tiles = mode < 0 && !rows;
   }
+  if (pr->P > 1 && sys->nb > 1 && mode != 0) rows = rows_pay(pr);
   if (on || rows) {
     TRY(ensure_rows(sys));
     pr->nblk_small = sys->hrow.quad0[sys->nb];
@@ -1195,10 +1229,18 @@ static int apply_small_path(mpci_prop *pr, int mode) {
   if (on && !pr->Xs2.p) TRY(pr->Xs2.alloc(pr->NP));
   if (rows && !pr->rwg.p) {
     std::vector<RowWg> wg;
-    rows = plan_rows(pr, wg, &pr->rows_lds, &pr->rows_kq);
+    rows = plan_rows(pr, 1, wg, &pr->rows_lds, &pr->rows_kq);
+    pr->rows_grp = pr->rows_slots = 1;
+    if (rows && pr->P > 1) {
+      pr->rows_grp = std::min(pr->P, sys->ncu / (int)wg.size());
+      pr->rows_slots = std::min(
+          (pr->P + pr->rows_grp - 1) / pr->rows_grp, kRwSlots);
+      rows = plan_rows(pr, pr->rows_slots, wg, &pr->rows_lds, &pr->rows_kq);
+    }
     if (rows) {
-      TRY(pr->xb.alloc(4 * (size_t)sys->N));
-      TRY(pr->rb.alloc(3 * (size_t)sys->hrow.quad0[sys->nb]));
+      const size_t ns = (size_t)pr->rows_slots;
+      TRY(pr->xb.alloc((size_t)pr->rows_grp * ns * 4 * sys->N));
+      TRY(pr->rb.alloc((size_t)pr->rows_grp * ns * 3 * sys->hrow.quad0[sys->nb]));
       DevBuf<RowWg> d;
       TRY(d.alloc(wg.size()));
       TRY(h2d(pr, d.p, wg.data(), sizeof(RowWg) * wg.size()));
@@ -1239,16 +1281,16 @@ extern "C" int mpci_prop_create(mpci_system *sys, int P, mpci_prop **out) {
     quads += (sys->s[L] + kRwQuad - 1) / kRwQuad;
   TRY(pr->red.alloc(
       (size_t)std::max({pr->nblk, pr->nblk_stage, quads}) * P * 2));
-  // behind the pulses' records: the one saved by k_rows_begin, and one whose
-  // status is k_rows_run's abort flag
-  TRY(pr->ctl.alloc(P + 2));
+  // behind the pulses' records: those saved by k_rows_begin, and one whose
+  // status is the persistent launches' abort flag
+  TRY(pr->ctl.alloc(2 * P + 1));
   TRY(pr->pulses.alloc(P));
   TRY(pr->log.alloc((size_t)pr->logcap * P));
   HIPCHK(hipMemsetAsync(pr->X.p, 0, sizeof(double2) * pr->NP, pr->stream));
   HIPCHK(hipMemsetAsync(pr->part.p, 0, sizeof(double2) * pr->part.n,
                         pr->stream));
   HIPCHK(hipStreamSynchronize(pr->stream));
-  std::vector<Ctl> c(P + 2);
+  std::vector<Ctl> c(2 * P + 1);
   std::memset(c.data(), 0, sizeof(Ctl) * c.size());
   for (auto &x : c) x.done = 1;
   TRY(h2d(pr.get(), pr->ctl.p, c.data(), sizeof(Ctl) * c.size()));
@@ -1552,16 +1594,16 @@ static int run_attempts_instrumented(mpci_prop *pr, int n) {
 // the launch.
 static bool run_attempts_persistent(mpci_prop *pr) {
   mpci_system *sys = pr->sys;
-  const int nxb = (pr->rows ? 4 : 3) * sys->N;
+  const int nxb = pr->rows ? (int)pr->xb.n : 3 * sys->N;
   const int npb = pr->rows ? 0 : 3 * pr->tiles_part;
-  const int nrb = 3 * (pr->rows ? sys->hrow.quad0[sys->nb] : pr->tiles_wg);
-  int *flag = &pr->ctl.p[pr->P + 1].status;
-  int *arrived = &pr->ctl.p[pr->P + 1].nlog;
-  const unsigned nb = (unsigned)((std::max(nxb, npb) + 255) / 256);
+  const int nrb = pr->rows ? (int)pr->rb.n : 3 * pr->tiles_wg;
+  int *flag = &pr->ctl.p[2 * pr->P].status;
+  int *arrived = &pr->ctl.p[2 * pr->P].nlog;
+  const int NP = (int)pr->NP;
+  const unsigned nb = (unsigned)((std::max({nxb, npb, NP}) + 255) / 256);
   hipLaunchKernelGGL(k_rows_begin, dim3(nb), dim3(256), 0, pr->stream,
                      pr->xb.p, nxb, pr->pb.p, npb, pr->rb.p, nrb, pr->X.p,
-                     sys->N, pr->Y.p, pr->ctl.p, pr->ctl.p + pr->P, flag,
-                     arrived);
+                     NP, pr->Y.p, pr->ctl.p, pr->P, flag, arrived);
   if (hipGetLastError() != hipSuccess) return false;
   auto common = [&](auto &a) {
     a.X = pr->X.p;
@@ -1606,16 +1648,22 @@ static bool run_attempts_persistent(mpci_prop *pr) {
     RowRun a{};
     common(a);
     a.wg = pr->rwg.p;
+    a.P = pr->P;
+    a.ngrp = pr->rows_grp;
+    a.nwg = pr->rows_wg;
+    a.nslot = pr->rows_slots;
     a.nquad = sys->hrow.quad0[sys->nb];
     const RowDesc *rd = sys->drow.p;
     const double *dq = sys->Dq.p;
     void *args[] = {&a, &d, &rd, &dq};
-    const void *fn = pr->rows_kq == 1
-                         ? reinterpret_cast<const void *>(k_rows_run<1>)
-                     : pr->rows_kq == 2
-                         ? reinterpret_cast<const void *>(k_rows_run<2>)
-                         : reinterpret_cast<const void *>(k_rows_run<4>);
-    e = launch(fn, pr->rows_wg, kRwThreads, args, &a.start_ms, pr->rows_lds);
+    const void *fn =
+        pr->P > 1 ? reinterpret_cast<const void *>(k_rows_run<1, true>)
+        : pr->rows_kq == 1
+            ? reinterpret_cast<const void *>(k_rows_run<1, false>)
+        : pr->rows_kq == 2
+            ? reinterpret_cast<const void *>(k_rows_run<2, false>)
+            : reinterpret_cast<const void *>(k_rows_run<4, false>);
+    e = launch(fn, pr->rows_wg * pr->rows_grp, kRwThreads, args, &a.start_ms, pr->rows_lds);
   } else {
     TileRun a{};
     common(a);
@@ -1658,18 +1706,18 @@ static int run_attempts(mpci_prop *pr, int n) {
 static int read_ctl(mpci_prop *pr, std::vector<Ctl> &c) {
   const int P = pr->P;
   const bool persistent = pr->rows || pr->tiles;
-  c.resize(persistent ? P + 2 : P);
+  c.resize(persistent ? 2 * P + 1 : P);
   HIPCHK(hipStreamSynchronize(pr->stream));
   TRY(d2h(pr, c.data(), pr->ctl.p, sizeof(Ctl) * c.size()));
-  if (persistent && c[P + 1].status) {
+  if (persistent && c[2 * P].status) {
     // the persistent launch gave up waiting (the device was held by others
     // for longer than its time limit): back to where it began, and from now
     // on one launch per stage
     pr->rows = pr->tiles = false;
     HIPCHK(hipMemcpyAsync(pr->X.p, pr->Y.p, sizeof(double2) * pr->NP,
                           hipMemcpyDeviceToDevice, pr->stream));
-    c[0] = c[P];
-    TRY(h2d(pr, pr->ctl.p, c.data(), sizeof(Ctl)));
+    std::copy(c.begin() + P, c.begin() + 2 * P, c.begin());
+    TRY(h2d(pr, pr->ctl.p, c.data(), sizeof(Ctl) * P));
   }
   c.resize(P);
   return MPCI_OK;
@@ -2123,6 +2171,32 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
     if (pr->sys->device != props[0]->sys->device)
       return fail(MPCI_ERR_NOTSUP, "mpci_multi_adaptive_grouped: members on "
                                    "different devices");
+  }
+  // members whose batch runs in one persistent launch run it, beside each
+  // other, and the group is made of the others
+  std::vector<int> alone, rest;
+  for (int i = 0; i < n; ++i)
+    (props[i]->rows && props[i]->use_graph ? alone : rest).push_back(i);
+  if (!alone.empty()) {
+    auto part = [&](const std::vector<int> &idx, bool grouped) {
+      std::vector<mpci_prop *> p;
+      std::vector<const double *> a, b, h;
+      std::vector<mpci_stats *> st;
+      for (int i : idx) {
+        p.push_back(props[i]);
+        a.push_back(t0[i]);
+        b.push_back(t1[i]);
+        h.push_back(h0[i]);
+        st.push_back(stats ? stats[i] : nullptr);
+      }
+      return (grouped ? mpci_multi_adaptive_grouped : mpci_multi_adaptive)(
+          (int)idx.size(), p.data(), a.data(), b.data(), h.data(), atol, rtol,
+          max_attempts, st.data());
+    };
+    const int rc = part(alone, false);
+    if ((rc != MPCI_OK && rc != MPCI_ERR_LIMIT) || rest.empty()) return rc;
+    const int rc2 = part(rest, true);
+    return rc2 != MPCI_OK ? rc2 : rc;
   }
   // the group's tile: that of the member with the most coupling work when
   // it is a direct-to-LDS tile, else 4 x 2 waves
@@ -2848,6 +2922,7 @@ extern "C" int mpci_prop_set_gemm_candidate(mpci_prop *pr, int index) {
   // are reallocated here
   HIPCHK(hipStreamSynchronize(pr->stream));
   drop_graph(pr);
+  if (pr->P > 1) pr->rows = false;  // the pinned tile is what runs
   return tune_gemm(pr, &kGemmCands[index]);
 }
 

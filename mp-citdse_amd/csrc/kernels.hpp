@@ -49,15 +49,16 @@ struct AdjArgs {
   int pad;
 };
 
-// The persistent row kernel: `attempts` attempts of one pulse in one
-// cooperative launch.
+// The persistent row kernel: up to `attempts` attempts of every pulse in one
+// cooperative launch: ngrp groups of nwg workgroups, nslot pulses at a time
+// in each.
 struct RowRun {
   const RowWg *wg;
-  double2 *X;            // committed state (N)
+  double2 *X;            // committed states (N x P)
   const double *E;
-  double2 *xb;           // stage inputs in exchange: 4 x N
-  double2 *rb;           // per-quad (error max, |y|^2) in exchange: 3 x nquad
-  Ctl *ctl;              // the pulse's control record
+  double2 *xb;           // stage inputs in exchange: 4 x N a slot
+  double2 *rb;           // per-quad (error max, |y|^2): 3 x nquad a slot
+  Ctl *ctl;              // the pulses' control records
   int *abort_flag;       // set when a wait ran into its time limit
   const double *hs;
   const double *Ftab;
@@ -65,6 +66,7 @@ struct RowRun {
   const double *env;
   LogEnt *log;
   int logcap, track, N, nquad, attempts;
+  int P, ngrp, nwg, nslot;
   int limit_ms;          // time limit of one wait
   int start_ms;          // > 0: not cooperative, wait for all workgroups
   int *arrived;          // workgroups that run
@@ -173,11 +175,11 @@ __global__ void k_relayout_rows(const double *Dg, const SysDesc *d,
                                 long long nelem, double *Dq);
 // Unsets the exchange buffers and saves the state and the control record.
 __global__ void k_rows_begin(double2 *xb, int nxb, double2 *pb, int npb,
-                             double2 *rb, int nrb, const double2 *X, int N,
-                             double2 *Xsave, const Ctl *ctl, Ctl *ctl_save,
+                             double2 *rb, int nrb, const double2 *X, int NP,
+                             double2 *Xsave, Ctl *ctl, int P,
                              int *abort_flag, int *arrived);
 __global__ void k_tiles_run(TileRun a, const SysDesc *d, const TileDesc *td);
-template <int kQ>
+template <int kQ, bool kMany>
 __global__ void k_rows_run(RowRun a, const SysDesc *d, const RowDesc *rd,
                            const double *Dq);
 __global__ void k_finalize(Ctl *ctl, const double *red, int nblk, int P,

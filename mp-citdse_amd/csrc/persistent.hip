@@ -1,8 +1,8 @@
-// Persistent kernels of the MI355X tdse engine (gfx950): one pulse, whole
-// attempts in one cooperative launch.
+// Persistent kernels of the MI355X tdse engine (gfx950): whole attempts in
+// one cooperative launch.
 //
 //   k_rows_begin     unsets the exchange buffers, saves the state.
-//   k_rows_run       small systems: workgroups own rows.
+//   k_rows_run       small systems, also a few pulses: workgroups own rows.
 //   k_tiles_run      larger systems: workgroups own tiles and rows.
 //
 // Compiled without the machine-code loop-invariant motion, which would hold
@@ -34,6 +34,18 @@ namespace mpci {
 // polling and storing (47 us: a poll waits for the acknowledgement of the
 // stores before it), 16 waves (register spills).
 //
+// A batch (kMany): the device holds ngrp groups of workgroups, each with all
+// rows, and a group runs some of the pulses, up to kRwSlots at a time: a
+// stage of each in turn, so that a pulse's exchange runs behind the others'
+// sums.  Pulses stay independent: each has its exchange buffers, its step
+// control (a polling wave each) and its attempts.  Per attempt of all pulses,
+// against the batched launches (13 GEMM and 13 stage launches of 5 to 14 us
+// each whatever they hold): 300 x 6, P = 5 164 -> 62 us; 198 x 4, P = 16 145
+// -> 78 us; 60 x 8, P = 5 128 -> 28 us.  A further pulse of a group costs
+// about 20 us, 1.5 us a stage: the computing waves' tableau sums, coupling
+// sums and stage algebra.  Fewer, larger groups (32 to 64 rows a workgroup)
+// were slower from P = 2 on (300 x 6, P = 5: 98 to 141 us).
+//
 // Exchange.  xb holds four copies of the state; stage g (counted over the
 // launch) uses copy g % 4.  An unset component holds kUnset, a signalling
 // NaN that no arithmetic produces (a raw copy of it is quieted).  The owner
@@ -45,9 +57,9 @@ namespace mpci {
 // reading stage g - 1), and unsets its own rows there; those stores have
 // landed before it publishes stage g + 2, ahead of any poll of that copy for
 // stage g + 3.  The step control needs every row's error and norm: quads
-// exchange them the same way (rb, three copies by attempt), every workgroup
-// reduces them in k_finalize's order and runs the controller on its own,
-// with the same bits everywhere.
+// exchange them the same way (rb, three copies by attempt), one wave of every
+// workgroup reduces them in k_finalize's order and runs the controller, with
+// the same bits everywhere.
 //
 // Every wait is bounded: past limit_ms a workgroup sets abort_flag and
 // leaves, the others see the flag; the host then restores the state saved
@@ -99,10 +111,10 @@ __device__ __forceinline__ double2 publishable(double2 v) {
   return make_double2(publishable1(v.x), publishable1(v.y));
 }
 
-// Unsets the exchange buffers and saves the state and the control record.
+// Unsets the exchange buffers and saves the states and control records.
 __global__ __launch_bounds__(256) void k_rows_begin(
     double2 *xb, int nxb, double2 *pb, int npb, double2 *rb, int nrb,
-    const double2 *X, int N, double2 *Xsave, const Ctl *ctl, Ctl *ctl_save,
+    const double2 *X, int NP, double2 *Xsave, Ctl *ctl, int P,
     int *abort_flag, int *arrived) {
   const double u = __longlong_as_double((long long)kUnset);
   const double2 unset = make_double2(u, u);
@@ -110,9 +122,9 @@ __global__ __launch_bounds__(256) void k_rows_begin(
   if (i < nxb) xb[i] = unset;
   if (i < npb) pb[i] = unset;
   if (i < nrb) rb[i] = unset;
-  if (i < N) Xsave[i] = X[i];
+  if (i < NP) Xsave[i] = X[i];
+  if (i < P) ctl[P + i] = ctl[i];
   if (i == 0) {
-    *ctl_save = *ctl;
     *abort_flag = 0;
     *arrived = 0;
   }
@@ -141,14 +153,19 @@ __device__ __forceinline__ bool all_started(int *arrived, int *abort_flag,
   return true;
 }
 
-template <int kQ>
+template <int kQ, bool kMany>
 __global__ __launch_bounds__(kRwThreads) void k_rows_run(
     RowRun a, const SysDesc *__restrict__ dp, const RowDesc *__restrict__ rp,
     const double *__restrict__ Dq) {
   // chunks of a quad kept in registers: one quad a wave leaves room for them
   constexpr int kReg = kQ == 1 ? kRwReg : 0;
+  static_assert(!kMany || kQ == 1, "several slots: a quad a wave");
+  constexpr int kSlots = kMany ? kRwSlots : 1;
   const SysDesc &d = *dp;
-  const RowWg g = a.wg[blockIdx.x];
+  // group grp of nwg workgroups runs pulses grp, grp + ngrp, .., nslot of
+  // them at a time, a stage of each in turn
+  const int grp = blockIdx.x / a.nwg, wgi = blockIdx.x - grp * a.nwg;
+  const RowWg g = a.wg[wgi];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int L = g.L, gauge = d.gauge;
@@ -160,29 +177,33 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
   const int nq = (g.nrows + kRwQuad - 1) / kRwQuad, nr4 = nq * kRwQuad;
 
   // LDS: two copies of the neighbours' stage input (zero padded to whole
-  // groups of chunks), the 13 stage derivatives of the own rows, the
-  // resident chunks of the row store ([quad][chunk])
+  // groups of chunks); per slot the 13 stage derivatives, the state and the
+  // stage input of the own rows; the resident chunks of the row store
+  // ([quad][chunk])
   extern __shared__ __align__(16) unsigned char smem[];
   double2 *xs0 = reinterpret_cast<double2 *>(smem);
-  double2 *Ks = xs0 + 2 * nchp * 64;
-  double2 *Dl = Ks + kStages * nr4;
-  __shared__ Ctl cl;
-  __shared__ double se[256], sn[256];
+  double2 *own_rows = xs0 + 2 * nchp * 64;
+  const int slot_n = (kStages + 2) * nr4;
+  const unsigned nslot = kMany ? (unsigned)a.nslot : 1u;
+  double2 *Dl = own_rows + nslot * slot_n;
+  __shared__ Ctl cl[kSlots];
+  __shared__ double2 en[kSlots][kRwMaxRows / kRwQuad];
   __shared__ int stop;
   // row s < 12: a_{s+1,j}; rows 12, 13: b, b - bhat
   __shared__ double coef[kStages + 1][kStages];
 
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)a.xb, (short)0, (int)(kXbCopies * (unsigned)a.N * 16u), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)a.rb, (short)0, (int)(3u * (unsigned)a.nquad * 16u), 0x00020000);
-  constexpr unsigned kOut = 0x80000000u;  // beyond any buffer range
   const unsigned N = (unsigned)a.N, NQ = (unsigned)a.nquad;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(a.xb + (long long)grp * nslot * kXbCopies * N), (short)0,
+      (int)(nslot * kXbCopies * N * 16u), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(a.rb + (long long)grp * nslot * 3 * NQ), (short)0,
+      (int)(nslot * 3u * NQ * 16u), 0x00020000);
+  constexpr unsigned kOut = 0x80000000u;  // beyond any buffer range
   const double u_ = __longlong_as_double((long long)kUnset);
   const double2 unset = make_double2(u_, u_);
 
   if (t == 0) {
-    cl = a.ctl[0];
     stop = 0;
     if (a.limit_ms < 0) {  // no wait at all
       stop = 1;
@@ -207,7 +228,6 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
     if (ch < nch) Dl[i] = D2[((long long)q * nch + ch) * 128 + (i & 127)];
   }
   __syncthreads();
-
   if (stop) return;  // uniform
 
   // true once the wait has to be given up (looked at now and then)
@@ -224,8 +244,29 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
                                      __HIP_MEMORY_SCOPE_AGENT) != 0;
   };
 
-  unsigned buf = 0, rbuf = 0;  // exchange copies of the coming stage, reduction
-  int par = 0;                 // LDS copy of the coming stage's input
+  // exchange copies, two bits a slot: of the coming attempt's stage 0 (13
+  // stages on, the next attempt's is the next one) and of its reduction
+  static_assert(kXbCopies == 4 && kStages % 4 == 1, "");
+  unsigned xcopy = 0, rcopy = 0;
+  auto bits2 = [](unsigned v, int b) { return (v >> (2 * b)) & 3u; };
+  // the slots whose pulse is not finished, and their copies moved on
+  auto live_slots = [&](int ns) {
+    if (!kMany) return cl[0].done ? 0u : 1u;
+    unsigned m = 0;
+    for (int b = 0; b < ns; ++b)
+      if (!cl[b].done) m |= 1u << b;
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)m);
+  };
+  auto advance = [&](unsigned act) {
+    for (unsigned m = act; m; m &= m - 1) {
+      const int b = kMany ? __builtin_ctz(m) : 0;
+      const unsigned x1 = (bits2(xcopy, b) + 1) & 3u;
+      const unsigned r1 = bits2(rcopy, b) == 2 ? 0u : bits2(rcopy, b) + 1;
+      xcopy = (xcopy & ~(3u << (2 * b))) | (x1 << (2 * b));
+      rcopy = (rcopy & ~(3u << (2 * b))) | (r1 << (2 * b));
+    }
+  };
+  int par = 0;  // LDS copy of the coming stage's input
   if (w >= kRwCompute) {
     // ================= the polling waves =================
     const int tp = t - 64 * kRwCompute;
@@ -268,84 +309,102 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
       }
     };
     const int nslots = (nx + kPoll - 1) / kPoll;
-    for (int n = 0; n < a.attempts && !cl.done; ++n) {
-      for (int s = 0; s < kStages; ++s) {
-        double2 *xs = xs0 + par * nchp * 64;
-        if (nslots <= 1) {
-          poll(buf, xs, 0, Int<1>());
-        } else if (nslots <= 2) {
-          poll(buf, xs, 0, Int<2>());
-        } else if (nslots <= 4) {
-          poll(buf, xs, 0, Int<4>());
-        } else {
-          // one row first: while it is not there, the others are not asked for
-          poll(buf, xs, 0, Int<1>());
-          for (int u = 1; u < nslots; u += 8) poll(buf, xs, u, Int<8>());
-        }
-        __syncthreads();
-        if (stop) return;  // uniform over the workgroup
-        buf = (buf + 1) % kXbCopies;
-        par ^= 1;
-      }
-      // ---- step control: every quad's (error max, |y|^2)
-      double em = 0.0, ns = 0.0;
-      for (int i0 = tp; i0 < (int)NQ; i0 += 4 * 256) {
-        double2 p[4];
-        unsigned miss = 0;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (i0 + u * 256 < (int)NQ) miss |= 1u << u;
-        for (int tries = 1; miss; ++tries) {
-          double2 q[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            q[u] = dev_load(
-                rr, (miss >> u) & 1u ? (rbuf * NQ + i0 + u * 256) * 16u : kOut);
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (((miss >> u) & 1u) && !is_unset(q[u].x) && !is_unset(q[u].y)) {
-              p[u] = q[u];
-              miss &= ~(1u << u);
+    for (int base = 0; grp + base * a.ngrp < a.P; base += nslot) {
+      const int ns =
+          kMany ? min((int)nslot, (a.P - 1 - grp) / a.ngrp - base + 1) : 1;
+      __syncthreads();  // the last pulses' records have been read
+      __syncthreads();  // these are there
+      for (int n = 0; n < a.attempts; ++n) {
+        const unsigned act = live_slots(ns);
+        if (act == 0) break;
+        for (int s = 0; s < kStages; ++s) {
+          for (unsigned m = act; m; m &= m - 1) {
+            const int b = kMany ? __builtin_ctz(m) : 0;
+            const unsigned buf = b * kXbCopies + ((bits2(xcopy, b) + s) & 3u);
+            double2 *xs = xs0 + par * nchp * 64;
+            if (nslots <= 1) {
+              poll(buf, xs, 0, Int<1>());
+            } else if (nslots <= 2) {
+              poll(buf, xs, 0, Int<2>());
+            } else if (nslots <= 4) {
+              poll(buf, xs, 0, Int<4>());
+            } else {
+              // one row first: while it is not there, the others are not
+              // asked for
+              poll(buf, xs, 0, Int<1>());
+              for (int u = 1; u < nslots; u += 8) poll(buf, xs, u, Int<8>());
             }
-          asm volatile("" ::: "memory");
-          if (miss && give_up(tries)) {
-            stop = 1;
-            break;
+            __syncthreads();
+            if (stop) return;  // uniform over the workgroup
+            par ^= 1;
           }
         }
-        if (miss) break;
+        // ---- step control: every quad's (error max, |y|^2), a wave a slot.
+        // k_finalize's order: 256 strided sums (four a lane), then halves of
+        // 128, 64 and, across the wave, 32 .. 1
+        for (unsigned m = act; m; m &= m - 1) {
+          const int b = kMany ? __builtin_ctz(m) : 0;
+          if ((b & 3) != w - kRwCompute) continue;
+          const int p = grp + (base + b) * a.ngrp;
+          double em4[4] = {}, ns4[4] = {};
+          bool lost = false;
+          for (int i0 = lane; i0 < (int)NQ && !lost; i0 += 256) {
+            double2 v[4];
+            unsigned miss = 0;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (i0 + u * 256 < (int)NQ) {
-            em = p[u].x > em ? p[u].x : em;
-            ns += p[u].y;
+            for (int u = 0; u < 4; ++u)
+              if (i0 + u * 64 < (int)NQ) miss |= 1u << u;
+            const unsigned r0 = (b * 3 + bits2(rcopy, b)) * NQ + i0;
+            for (int tries = 1; miss; ++tries) {
+              double2 q[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u)
+                q[u] = dev_load(rr, (miss >> u) & 1u ? (r0 + u * 64) * 16u
+                                                     : kOut);
+#pragma unroll
+              for (int u = 0; u < 4; ++u)
+                if (((miss >> u) & 1u) && !is_unset(q[u].x) &&
+                    !is_unset(q[u].y)) {
+                  v[u] = q[u];
+                  miss &= ~(1u << u);
+                }
+              asm volatile("" ::: "memory");
+              if (miss && give_up(tries)) {
+                stop = 1;
+                lost = true;
+                break;
+              }
+            }
+            if (lost) break;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (i0 + u * 64 < (int)NQ) {
+                em4[u] = v[u].x > em4[u] ? v[u].x : em4[u];
+                ns4[u] += v[u].y;
+              }
           }
-      }
-      se[tp] = em;
-      sn[tp] = ns;
-      __syncthreads();
-      if (stop) return;
-      if (w == kRwCompute) {
-        // k_finalize's tree: halves of 128, 64, then 32 .. 1 across the wave
-        auto mx = [](double p, double q) { return p > q ? p : q; };
-        em = mx(mx(se[lane], se[lane + 128]), mx(se[lane + 64], se[lane + 192]));
-        ns = (sn[lane] + sn[lane + 128]) + (sn[lane + 64] + sn[lane + 192]);
+          auto mx = [](double p, double q) { return p > q ? p : q; };
+          double em = mx(mx(em4[0], em4[2]), mx(em4[1], em4[3]));
+          double n2 = (ns4[0] + ns4[2]) + (ns4[1] + ns4[3]);
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          em = mx(em, __shfl_xor(em, o));
-          ns += __shfl_xor(ns, o);
+          for (int o = 32; o > 0; o >>= 1) {
+            em = mx(em, __shfl_xor(em, o));
+            n2 += __shfl_xor(n2, o);
+          }
+          if (lane == 0) cl[b] = control_step(cl[b], em, n2, p, a.hs);
+          // the record is in LDS before the wave's other lanes read it
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_wave_barrier();
+          if (lane < kStages && !cl[b].done)
+            cl[b].Fs[lane] =
+                stage_field(cl[b], lane, p, a.Ftab, a.pulses, a.env);
         }
-        if (lane == 0) cl = control_step(cl, em, ns, 0, a.hs);
-        // the record is in LDS before the wave's other lanes read it
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_wave_barrier();
-        if (lane < kStages && !cl.done)
-          cl.Fs[lane] = stage_field(cl, lane, 0, a.Ftab, a.pulses, a.env);
+        advance(act);
+        __syncthreads();
+        if (stop) return;
       }
-      rbuf = rbuf == 2 ? 0 : rbuf + 1;
-      __syncthreads();
+      if (wgi == 0 && tp < ns) a.ctl[grp + (base + tp) * a.ngrp] = cl[tp];
     }
-    if (blockIdx.x == 0 && tp == 0) a.ctl[0] = cl;
     return;
   }
 
@@ -355,19 +414,14 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
   bool own[kQ];
   int lr[kQ];
   unsigned row[kQ];
-  double2 x[kQ], v[kQ], xin[kQ];
   double e[kQ];
 #pragma unroll
   for (int m = 0; m < kQ; ++m) {
     lr[m] = (w + m * kRwCompute) * kRwQuad + (lane >> 4);
     own[m] = (lane & 15) == 0 && lr[m] < g.nrows;
     row[m] = (unsigned)(d.off[L] + g.row0 + lr[m]);
-    x[m] = make_double2(0.0, 0.0);
     e[m] = 0.0;
-    if (own[m]) {
-      x[m] = a.X[row[m]];
-      e[m] = a.E[row[m]];
-    }
+    if (own[m]) e[m] = a.E[row[m]];
   }
   // the first quad's first chunks (zeros beyond the last)
   double2 R[kReg + 1][2];
@@ -378,166 +432,228 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
       R[c][p] = c < nch && w < nq
                     ? D2[((long long)w * nch + c) * 128 + p * 64 + lane]
                     : make_double2(0.0, 0.0);
-  for (int n = 0; n < a.attempts && !cl.done; ++n) {
-    const double h = cl.hc;
-    const unsigned rnext = rbuf == 2 ? 0 : rbuf + 1;
-    double errv[kQ] = {}, nrm2[kQ] = {};
+  // state and stage input of the own rows: with several slots in LDS
+  double2 x[kQ], xin[kQ], v[kQ];
+  for (int base = 0; grp + base * a.ngrp < a.P; base += nslot) {
+    const int ns =
+        kMany ? min((int)nslot, (a.P - 1 - grp) / a.ngrp - base + 1) : 1;
+    __syncthreads();
+    if (t < ns) cl[t] = a.ctl[grp + (base + t) * a.ngrp];
 #pragma unroll
-    for (int m = 0; m < kQ; ++m) {
-      xin[m] = x[m];
+    for (int m = 0; m < kQ; ++m)
       if (own[m])
-        dev_store(rx, (buf * N + row[m]) * 16u, publishable(x[m]));
-      // the reduction's copy last read two attempts ago, whose results every
-      // workgroup has used since
-      if (lane == 0 && own[m])
-        dev_store(rr, (rnext * NQ + g.quad0 + w + m * kRwCompute) * 16u, unset);
-    }
-    for (int s = 0; s < kStages; ++s) {
-      const unsigned b1 = (buf + 1) % kXbCopies, b3 = (buf + 3) % kXbCopies;
-      const bool last = s == kStages - 1;
-      const double2 *xs = xs0 + par * nchp * 64 + lane;
-      // while the stage input arrives: the tableau sums of the next one but
-      // for k_s (stage_row's terms in stage_row's order)
-      const double F = cl.Fs[s];
-      const double co = h * coef[s][s];
-      double2 err[kQ] = {};
+        for (int b = 0; b < ns; ++b) {
+          x[m] = a.X[(long long)row[m] * a.P + grp + (base + b) * a.ngrp];
+          if (kMany) own_rows[b * slot_n + kStages * nr4 + lr[m]] = x[m];
+        }
+    __syncthreads();
+    for (int n = 0; n < a.attempts; ++n) {
+      const unsigned act = live_slots(ns);
+      if (act == 0) break;
+      for (unsigned mb = act; mb; mb &= mb - 1) {
+        const int b = kMany ? __builtin_ctz(mb) : 0;
+        double2 *xv = own_rows + b * slot_n + kStages * nr4;
+        const unsigned buf = b * kXbCopies + bits2(xcopy, b);
+        const unsigned rc = bits2(rcopy, b);
+        const unsigned rnext = b * 3 + (rc == 2 ? 0u : rc + 1);
 #pragma unroll
-      for (int m = 0; m < kQ; ++m) {
-        if (!own[m]) continue;
-        v[m] = x[m];
-        if (!last) {
-#pragma unroll 4
-          for (int j = 0; j < s; ++j) {
-            const double cj = h * coef[s][j];
-            const double2 kj = Ks[j * nr4 + lr[m]];
-            v[m].x = fma(cj, kj.x, v[m].x);
-            v[m].y = fma(cj, kj.y, v[m].y);
+        for (int m = 0; m < kQ; ++m) {
+          if (own[m]) {
+            if (kMany) x[m] = xv[lr[m]];
+            if (kMany) xv[nr4 + lr[m]] = x[m];
+            xin[m] = x[m];
+            dev_store(rx, (buf * N + row[m]) * 16u, publishable(x[m]));
           }
-        } else {
+          // the reduction's copy last read two attempts ago, whose results
+          // every workgroup has used since
+          if (lane == 0 && own[m])
+            dev_store(rr, (rnext * NQ + g.quad0 + w + m * kRwCompute) * 16u,
+                      unset);
+        }
+      }
+      for (int s = 0; s < kStages; ++s) {
+        const bool last = s == kStages - 1;
+        for (unsigned mb = act; mb; mb &= mb - 1) {
+          const int b = kMany ? __builtin_ctz(mb) : 0;
+          const unsigned c0 = bits2(xcopy, b) + s, bx = b * kXbCopies;
+          const unsigned b1 = bx + ((c0 + 1) & 3u), b3 = bx + ((c0 + 3) & 3u);
+          double2 *Ks = own_rows + b * slot_n;
+          double2 *xv = Ks + kStages * nr4, *xiv = xv + nr4;
+          const double2 *xs = xs0 + par * nchp * 64 + lane;
+          // while the stage input arrives: the tableau sums of the next one
+          // but for k_s (stage_row's terms in stage_row's order)
+          const double F = cl[b].Fs[s], h = cl[b].hc;
+          const double co = h * coef[s][s];
+          double2 err[kQ] = {};
+#pragma unroll
+          for (int m = 0; m < kQ; ++m) {
+            if (!own[m]) continue;
+            if (kMany) x[m] = xv[lr[m]];
+            if (kMany) xin[m] = xiv[lr[m]];
+            v[m] = x[m];
+            if (!last) {
 #pragma unroll 4
-          for (int j = 0; j < kStages - 1; ++j) {
-            const double cb = h * coef[kStages - 1][j], cd = h * coef[kStages][j];
-            const double2 kj = Ks[j * nr4 + lr[m]];
-            v[m].x = fma(cb, kj.x, v[m].x);
-            v[m].y = fma(cb, kj.y, v[m].y);
-            err[m].x = fma(cd, kj.x, err[m].x);
-            err[m].y = fma(cd, kj.y, err[m].y);
+              for (int j = 0; j < s; ++j) {
+                const double cj = h * coef[s][j];
+                const double2 kj = Ks[j * nr4 + lr[m]];
+                v[m].x = fma(cj, kj.x, v[m].x);
+                v[m].y = fma(cj, kj.y, v[m].y);
+              }
+            } else {
+#pragma unroll 4
+              for (int j = 0; j < kStages - 1; ++j) {
+                const double cb = h * coef[kStages - 1][j],
+                             cd = h * coef[kStages][j];
+                const double2 kj = Ks[j * nr4 + lr[m]];
+                v[m].x = fma(cb, kj.x, v[m].x);
+                v[m].y = fma(cb, kj.y, v[m].y);
+                err[m].x = fma(cd, kj.x, err[m].x);
+                err[m].y = fma(cd, kj.y, err[m].y);
+              }
+            }
           }
+          __syncthreads();
+          if (stop) return;  // uniform over the workgroup
+#pragma unroll
+          for (int m = 0; m < kQ; ++m) {
+            const int q = w + m * kRwCompute;
+            if (q >= nq) continue;  // uniform over the wave
+            double2 acc[4] = {};
+            // every x is read a group of four chunks ahead (past the last
+            // group that stays inside the LDS buffer and is not used)
+            double2 xn[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) xn[u] = xs[u * 64];
+#pragma unroll
+            for (int c0 = 0; c0 < kReg; c0 += 4) {
+              if (c0 < nch) {
+                double2 xc[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                  xc[u] = xn[u];
+                  xn[u] = xs[(c0 + 4 + u) * 64];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                  quad_fma(acc, R[c0 + u][0], R[c0 + u][1], xc[u]);
+              }
+            }
+            int c = kReg;
+            const int cl1 = min(c + g.nlds, nch);
+            const double2 *Dr = Dl + ((long long)q * g.nlds - c) * 128 + lane;
+#pragma unroll 4
+            for (; c < cl1; ++c)
+              quad_fma(acc, Dr[c * 128], Dr[c * 128 + 64], xs[c * 64]);
+            if (c < nch) {
+              // the chunks past the LDS share
+              const double2 *Dg = D2 + (long long)q * nch * 128 + lane;
+#pragma unroll 4
+              for (; c < nch; ++c)
+                quad_fma(acc, Dg[c * 128], Dg[c * 128 + 64], xs[c * 64]);
+            }
+            const double2 cs = quad_reduce(acc, lane);
+            double errv = 0.0, nrm2 = 0.0;
+            if (own[m]) {
+              const double2 k =
+                  stage_deriv(gauge, e[m], xin[m], F, cs, make_double2(0.0, 0.0));
+              if (!last) {
+                v[m].x = fma(co, k.x, v[m].x);
+                v[m].y = fma(co, k.y, v[m].y);
+                // this slot's rows unset a stage ago have landed: two stores
+                // a quad and stage, so with other slots in between they are
+                // older than the last two
+                if (kMany && (act & (act - 1)))
+                  asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+                else
+                  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                dev_store(rx, (b1 * N + row[m]) * 16u, publishable(v[m]));
+                xin[m] = v[m];
+                if (kMany) xiv[lr[m]] = v[m];
+              } else {
+                const double cb = h * cB[kStages - 1], cd = h * cDB[kStages - 1];
+                v[m].x = fma(cb, k.x, v[m].x);
+                v[m].y = fma(cb, k.y, v[m].y);
+                err[m].x = fma(cd, k.x, err[m].x);
+                err[m].y = fma(cd, k.y, err[m].y);
+                const double2 k1 = Ks[lr[m]];
+                const Ctl &c = cl[b];
+                const double ex =
+                    fabs(err[m].x) / (c.atol + c.rtol * (fabs(x[m].x) + h * fabs(k1.x)));
+                const double ey =
+                    fabs(err[m].y) / (c.atol + c.rtol * (fabs(x[m].y) + h * fabs(k1.y)));
+                errv = ex > ey ? ex : ey;
+                nrm2 = abs2(v[m].x, v[m].y);
+                if (kMany) xiv[lr[m]] = v[m];
+              }
+              Ks[s * nr4 + lr[m]] = k;
+            }
+            if (last) {
+              const double2 q2 = quad_norms(errv, nrm2);
+              if (lane == 0) en[b][q] = q2;
+            }
+          }
+          // copy b3 (stage g - 1's) has been read by all its readers
+#pragma unroll
+          for (int m = 0; m < kQ; ++m)
+            if (own[m]) dev_store(rx, (b3 * N + row[m]) * 16u, unset);
+          par ^= 1;
+        }
+      }
+      // ---- step control
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      for (unsigned mb = act; mb; mb &= mb - 1) {
+        const int b = kMany ? __builtin_ctz(mb) : 0;
+        const unsigned rc = b * 3 + bits2(rcopy, b);
+#pragma unroll
+        for (int m = 0; m < kQ; ++m) {
+          const int q = w + m * kRwCompute;
+          if (lane == 0 && q < nq)
+            dev_store(rr, (rc * NQ + g.quad0 + q) * 16u, publishable(en[b][q]));
         }
       }
       __syncthreads();
-      if (stop) return;  // uniform over the workgroup
+      if (stop) return;
+      for (unsigned mb = act; mb; mb &= mb - 1) {
+        const int b = kMany ? __builtin_ctz(mb) : 0;
+        const Ctl &c = cl[b];
+        if (!c.accept) continue;
+        double2 *xv = own_rows + b * slot_n + kStages * nr4;
 #pragma unroll
-      for (int m = 0; m < kQ; ++m) {
-        const int q = w + m * kRwCompute;
-        if (q >= nq) continue;  // uniform over the wave
-        double2 acc[4] = {};
-        // every x is read a group of four chunks ahead (past the last group
-        // that stays inside the LDS buffer and is not used)
-        double2 xn[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) xn[u] = xs[u * 64];
-#pragma unroll
-        for (int c0 = 0; c0 < kReg; c0 += 4) {
-          if (c0 < nch) {
-            double2 xc[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              xc[u] = xn[u];
-              xn[u] = xs[(c0 + 4 + u) * 64];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-              quad_fma(acc, R[c0 + u][0], R[c0 + u][1], xc[u]);
+        for (int m = 0; m < kQ; ++m) {
+          if (!own[m]) continue;
+          if (kMany) v[m] = xv[nr4 + lr[m]];
+          x[m] = make_double2(v[m].x / c.nrm, v[m].y / c.nrm);
+          if (kMany) xv[lr[m]] = x[m];
+          if ((int)row[m] == a.track && c.nlog >= 1 && c.nlog <= a.logcap) {
+            LogEnt le;
+            le.t = c.t;
+            le.h = c.hacc;
+            le.pop = abs2(x[m].x, x[m].y);
+            a.log[(long long)(grp + (base + b) * a.ngrp) * a.logcap + c.nlog -
+                  1] = le;
           }
         }
-        int c = kReg;
-        const int cl1 = min(c + g.nlds, nch);
-        const double2 *Dr = Dl + ((long long)q * g.nlds - c) * 128 + lane;
-#pragma unroll 4
-        for (; c < cl1; ++c)
-          quad_fma(acc, Dr[c * 128], Dr[c * 128 + 64], xs[c * 64]);
-        if (c < nch) {
-          // the chunks past the LDS share
-          const double2 *Dg = D2 + (long long)q * nch * 128 + lane;
-#pragma unroll 4
-          for (; c < nch; ++c)
-            quad_fma(acc, Dg[c * 128], Dg[c * 128 + 64], xs[c * 64]);
-        }
-        const double2 cs = quad_reduce(acc, lane);
-        if (!own[m]) continue;
-        const double2 k =
-            stage_deriv(gauge, e[m], xin[m], F, cs, make_double2(0.0, 0.0));
-        if (!last) {
-          v[m].x = fma(co, k.x, v[m].x);
-          v[m].y = fma(co, k.y, v[m].y);
-          xin[m] = v[m];
-          // the rows unset a stage ago have landed
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          dev_store(rx, (b1 * N + row[m]) * 16u, publishable(v[m]));
-        } else {
-          const double cb = h * cB[kStages - 1], cd = h * cDB[kStages - 1];
-          v[m].x = fma(cb, k.x, v[m].x);
-          v[m].y = fma(cb, k.y, v[m].y);
-          err[m].x = fma(cd, k.x, err[m].x);
-          err[m].y = fma(cd, k.y, err[m].y);
-          const double2 k1 = Ks[lr[m]];
-          const double ex = fabs(err[m].x) / (cl.atol + cl.rtol * (fabs(x[m].x) +
-                                                         h * fabs(k1.x)));
-          const double ey = fabs(err[m].y) / (cl.atol + cl.rtol * (fabs(x[m].y) +
-                                                         h * fabs(k1.y)));
-          errv[m] = ex > ey ? ex : ey;
-          nrm2[m] = abs2(v[m].x, v[m].y);
-        }
-        Ks[s * nr4 + lr[m]] = k;
       }
-      // copy b3 (stage g - 1's) has been read by all its readers
-#pragma unroll
-      for (int m = 0; m < kQ; ++m)
-        if (own[m]) dev_store(rx, (b3 * N + row[m]) * 16u, unset);
-      buf = b1;
-      par ^= 1;
+      advance(act);
     }
-    // ---- step control
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int m = 0; m < kQ; ++m) {
-      const int q = w + m * kRwCompute;
-      if (q >= nq) continue;
-      const double2 en = quad_norms(errv[m], nrm2[m]);
-      if (lane == 0)
-        dev_store(rr, (rbuf * NQ + g.quad0 + q) * 16u, publishable(en));
-    }
-    __syncthreads();
-    if (stop) return;
-    __syncthreads();
-    if (cl.accept) {
-#pragma unroll
-      for (int m = 0; m < kQ; ++m) {
-        if (!own[m]) continue;
-        x[m] = make_double2(v[m].x / cl.nrm, v[m].y / cl.nrm);
-        if ((int)row[m] == a.track && cl.nlog >= 1 && cl.nlog <= a.logcap) {
-          LogEnt le;
-          le.t = cl.t;
-          le.h = cl.hacc;
-          le.pop = abs2(x[m].x, x[m].y);
-          a.log[cl.nlog - 1] = le;
-        }
-      }
-    }
-    rbuf = rnext;
+    for (int m = 0; m < kQ; ++m)
+      if (own[m])
+        for (int b = 0; b < ns; ++b)
+          a.X[(long long)row[m] * a.P + grp + (base + b) * a.ngrp] =
+              kMany ? own_rows[b * slot_n + kStages * nr4 + lr[m]] : x[m];
   }
-#pragma unroll
-  for (int m = 0; m < kQ; ++m)
-    if (own[m]) a.X[row[m]] = x[m];
 }
 
-template __global__ void k_rows_run<1>(RowRun, const SysDesc *,
-                                        const RowDesc *, const double *);
-template __global__ void k_rows_run<2>(RowRun, const SysDesc *,
-                                        const RowDesc *, const double *);
-template __global__ void k_rows_run<4>(RowRun, const SysDesc *,
-                                        const RowDesc *, const double *);
+#define MPCI_ROWS(Q, MANY)                                          \
+  template __global__ void k_rows_run<Q, MANY>(RowRun, const SysDesc *, \
+                                               const RowDesc *,     \
+                                               const double *)
+MPCI_ROWS(1, false);
+MPCI_ROWS(2, false);
+MPCI_ROWS(4, false);
+MPCI_ROWS(1, true);
+#undef MPCI_ROWS
 
 // ---------------------------------------------------------------------
 // Persistent tile kernel: whole attempts of one pulse on a larger system in

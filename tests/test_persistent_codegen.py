@@ -29,6 +29,6 @@ def test_persistent_kernels(tmp_path):
              if n.startswith("_Z")]
     priv = [int(p) for p in re.findall(
         r"^\s+\.private_segment_fixed_size:\s+(\d+)", asm, flags=re.M)]
-    assert len(names) == len(priv) == 5
+    assert len(names) == len(priv) == 6
     for n, p in zip(names, priv):
         assert p <= (16 if "k_tiles_run" in n else 0), (n, p)
