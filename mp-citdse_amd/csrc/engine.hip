@@ -157,6 +157,7 @@ struct mpci_prop {
   DevBuf<PulseDev> pulses;
   DevBuf<double> env;
   DevBuf<double> Ftab;
+  char *hstates = nullptr;  // states in pinned host memory
   DevBuf<double> hs;
   DevBuf<LogEnt> log;
   int logcap = 4096;
@@ -188,6 +189,7 @@ struct mpci_prop {
     if (graph) (void)hipGraphDestroy(graph);
     for (auto e : ev) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
+    if (hstates) (void)hipHostFree(hstates);
   }
 };
 
@@ -947,6 +949,7 @@ constexpr long long kSmallPathBytes = 12LL << 20;
 // us.  The launches these replace took 105 us (6 x 300), 164 us (4 x 900),
 // 200 us (4 x 1500), 474 us (He_test.yaml shape), 910 us (He 4 x 4000); the
 // tile form takes 127, 355 and 763 us there.
+constexpr size_t kPinnedStates = 8u << 20;  // bound of the pinned buffer
 constexpr int kWaitLimitMs = 20000;  // time limit of one wait in them
 // Time limit of the start of an ordinary launch: two processes' launches
 // that hold half the device each let go of it after this.
@@ -1313,21 +1316,99 @@ extern "C" int mpci_prop_destroy(mpci_prop *pr) {
   return MPCI_OK;
 }
 
+// States travel between the caller's memory and the batch layout by way of a
+// pinned buffer that a kernel reads or writes in the layout's order, as many
+// pulses at a time as it holds (a copy from pageable memory into a device
+// buffer, a kernel and their waits took 33 us in and 69 us out per state of
+// 335 KB; this 25 and 56 us, for 19 KB 36 and 16 us).  Behind the states it
+// has a double per pulse.  Null where a state is larger than kPinnedStates or
+// there is no pinned memory.
+static char *pinned_states(mpci_prop *pr, int *pulses) {
+  const size_t one = sizeof(double2) * pr->sys->N;
+  const int n = (int)std::min<size_t>(pr->P, kPinnedStates / one);
+  if (n < 1) return nullptr;
+  if (!pr->hstates &&
+      hipHostMalloc((void **)&pr->hstates, n * one + sizeof(double) * pr->P,
+                    hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    pr->hstates = nullptr;
+  }
+  *pulses = n;
+  return pr->hstates;
+}
+
+static int copy_states(mpci_prop *pr, double2 *dst, int dst_stride,
+                       int dst_pulse, const double2 *src, int src_stride,
+                       int src_pulse, int np) {
+  const int N = pr->sys->N;
+  hipLaunchKernelGGL(k_copy_strided, dim3((N + 255) / 256, np), dim3(256), 0,
+                     pr->stream, dst, dst_stride, dst_pulse, src, src_stride,
+                     src_pulse, N);
+  HIPCHK(hipGetLastError());
+  return MPCI_OK;
+}
+
+// Pulses p0 .. p0 + np - 1 of X from ct; the caller waits for the stream.
+static int put_states(mpci_prop *pr, const double *ct, int p0, int np) {
+  const int N = pr->sys->N, P = pr->P;
+  const size_t one = sizeof(double2) * N;
+  const char *from = reinterpret_cast<const char *>(ct);
+  int cap = 0;
+  if (char *h = pinned_states(pr, &cap)) {
+    for (int k = 0; k < np; k += cap) {
+      const int m = std::min(cap, np - k);
+      if (k > 0) HIPCHK(hipStreamSynchronize(pr->stream));
+      std::memcpy(h, from + k * one, m * one);
+      TRY(copy_states(pr, pr->X.p + p0 + k, P, 1,
+                      reinterpret_cast<const double2 *>(h), 1, N, m));
+    }
+    return MPCI_OK;
+  }
+  if (P == 1) return h2d(pr, pr->X.p, ct, one);
+  // one contiguous copy, then a strided kernel copy into the batch layout
+  // (a 2-D copy of N 16-byte rows from host memory moves row by row)
+  if (!pr->xstage.p) TRY(pr->xstage.alloc(N));
+  for (int k = 0; k < np; ++k) {
+    TRY(h2d(pr, pr->xstage.p, from + k * one, one));
+    TRY(copy_states(pr, pr->X.p + p0 + k, P, 1, pr->xstage.p, 1, N, 1));
+  }
+  return MPCI_OK;
+}
+
+// Pulses p0 .. p0 + np - 1 of src (batch layout) to ct, complete on return.
+static int take_states(mpci_prop *pr, const double2 *src, double *ct, int p0,
+                       int np) {
+  const int N = pr->sys->N, P = pr->P;
+  const size_t one = sizeof(double2) * N;
+  char *to = reinterpret_cast<char *>(ct);
+  int cap = 0;
+  if (char *h = pinned_states(pr, &cap)) {
+    for (int k = 0; k < np; k += cap) {
+      const int m = std::min(cap, np - k);
+      TRY(copy_states(pr, reinterpret_cast<double2 *>(h), 1, N, src + p0 + k,
+                      P, 1, m));
+      // the pages of the caller's memory, often new, while the device copies
+      volatile char *c = to + k * one;
+      for (size_t o = 0; o < m * one; o += 4096) c[o] = 0;
+      HIPCHK(hipStreamSynchronize(pr->stream));
+      std::memcpy(to + k * one, h, m * one);
+    }
+    return MPCI_OK;
+  }
+  HIPCHK(hipStreamSynchronize(pr->stream));
+  if (P == 1) return d2h(pr, ct, src, one);
+  if (!pr->xstage.p) TRY(pr->xstage.alloc(N));
+  for (int k = 0; k < np; ++k) {
+    TRY(copy_states(pr, pr->xstage.p, 1, N, src + p0 + k, P, 1, 1));
+    TRY(d2h(pr, to + k * one, pr->xstage.p, one));
+  }
+  return MPCI_OK;
+}
+
 extern "C" int mpci_prop_set_state(mpci_prop *pr, int p, const double *ct) {
   if (!pr || !ct || p < 0 || p >= pr->P)
     return fail(MPCI_ERR_ARG, "mpci_prop_set_state: bad argument");
-  if (pr->P == 1) {
-    return h2d(pr, pr->X.p, ct, sizeof(double2) * pr->sys->N);
-  }
-  // one contiguous copy, then a strided kernel copy into the batch layout
-  // (a 2-D copy of N 16-byte rows from host memory moves row by row)
-  const int N = pr->sys->N;
-  if (!pr->xstage.p) TRY(pr->xstage.alloc(N));
-  HIPCHK(hipMemcpyAsync(pr->xstage.p, ct, sizeof(double2) * N,
-                        hipMemcpyHostToDevice, pr->stream));
-  hipLaunchKernelGGL(k_copy_strided, dim3((N + 255) / 256), dim3(256), 0,
-                     pr->stream, pr->X.p + p, pr->P, pr->xstage.p, 1, N);
-  HIPCHK(hipGetLastError());
+  TRY(put_states(pr, ct, p, 1));
   HIPCHK(hipStreamSynchronize(pr->stream));
   return MPCI_OK;
 }
@@ -1335,22 +1416,18 @@ extern "C" int mpci_prop_set_state(mpci_prop *pr, int p, const double *ct) {
 extern "C" int mpci_prop_get_state(mpci_prop *pr, int p, double *ct) {
   if (!pr || !ct || p < 0 || p >= pr->P)
     return fail(MPCI_ERR_ARG, "mpci_prop_get_state: bad argument");
-  HIPCHK(hipStreamSynchronize(pr->stream));
-  if (pr->P == 1) {
-    return d2h(pr, ct, pr->X.p, sizeof(double2) * pr->sys->N);
-  }
-  const int N = pr->sys->N;
-  if (!pr->xstage.p) TRY(pr->xstage.alloc(N));
-  hipLaunchKernelGGL(k_copy_strided, dim3((N + 255) / 256), dim3(256), 0,
-                     pr->stream, pr->xstage.p, 1, pr->X.p + p, pr->P, N);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(ct, pr->xstage.p, sizeof(double2) * N,
-                        hipMemcpyDeviceToHost, pr->stream));
-  HIPCHK(hipStreamSynchronize(pr->stream));
-  return MPCI_OK;
+  return take_states(pr, pr->X.p, ct, p, 1);
 }
 
 static void drop_graph(mpci_prop *pr);
+
+// The step and field tables only grow, as the envelope store does.
+static int grow_table(mpci_prop *pr, DevBuf<double> &b, size_t n) {
+  if (n <= b.n) return MPCI_OK;
+  HIPCHK(hipStreamSynchronize(pr->stream));
+  drop_graph(pr);
+  return b.alloc(n);
+}
 
 // The envelope store only grows.  A captured step holds its address in the
 // stage kernels' arguments, so when it has to move, the graph is dropped
@@ -1747,11 +1824,12 @@ static int drain_log(mpci_prop *pr, std::vector<Ctl> &c,
   if (maxn > pr->logcap)
     return fail(MPCI_ERR_STATE, "internal: log overflow");
   if (maxn > 0) {
-    std::vector<LogEnt> h((size_t)pr->logcap * pr->P);
+    // entry k of pulse p at k P + p: one copy holds all that were written
+    std::vector<LogEnt> h((size_t)maxn * pr->P);
     TRY(d2h(pr, h.data(), pr->log.p, sizeof(LogEnt) * h.size()));
     for (int p = 0; p < pr->P; ++p)
-      acc[p].insert(acc[p].end(), h.begin() + (size_t)p * pr->logcap,
-                    h.begin() + (size_t)p * pr->logcap + c[p].nlog);
+      for (int k = 0; k < c[p].nlog; ++k)
+        acc[p].push_back(h[(size_t)k * pr->P + p]);
   }
   for (auto &x : c) x.nlog = 0;
   return write_ctl(pr, c);
@@ -1760,16 +1838,28 @@ static int drain_log(mpci_prop *pr, std::vector<Ctl> &c,
 extern "C" int mpci_prop_rhs(mpci_prop *pr, const double *F, const double *x,
                              double *dxdt) {
   if (!pr || !F || !x || !dxdt) return fail(MPCI_ERR_ARG, "NULL argument");
-  for (int p = 0; p < pr->P; ++p)
-    TRY(mpci_prop_set_state(pr, p, x + (size_t)p * 2 * pr->sys->N));
-  std::vector<Ctl> c(pr->P);
-  std::memset(c.data(), 0, sizeof(Ctl) * pr->P);
-  for (int p = 0; p < pr->P; ++p) {
-    c[p].mode = kModeRhs;
-    c[p].fmode = kFieldConst;
-    c[p].Fc = F[p];
+  const int P = pr->P;
+  TRY(put_states(pr, x, 0, P));
+  int cap = 0;
+  char *h = pinned_states(pr, &cap);
+  std::vector<Ctl> c;
+  if (h) {
+    double *Fp = reinterpret_cast<double *>(
+        h + (size_t)cap * sizeof(double2) * pr->sys->N);
+    std::copy(F, F + P, Fp);
+    hipLaunchKernelGGL(k_rhs_ctl_batch, dim3((P + 63) / 64), dim3(64), 0,
+                       pr->stream, pr->ctl.p, Fp, P, 0);
+    HIPCHK(hipGetLastError());
+  } else {
+    c.resize(P);
+    std::memset(c.data(), 0, sizeof(Ctl) * P);
+    for (int p = 0; p < P; ++p) {
+      c[p].mode = kModeRhs;
+      c[p].fmode = kFieldConst;
+      c[p].Fc = F[p];
+    }
+    TRY(start_ctl(pr, c));
   }
-  TRY(start_ctl(pr, c));
   StageArgs a = stage_args(pr, 0);
   a.red = nullptr;
   if (pr->small) {
@@ -1779,15 +1869,16 @@ extern "C" int mpci_prop_rhs(mpci_prop *pr, const double *F, const double *x,
     TRY(launch_stage(pr, a));
   }
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(pr->stream));
-  std::vector<double2> k(pr->NP);
-  TRY(d2h(pr, k.data(), pr->K.p, sizeof(double2) * pr->NP));
-  const int N = pr->sys->N;
-  for (int p = 0; p < pr->P; ++p)
-    for (int i = 0; i < N; ++i) {
-      dxdt[(size_t)p * 2 * N + 2 * i] = k[(size_t)i * pr->P + p].x;
-      dxdt[(size_t)p * 2 * N + 2 * i + 1] = k[(size_t)i * pr->P + p].y;
-    }
+  if (h) {
+    hipLaunchKernelGGL(k_rhs_ctl_batch, dim3((P + 63) / 64), dim3(64), 0,
+                       pr->stream, pr->ctl.p,
+                       reinterpret_cast<const double *>(
+                           h + (size_t)cap * sizeof(double2) * pr->sys->N),
+                       P, 1);
+    HIPCHK(hipGetLastError());
+  }
+  TRY(take_states(pr, pr->K.p, dxdt, 0, P));
+  if (h) return MPCI_OK;
   for (auto &x : c) x.done = 1;
   return write_ctl(pr, c);
 }
@@ -1894,10 +1985,9 @@ extern "C" int mpci_prop_fixed(mpci_prop *pr, double t0, double dt, int steps,
   if (track < 0 || track >= pr->sys->N)
     return fail(MPCI_ERR_ARG, "track index out of range");
   if (steps == 0) return MPCI_OK;
-  TRY(pr->Ftab.alloc((size_t)pr->P * steps));
+  TRY(grow_table(pr, pr->Ftab, (size_t)pr->P * steps));
   TRY(h2d(pr, pr->Ftab.p, F, sizeof(double) * pr->P * steps));
   pr->track = track;
-  drop_graph(pr);  // Ftab moved
   std::vector<Ctl> c(pr->P);
   std::memset(c.data(), 0, sizeof(Ctl) * pr->P);
   for (auto &x : c) {
@@ -2377,9 +2467,8 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
 // segment recompute.
 static int run_schedule(mpci_prop *pr, const double *t0, const int *n,
                         int stride, const double *hs) {
-  TRY(pr->hs.alloc((size_t)pr->P * std::max(stride, 1)));
+  TRY(grow_table(pr, pr->hs, (size_t)pr->P * std::max(stride, 1)));
   TRY(h2d(pr, pr->hs.p, hs, sizeof(double) * pr->P * stride));
-  drop_graph(pr);  // hs moved
   std::vector<Ctl> c(pr->P);
   std::memset(c.data(), 0, sizeof(Ctl) * pr->P);
   for (int p = 0; p < pr->P; ++p) {

@@ -1744,7 +1744,7 @@ __device__ __forceinline__ void apply_block(double2 *__restrict__ X,
     le.t = c.t;
     le.h = c.hacc;
     le.pop = abs2(xn.x, xn.y);
-    log[(long long)p * logcap + c.nlog - 1] = le;
+    log[(long long)(c.nlog - 1) * P + p] = le;
   }
   if (st.xn) {
     const int slot = (steps_taken(c) - 1) % st.cap;
@@ -1977,13 +1977,32 @@ __global__ void k_rhs_ctl(Ctl *ctl, double F) {
   }
 }
 
-// One pulse's state into or out of the pulse-interleaved batch layout
-// (element i of pulse p at i P + p): dst[i dst_stride] = src[i src_stride].
+// The pulses' control records of one RHS evaluation from their fields F,
+// live or (done) afterwards.
+__global__ void k_rhs_ctl_batch(Ctl *ctl, const double *__restrict__ F, int P,
+                                int done) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  Ctl c{};
+  c.mode = kModeRhs;
+  c.fmode = kFieldConst;
+  c.done = done;
+  c.Fc = F[p];
+  for (int s = 0; s < kStages; ++s) c.Fs[s] = F[p];
+  ctl[p] = c;
+}
+
+// Pulses' states into or out of the pulse-interleaved batch layout (element
+// i of pulse p at i P + p), pulse blockIdx.y:
+// dst[y dst_pulse + i dst_stride] = src[y src_pulse + i src_stride].
 __global__ __launch_bounds__(256) void k_copy_strided(
-    double2 *__restrict__ dst, int dst_stride, const double2 *__restrict__ src,
-    int src_stride, int n) {
+    double2 *__restrict__ dst, int dst_stride, int dst_pulse,
+    const double2 *__restrict__ src, int src_stride, int src_pulse, int n) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) dst[(long long)i * dst_stride] = src[(long long)i * src_stride];
+  const long long y = blockIdx.y;
+  if (i < n)
+    dst[y * dst_pulse + (long long)i * dst_stride] =
+        src[y * src_pulse + (long long)i * src_stride];
 }
 
 // ---------------------------------------------------------------------

@@ -629,8 +629,8 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
             le.t = c.t;
             le.h = c.hacc;
             le.pop = abs2(x[m].x, x[m].y);
-            a.log[(long long)(grp + (base + b) * a.ngrp) * a.logcap + c.nlog -
-                  1] = le;
+            a.log[(long long)(c.nlog - 1) * a.P + grp + (base + b) * a.ngrp] =
+                le;
           }
         }
       }
