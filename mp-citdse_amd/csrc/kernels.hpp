@@ -139,6 +139,8 @@ struct GroupMember {
 __global__ void k_relayout_gemv(const double *D, int sL, int sL1, int ncb,
                                 long long nelem, int job0, int njobs,
                                 double *out);
+// kOnce: no control record is looked at; kNt: non-temporal dipole loads
+template <bool kOnce, bool kNt>
 __global__ void k_gemv_tile(const TileJob *jobs, int njobs, const double *Dg,
                             const double2 *X, double2 *part, const SysDesc *d,
                             const Ctl *ctl, int rev);
@@ -204,7 +206,8 @@ __global__ void k_adj_stage(AdjArgs a, const SysDesc *d);
 __global__ void k_weighted_pop(const double2 *X, const double *W, int N, int P,
                                double *out);
 // Ctl record of one RHS evaluation at constant field F (mode RHS).
-__global__ void k_rhs_ctl(Ctl *ctl, double F);
+__global__ void k_rhs1(const double2 *part, const double2 *X, const double *E,
+                       double F, double2 *dxdt, const SysDesc *d);
 __global__ void k_rhs_ctl_batch(Ctl *ctl, const double *F, int P, int done);
 // grid (rows / 256, pulses)
 __global__ void k_copy_strided(double2 *dst, int dst_stride, int dst_pulse,
