@@ -815,7 +815,8 @@ static const GemmCand kGemmCands[] = {
     {2, 2, 2, 2, 2, 16, 4}, {2, 4, 2, 2, 2, 16, 1}, {2, 4, 2, 2, 2, 16, 2},
     {2, 4, 2, 2, 2, 16, 4}, {2, 2, 4, 2, 2, 16, 1}, {2, 2, 4, 2, 2, 16, 2},
     {2, 2, 4, 2, 2, 16, 4}, {2, 4, 4, 2, 2, 16, 1}, {2, 4, 4, 2, 2, 16, 2},
-    {2, 4, 4, 2, 2, 16, 4}, {3, 16, 1, 2, 2, 16, 1}, {3, 16, 1, 2, 2, 16, 2}};
+    {2, 4, 4, 2, 2, 16, 4}, {2, 2, 1, 2, 2, 16, 8}, {2, 4, 1, 2, 2, 16, 8},
+    {3, 16, 1, 2, 2, 16, 1}, {3, 16, 1, 2, 2, 16, 2}};
 
 // k_gemm_lds addresses its operands through 32-bit buffer offsets: every
 // D_L copy and the X slab of the propagator must stay below 2 GiB.
@@ -888,6 +889,15 @@ static int tune_gemm(mpci_prop *pr, const GemmCand *only) {
       const bool lds_ok = gemm_lds_fits(pr);
       for (const GemmCand &cd : kGemmCands) {
         if (cd.kind >= 2 && !lds_ok) continue;
+        // finer splits are for launches of few panels, whose chains of K
+        // chunks are what they wait for (3 x 1000, 8 pulses: 21.0 -> 16.3 us
+        // a stage, 6 x 800, 6 pulses: 23.6 -> 21.3 us); with eight panels a
+        // compute unit and more they only add partial sums (4 x 2200, 6
+        // pulses: 56.9 -> 62 us)
+        if (cd.ks > 4 &&
+            gemm_job_list(pr, cd.wm, cd.wn, cd.fm, cd.fn, cd.ks, 0).size() >
+                8 * (size_t)pr->sys->ncu)
+          continue;
         float ms = 0.f;
         rc = time_gemm_cand(pr, cd, e0, e1, &ms);
         if (rc != MPCI_OK) break;

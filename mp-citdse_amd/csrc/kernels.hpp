@@ -205,7 +205,7 @@ __global__ void k_adj_init(AdjArgs a, const SysDesc *d);
 __global__ void k_adj_stage(AdjArgs a, const SysDesc *d);
 __global__ void k_weighted_pop(const double2 *X, const double *W, int N, int P,
                                double *out);
-// Ctl record of one RHS evaluation at constant field F (mode RHS).
+// dx/dt of one state at field F from its coupling partials.
 __global__ void k_rhs1(const double2 *part, const double2 *X, const double *E,
                        double F, double2 *dxdt, const SysDesc *d);
 __global__ void k_rhs_ctl_batch(Ctl *ctl, const double *F, int P, int done);
