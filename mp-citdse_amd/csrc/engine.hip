@@ -707,8 +707,9 @@ static int launch_gemm(mpci_prop *pr, const double2 *xin,
                         dim3(64 * WM * WN), 0, pr->stream, e0, e1, 0,       \
                         pr->dgjobs.p, sys->Dr.p, sys->dr_off.p, X, part,    \
                         pr->ddesc.p, pr->ctl.p)
-#define MPCI_GEMM_LDS(WM, WN)                                                \
-  hipExtLaunchKernelGGL((k_gemm_lds<WM, WN>), grid, dim3(64 * WM * WN), 0,   \
+#define MPCI_GEMM_LDS(WM, WN, FM, FN)                                        \
+  hipExtLaunchKernelGGL((k_gemm_lds<WM, WN, FM, FN>), grid,                  \
+                        dim3(64 * WM * WN), 0,                               \
                         pr->stream, e0, e1, 0, pr->dgjobs.p, sys->Dr.p,      \
                         sys->dr_off.p, X, part, pr->ddesc.p, pr->ctl.p)
   const int wm = pr->gm_wm, wn = pr->gm_wn, tk = pr->gm_tk;
@@ -718,18 +719,32 @@ static int launch_gemm(mpci_prop *pr, const double2 *xin,
                           0, pr->dgjobs.p, sys->Dr.p, sys->dr_off.p, X, part,
                           pr->ddesc.p, pr->ctl.p);
   } else if (pr->gm_kind == 2) {
-    if (wm == 2 && wn == 1)
-      MPCI_GEMM_LDS(2, 1);
-    else if (wm == 4 && wn == 1)
-      MPCI_GEMM_LDS(4, 1);
-    else if (wm == 2 && wn == 2)
-      MPCI_GEMM_LDS(2, 2);
-    else if (wm == 4 && wn == 2)
-      MPCI_GEMM_LDS(4, 2);
-    else if (wm == 2 && wn == 4)
-      MPCI_GEMM_LDS(2, 4);
-    else
-      MPCI_GEMM_LDS(4, 4);
+    const int w = wm * 10 + wn;
+    if (f == 11) {
+      if (w == 22)
+        MPCI_GEMM_LDS(2, 2, 1, 1);
+      else if (w == 42)
+        MPCI_GEMM_LDS(4, 2, 1, 1);
+      else
+        MPCI_GEMM_LDS(4, 1, 1, 1);
+    } else if (f == 21) {
+      if (w == 22)
+        MPCI_GEMM_LDS(2, 2, 2, 1);
+      else
+        MPCI_GEMM_LDS(4, 1, 2, 1);
+    } else if (w == 21) {
+      MPCI_GEMM_LDS(2, 1, 2, 2);
+    } else if (w == 41) {
+      MPCI_GEMM_LDS(4, 1, 2, 2);
+    } else if (w == 22) {
+      MPCI_GEMM_LDS(2, 2, 2, 2);
+    } else if (w == 42) {
+      MPCI_GEMM_LDS(4, 2, 2, 2);
+    } else if (w == 24) {
+      MPCI_GEMM_LDS(2, 4, 2, 2);
+    } else {
+      MPCI_GEMM_LDS(4, 4, 2, 2);
+    }
   } else if (pr->gm_kind == 0) {
     if (wm == 2 && wn == 2)
       MPCI_GEMM(2, 2);
@@ -816,6 +831,11 @@ static const GemmCand kGemmCands[] = {
     {2, 4, 2, 2, 2, 16, 4}, {2, 2, 4, 2, 2, 16, 1}, {2, 2, 4, 2, 2, 16, 2},
     {2, 2, 4, 2, 2, 16, 4}, {2, 4, 4, 2, 2, 16, 1}, {2, 4, 4, 2, 2, 16, 2},
     {2, 4, 4, 2, 2, 16, 4}, {2, 2, 1, 2, 2, 16, 8}, {2, 4, 1, 2, 2, 16, 8},
+    {2, 2, 2, 1, 1, 16, 1}, {2, 2, 2, 1, 1, 16, 2}, {2, 2, 2, 1, 1, 16, 4},
+    {2, 2, 2, 1, 1, 16, 8}, {2, 4, 2, 1, 1, 16, 1}, {2, 4, 2, 1, 1, 16, 4},
+    {2, 4, 2, 1, 1, 16, 8}, {2, 2, 2, 2, 1, 16, 2}, {2, 2, 2, 2, 1, 16, 4},
+    {2, 4, 1, 1, 1, 16, 2}, {2, 4, 1, 1, 1, 16, 4}, {2, 4, 1, 1, 1, 16, 8},
+    {2, 4, 1, 2, 1, 16, 4},
     {3, 16, 1, 2, 2, 16, 1}, {3, 16, 1, 2, 2, 16, 2}};
 
 // k_gemm_lds addresses its operands through 32-bit buffer offsets: every
@@ -843,7 +863,7 @@ static StageArgs stage_args(mpci_prop *pr, int s);
 // behind the best K-split tile at 16 pulses on most devices, while whole
 // attempts run it 2-5 % faster.)
 static int time_gemm_cand(mpci_prop *pr, const GemmCand &cd, hipEvent_t e0,
-                          hipEvent_t e1, float *ms) {
+                          hipEvent_t e1, float *ms, float best) {
   TRY(init_desc_kind(pr, cd.kind, cd.ks));
   TRY(build_gemm_jobs(pr, cd.kind, cd.wm, cd.wn, cd.fm, cd.fn, cd.tk, cd.ks));
   auto eval = [&](int s) {
@@ -852,9 +872,16 @@ static int time_gemm_cand(mpci_prop *pr, const GemmCand &cd, hipEvent_t e0,
     a.xs_store = nullptr;  // leave any adjoint stage store alone
     return launch_stage(pr, a);
   };
-  // two warm evaluations, then the twelve stages timed
+  // two warm evaluations, then the twelve stages timed unless the second is
+  // three times slower than the best so far
   constexpr int kReps = kStages - 1;
-  for (int s = 0; s < 2; ++s) TRY(eval(s));
+  TRY(eval(0));
+  HIPCHK(hipEventRecord(e0, pr->stream));
+  TRY(eval(1));
+  HIPCHK(hipEventRecord(e1, pr->stream));
+  HIPCHK(hipEventSynchronize(e1));
+  HIPCHK(hipEventElapsedTime(ms, e0, e1));
+  if (*ms > 3.f * best + 0.02f) return MPCI_OK;
   HIPCHK(hipEventRecord(e0, pr->stream));
   for (int s = 0; s < kReps; ++s) TRY(eval(s));
   HIPCHK(hipEventRecord(e1, pr->stream));
@@ -871,6 +898,8 @@ static int set_all_live(mpci_prop *pr, int done) {
   return h2d(pr, pr->ctl.p, c.data(), sizeof(Ctl) * pr->P);
 }
 
+constexpr long long kFineTiles = 1 << 16;
+
 // Times every candidate of kGemmCands (or only `only`, when given), sets up
 // the fastest (GEMM plus the stage kernel's reading of its partial sums)
 // and, for a full search, records it in the system's tune cache for this
@@ -884,22 +913,30 @@ static int tune_gemm(mpci_prop *pr, const GemmCand *only) {
   GemmCand bc = only ? *only : kGemmCands[0];
   if (rc == MPCI_OK) {
     if (only) {
-      rc = time_gemm_cand(pr, *only, e0, e1, &best);
+      rc = time_gemm_cand(pr, *only, e0, e1, &best, best);
     } else {
       const bool lds_ok = gemm_lds_fits(pr);
       for (const GemmCand &cd : kGemmCands) {
         if (cd.kind >= 2 && !lds_ok) continue;
-        // finer splits are for launches of few panels, whose chains of K
-        // chunks are what they wait for (3 x 1000, 8 pulses: 21.0 -> 16.3 us
-        // a stage, 6 x 800, 6 pulses: 23.6 -> 21.3 us); with eight panels a
-        // compute unit and more they only add partial sums (4 x 2200, 6
-        // pulses: 56.9 -> 62 us)
-        if (cd.ks > 4 &&
-            gemm_job_list(pr, cd.wm, cd.wn, cd.fm, cd.fn, cd.ks, 0).size() >
-                8 * (size_t)pr->sys->ncu)
+        // finer splits, and tiles of fewer blocks a wave, are for launches of
+        // few panels, which wait for their chains of K chunks and leave
+        // matrix cores idle (us a stage with the stage kernel, against the
+        // 2 x 2 blocks and splits of up to four: 3 x 1000, 8 pulses 21.0 ->
+        // 14.5; 6 x 800, 6 pulses 23.6 -> 17.2; 5 x 600, 12 pulses 17.3 ->
+        // 14.6; 4 x 500, 64 pulses 23.4 -> 21.2); with eight panels of 2 x 2
+        // blocks a compute unit and more they add partial sums and reads (4
+        // x 2200, 6 pulses, split in eight: 56.9 -> 62; 21 x 998, 32 pulses,
+        // 1 x 1 blocks: 119.9 -> 127).  Below kFineTiles dipoles a launch
+        // takes what launches take (3 x 30, 40 pulses: 8.6 to 9 us a stage
+        // with every tile).
+        const size_t most = (size_t)(32 / (cd.fm * cd.fn)) * pr->sys->ncu;
+        if ((cd.ks > 4 || cd.fm * cd.fn < 4) &&
+            (pr->sys->S < kFineTiles ||
+             gemm_job_list(pr, cd.wm, cd.wn, cd.fm, cd.fn, cd.ks, 0).size() >
+                 most))
           continue;
         float ms = 0.f;
-        rc = time_gemm_cand(pr, cd, e0, e1, &ms);
+        rc = time_gemm_cand(pr, cd, e0, e1, &ms, best);
         if (rc != MPCI_OK) break;
         if (ms < best) {
           best = ms;
@@ -1037,13 +1074,13 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
 // groups of workgroups take some each and a group runs a stage of each of its
 // pulses in turn, which hides one's exchange behind the others'.  A pulse
 // then costs its group about 20 us an attempt while the rows' chunks fit in
-// registers, and more past that; the batched launches cost 110 to 300 us an
-// attempt at any P.  Measured, row form against batched launches, in us per
-// attempt: 60 x 8, P = 5 28 / 128, P = 40 97 / 139, P = 64 151 / 148; 198 x
-// 4, P = 5 45 / 148, P = 16 81 / 158, P = 40 197 / 168; 300 x 6, P = 5 66 /
-// 171, P = 16 159 / 194, P = 40 392 / 250; 800 x 5, P = 3 93 / 270, P = 8
-// 275 / 276; 2000 x 2, P = 2 105 / 314, P = 8 456 / 342; 1500, 1000, 1500,
-// P = 3 257 / 304, P = 5 420 / 312.
+// registers, and more past that; the batched launches cost 105 to 260 us an
+// attempt at any small P.  Measured, row form against batched launches, in us
+// per attempt: 60 x 8, P = 5 28 / 112, P = 40 88 / 117, P = 56 119 / 120; 198
+// x 4, P = 5 45 / 123, P = 24 112 / 132; 300 x 6, P = 5 64 / 139, P = 12 118 /
+// 149, P = 20 196 / 175; 800 x 5, P = 3 93 / 210, P = 5 164 / 218; 2000 x 2, P
+// = 2 103 / 261, P = 4 196 / 265, P = 5 275 / 264; 1500, 1000, 1500, P = 2
+// 175 / 234; 80 x 32, P = 5 92 / 144.
 static bool rows_pay(const mpci_prop *pr) {
   const mpci_system *sys = pr->sys;
   const int n16 = row_groups(sys);
@@ -1055,10 +1092,11 @@ static bool rows_pay(const mpci_prop *pr) {
   if (n16 > sys->ncu) return false;
   const int groups = std::min(pr->P, sys->ncu / n16);
   const int each = (pr->P + groups - 1) / groups;
-  const double pulse = 20.0 + 2.4 * std::max(chunks - kRwReg, 0);
-  const double batched = 110.0 + 0.15 * std::min(smax, 1000) +
-                         2.5e-6 * (double)sys->S * pr->P;
-  return each * pulse < 0.95 * batched;
+  const int c = std::max(chunks - kRwReg, 0);
+  const double pulse = 20.0 + 1.2 * c + 0.045 * c * c;
+  const double batched = 100.0 + 0.075 * std::min(smax, 1500) + 1.1 * sys->nb +
+                         2e-6 * (double)sys->S * pr->P;
+  return each * pulse < 0.97 * batched;
 }
 
 struct TilePlan {

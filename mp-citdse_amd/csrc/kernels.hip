@@ -599,7 +599,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_db(
 // ---------------------------------------------------------------------
 // Batched coupling on FP64 MFMA with direct-to-LDS operand loads.  Same
 // panels, operand layouts and partial slots as k_gemm_db (wm x wn waves,
-// each 2 x 2 blocks of 16 x 16; K in chunks of 16), but the chunk operands
+// each fm x fn blocks of 16 x 16, two each way, or for launches of few panels
+// fewer, so that the chunks' chains of MFMAs are shorter and a panel pads
+// less; K in chunks of 16), but the chunk operands
 // travel HBM -> LDS with buffer_load_dwordx4 ... lds: no VGPR staging, no
 // LDS store instructions, and a lane outside the panel gets an offset
 // beyond the buffer's range, which the hardware returns as zeros.
@@ -619,17 +621,21 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_db(
 // ---------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-template <int WM, int WN, int DIR>
+template <int WM, int WN, int FM, int FN, int DIR>
 __device__ __forceinline__ void gemm_lds_body(
     const GemmJob &jb, __amdgpu_buffer_rsrc_t rsA, __amdgpu_buffer_rsrc_t rsB,
     double *__restrict__ out, int Mdim, int P2, double *As0, double *As1,
     double *Bs0, double *Bs1) {
-  constexpr int TM = 32 * WM, TN = 32 * WN, TK = 16;
+  constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN, TK = 16;
+  static_assert(TM <= 128 && TN <= 128, "a load holds whole rows");
   constexpr int NW = WM * WN;
   constexpr int NIA = TM * TK / 128, NIB = TK * TN / 128;  // 1 KiB loads
-  static_assert(NIA % NW == 0 && NIB % NW == 0, "loads must split evenly");
-  constexpr int LA = NIA / NW, LB = NIB / NW;  // per wave
+  // per wave; with fewer loads than waves, the first waves have one each
+  static_assert((NIA % NW == 0 || NIA < NW) && (NIB % NW == 0 || NIB < NW),
+                "loads must split evenly");
+  constexpr int LA = NIA < NW ? 1 : NIA / NW, LB = NIB < NW ? 1 : NIB / NW;
   constexpr unsigned kOut = 0x80000000u;       // beyond any buffer range
+  constexpr int kSwB = TN >= 32 ? 8 : 0;  // four rows of 16: no conflict
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int ld = jb.ld;
 
@@ -662,7 +668,7 @@ __device__ __forceinline__ void gemm_lds_body(
     constexpr int PPR = TN / 2;
     const int I = w * LB + u;
     const int krow = I * (128 / TN) + lane / PPR, q = lane % PPR;
-    const int gn = jb.n0 + 2 * (q ^ (8 * (krow & 1)));
+    const int gn = jb.n0 + 2 * (q ^ (kSwB * (krow & 1)));
     b_in[u] = gn < P2;
     b_k[u] = jb.k0 + krow;
     b_off[u] = b_in[u] ? (unsigned)(((jb.k0 + krow) * P2 + gn) * 8) : 0u;
@@ -673,6 +679,7 @@ __device__ __forceinline__ void gemm_lds_body(
   auto issue = [&](int c, double *As, double *Bs) {
 #pragma unroll
     for (int u = 0; u < LA; ++u) {
+      if (NIA < NW && w >= NIA) break;  // uniform over the wave
       const bool ok = a_in[u] && a_k[u] + c * TK < jb.k1;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rsA, (lds_void_t *)(As + (w * LA + u) * 128), 16,
@@ -680,6 +687,7 @@ __device__ __forceinline__ void gemm_lds_body(
     }
 #pragma unroll
     for (int u = 0; u < LB; ++u) {
+      if (NIB < NW && w >= NIB) break;
       const bool ok = b_in[u] && b_k[u] + c * TK < jb.k1;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rsB, (lds_void_t *)(Bs + (w * LB + u) * 128), 16,
@@ -691,45 +699,45 @@ __device__ __forceinline__ void gemm_lds_body(
   const int li = lane & 15, lk = lane >> 4;
   // fragment read offsets (doubles) at k-step 0.  k-major layouts: k-step
   // ks adds 4 ks rows.  A dir 0: element (m, k) sits at
-  // 16 m + 2 ((k >> 1) ^ sw) + (k & 1), sw = (m >> 1) & 7; the two blocks
-  // bi = 0, 1 (m and m + 16) share sw, and k >> 1 = 2 ks + (lk >> 1)
-  int aoff[2], boff[2];
+  // 16 m + 2 ((k >> 1) ^ sw) + (k & 1), sw = (m >> 1) & 7; the blocks bi
+  // (m, m + 16) share sw, and k >> 1 = 2 ks + (lk >> 1)
+  int aoff[FM], boff[FN];
 #pragma unroll
-  for (int bi = 0; bi < 2; ++bi) {
-    const int m = wm * 32 + bi * 16 + li;
+  for (int bi = 0; bi < FM; ++bi) {
+    const int m = wm * 16 * FM + bi * 16 + li;
     aoff[bi] = DIR == 0 ? m * TK + (lk & 1)
                         : lk * TM + 2 * ((m >> 1) ^ (8 * (lk & 1))) + (m & 1);
   }
   int a_sw = ((li >> 1) & 7) ^ (lk >> 1);  // dir 0: pair slot at k-step 0
 #pragma unroll
-  for (int bj = 0; bj < 2; ++bj) {
-    const int n = wn * 32 + bj * 16 + li;
-    boff[bj] = lk * TN + 2 * ((n >> 1) ^ (8 * (lk & 1))) + (n & 1);
+  for (int bj = 0; bj < FN; ++bj) {
+    const int n = wn * 16 * FN + bj * 16 + li;
+    boff[bj] = lk * TN + 2 * ((n >> 1) ^ (kSwB * (lk & 1))) + (n & 1);
   }
 
-  dmf4 acc[2][2];
+  dmf4 acc[FM][FN];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < FM; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = dmf4{0.0, 0.0, 0.0, 0.0};
+    for (int b = 0; b < FN; ++b) acc[a][b] = dmf4{0.0, 0.0, 0.0, 0.0};
   auto mfma_chunk = [&](const double *As, const double *Bs) {
     // recomputed per chunk rather than held in registers across the loop
     asm volatile("" : "+v"(a_sw));
 #pragma unroll
     for (int ks = 0; ks < TK / 4; ++ks) {
-      double a[2], bb[2];
+      double a[FM], bb[FN];
       // dir 0: (2 ks + (lk >> 1)) ^ sw = 2 ks ^ a_sw, as 2 ks has no low
       // bit
       const int slot = DIR == 0 ? ((2 * ks) ^ a_sw) : 0;
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
+      for (int bi = 0; bi < FM; ++bi)
         a[bi] = DIR == 0 ? As[aoff[bi] + 2 * slot] : As[aoff[bi] + 4 * ks * TM];
 #pragma unroll
-      for (int bj = 0; bj < 2; ++bj) bb[bj] = Bs[boff[bj] + 4 * ks * TN];
+      for (int bj = 0; bj < FN; ++bj) bb[bj] = Bs[boff[bj] + 4 * ks * TN];
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
+      for (int bi = 0; bi < FM; ++bi)
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
+        for (int bj = 0; bj < FN; ++bj)
           acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(
               a[bi], bb[bj], acc[bi][bj], 0, 0, 0);
     }
@@ -756,25 +764,25 @@ __device__ __forceinline__ void gemm_lds_body(
   if (c < nch) mfma_chunk(As0, Bs0);  // odd chunk count: the last one
 
 #pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
+  for (int bi = 0; bi < FM; ++bi)
 #pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
+    for (int bj = 0; bj < FN; ++bj)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = jb.m0 + wm * 32 + bi * 16 + 4 * r + lk;
-        const int n = jb.n0 + wn * 32 + bj * 16 + li;
+        const int m = jb.m0 + wm * 16 * FM + bi * 16 + 4 * r + lk;
+        const int n = jb.n0 + wn * 16 * FN + bj * 16 + li;
         if (m < Mdim && n < P2) out[(long long)m * P2 + n] = acc[bi][bj][r];
       }
 }
 
 // One panel job of the direct-to-LDS GEMM (the body of k_gemm_lds and of
 // its grouped form k_gemm_lds_g).
-template <int WM, int WN>
+template <int WM, int WN, int FM, int FN>
 __device__ __forceinline__ void gemm_lds_panel(
     const GemmJob &jb, const double *__restrict__ Dr,
     const long long *__restrict__ dr_off, const double *__restrict__ X,
     double *__restrict__ part, const SysDesc &d, const Ctl *__restrict__ ctl) {
-  constexpr int TM = 32 * WM, TN = 32 * WN, TK = 16;
+  constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN, TK = 16;
   constexpr int NTH = 64 * WM * WN;
   __shared__ __align__(16) double As0[TM * TK], As1[TM * TK];
   __shared__ __align__(16) double Bs0[TK * TN], Bs1[TK * TN];
@@ -810,14 +818,14 @@ __device__ __forceinline__ void gemm_lds_panel(
       jb.dir == 0 ? d.row_part_off[L] : d.col_part_off[L];  // double2 units
   double *out = part + 2 * base + (long long)jb.q * Mdim * P2;
   if (jb.dir == 0)
-    gemm_lds_body<WM, WN, 0>(jb, rsA, rsB, out, Mdim, P2, As0, As1, Bs0, Bs1);
+    gemm_lds_body<WM, WN, FM, FN, 0>(jb, rsA, rsB, out, Mdim, P2, As0, As1, Bs0, Bs1);
   else
-    gemm_lds_body<WM, WN, 1>(jb, rsA, rsB, out, Mdim, P2, As0, As1, Bs0, Bs1);
+    gemm_lds_body<WM, WN, FM, FN, 1>(jb, rsA, rsB, out, Mdim, P2, As0, As1, Bs0, Bs1);
 }
 
 // eight-wave tiles: registers held to 80 so that three workgroups (the
 // LDS limit, 48 KiB each) share a compute unit
-template <int WM, int WN>
+template <int WM, int WN, int FM, int FN>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((
     amdgpu_waves_per_eu(WM * WN == 8 ? 6 : 1))) void k_gemm_lds(
     const GemmJob *__restrict__ jobs, const double *__restrict__ Dr,
@@ -825,7 +833,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((
     double *__restrict__ part, const SysDesc *__restrict__ dp,
     const Ctl *__restrict__ ctl) {
   const GemmJob jb = jobs[blockIdx.x];
-  gemm_lds_panel<WM, WN>(jb, Dr, dr_off, X, part, *dp, ctl);
+  gemm_lds_panel<WM, WN, FM, FN>(jb, Dr, dr_off, X, part, *dp, ctl);
 }
 
 // Grouped form: one launch over the panels of several members (each job
@@ -836,22 +844,30 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((
     const GemmJob *__restrict__ jobs, GroupGemm g, int s) {
   const GemmJob jb = jobs[blockIdx.x];
   const int i = jb.member;
-  gemm_lds_panel<WM, WN>(jb, g.Dr[i], g.dr_off[i], s == 0 ? g.X[i] : g.Xs[i],
+  gemm_lds_panel<WM, WN, 2, 2>(jb, g.Dr[i], g.dr_off[i], s == 0 ? g.X[i] : g.Xs[i],
                          g.part[i], *g.d[i], g.ctl[i]);
 }
 
-#define MPCI_GEMM_LDS(WM, WN)                                                 \
-  template __global__ void k_gemm_lds<WM, WN>(                               \
-      const GemmJob *, const double *, const long long *, const double *,    \
-      double *, const SysDesc *, const Ctl *);                               \
+#define MPCI_GEMM_LDS(WM, WN, FM, FN)                                      \
+  template __global__ void k_gemm_lds<WM, WN, FM, FN>(                    \
+      const GemmJob *, const double *, const long long *, const double *, \
+      double *, const SysDesc *, const Ctl *);
+#define MPCI_GEMM_LDS_G(WM, WN)                                             \
+  MPCI_GEMM_LDS(WM, WN, 2, 2)                                               \
   template __global__ void k_gemm_lds_g<WM, WN>(const GemmJob *, GroupGemm, \
-                                                 int);
-MPCI_GEMM_LDS(2, 1)
-MPCI_GEMM_LDS(4, 1)
-MPCI_GEMM_LDS(2, 2)
-MPCI_GEMM_LDS(4, 2)
-MPCI_GEMM_LDS(2, 4)
-MPCI_GEMM_LDS(4, 4)
+                                                int);
+MPCI_GEMM_LDS_G(2, 1)
+MPCI_GEMM_LDS_G(4, 1)
+MPCI_GEMM_LDS_G(2, 2)
+MPCI_GEMM_LDS_G(4, 2)
+MPCI_GEMM_LDS_G(2, 4)
+MPCI_GEMM_LDS_G(4, 4)
+MPCI_GEMM_LDS(2, 2, 1, 1)
+MPCI_GEMM_LDS(4, 2, 1, 1)
+MPCI_GEMM_LDS(2, 2, 2, 1)
+MPCI_GEMM_LDS(4, 1, 1, 1)
+MPCI_GEMM_LDS(4, 1, 2, 1)
+#undef MPCI_GEMM_LDS_G
 #undef MPCI_GEMM_LDS
 
 // ---------------------------------------------------------------------

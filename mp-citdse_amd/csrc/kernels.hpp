@@ -144,7 +144,7 @@ template <bool kOnce, bool kNt>
 __global__ void k_gemv_tile(const TileJob *jobs, int njobs, const double *Dg,
                             const double2 *X, double2 *part, const SysDesc *d,
                             const Ctl *ctl, int rev);
-template <int WM, int WN>
+template <int WM, int WN, int FM, int FN>
 __global__ void k_gemm_lds(const GemmJob *jobs, const double *Dr,
                            const long long *dr_off, const double *X,
                            double *part, const SysDesc *d, const Ctl *ctl);

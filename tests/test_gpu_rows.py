@@ -114,10 +114,10 @@ def test_persistent_tiles_against_oracle(mpci, oracle, s, gauge):
 
 
 # one and several pulses a group, groups with a pulse less, a workgroup's
-# eight slots used up (each pulse of [1000, 4] needs 64 of the 256)
+# eight slots used up (nine pulses a group of the blocks 950, 2, 2, ..)
 @pytest.mark.parametrize("s,P", [([1, 1], 2), ([17, 64, 65, 5], 3),
                                  ([60, 72, 48], 100), ([300] * 6, 5),
-                                 ([250] * 16, 3), ([1000, 4], 38),
+                                 ([250] * 16, 3), ([950] + [2] * 20, 26),
                                  ([2000, 2000], 2)])
 def test_batch_equals_single_pulses(mpci, s, P):
     """A batch in the persistent row form: every pulse equals its own run
