@@ -495,7 +495,10 @@ static long long fill_desc(const mpci_system *sys, int P, int ks,
 }
 
 static int upload_desc(mpci_prop *pr, long long o) {
-  TRY(pr->part.alloc(std::max<long long>(o, 1)));
+  // (the tile search, which changes the layout for every candidate, makes
+  // both buffers exact at its end)
+  if ((size_t)std::max<long long>(o, 1) > pr->part.n)
+    TRY(pr->part.alloc(std::max<long long>(o, 1)));
   if (!pr->ddesc.p) TRY(pr->ddesc.alloc(1));
   TRY(h2d(pr, pr->ddesc.p, &pr->desc, sizeof(SysDesc)));
   return MPCI_OK;
@@ -676,7 +679,7 @@ static int build_gemm_jobs(mpci_prop *pr, int kind, int wm, int wn, int fm,
                            int fn, int tk, int ks) {
   pr->gjobs = kind == 3 ? pair_job_list(pr, ks, 0)
                         : gemm_job_list(pr, wm, wn, fm, fn, ks, 0);
-  TRY(pr->dgjobs.alloc(pr->gjobs.size()));
+  if (pr->gjobs.size() > pr->dgjobs.n) TRY(pr->dgjobs.alloc(pr->gjobs.size()));
   if (!pr->gjobs.empty())
     TRY(h2d(pr, pr->dgjobs.p, pr->gjobs.data(),
             sizeof(GemmJob) * pr->gjobs.size()));
@@ -949,6 +952,8 @@ static int tune_gemm(mpci_prop *pr, const GemmCand *only) {
   (void)hipEventDestroy(e1);
   TRY(rc);
   TRY(set_all_live(pr, 1));
+  TRY(pr->part.alloc(0));
+  TRY(pr->dgjobs.alloc(0));
   TRY(init_desc_kind(pr, bc.kind, bc.ks));
   TRY(build_gemm_jobs(pr, bc.kind, bc.wm, bc.wn, bc.fm, bc.fn, bc.tk, bc.ks));
   pr->gemm_ms = best;
