@@ -7,12 +7,13 @@ blocks L <-> L+1 of 4000 x 4000), velocity gauge, one sin^2 pulse of
 1e-10 from the lowest L = 0 level.  A step is one RKF78 attempt; `value`
 is accepted steps per second with all inputs resident in HBM.
 
-The timed region replays the captured step graph once per attempt (the
-production mode).  The same attempts are then run once more with a HIP
-event pair attached to each coupling-kernel dispatch on the propagator's
-stream (hipExtLaunchKernelGGL), which gives the average duration of the
-dominant kernel (k_gemv_tile) for the roofline figure (events do not time
-kernels inside graph replays).
+The timed region runs the attempts in the production mode, whole attempts
+in one cooperative launch (k_tiles_run).  The same attempts are then run
+once more launch by launch, with a HIP event pair attached to each
+coupling-kernel dispatch on the propagator's stream (hipExtLaunchKernelGGL),
+which gives the average duration of the coupling kernel (k_gemv_tile) for
+the roofline figure: what a sweep of all dipoles takes from HBM, most of
+which the persistent launch does too.
 
 Extra figures on the same line: the reference mode (fixed dt = 0.1, field
 frozen per step, as src/tdse/tdse.cpp:186-204), the batch of 64 pulses on
@@ -126,7 +127,7 @@ S_HE_TEST = [3030, 2799, 2808, 2808]  # inp/He_test.yaml states_in_l
 def run_he_test_shape(mpci, synth, attempts=300):
     """The block sizes of the reference's own He input (uneven, ragged
     against the GEMV units), synthetic E and D of that shape, the same
-    single pulse and tolerance as the headline: graph-replayed attempts,
+    single pulse and tolerance as the headline: attempts in the default form,
     then the same attempts instrumented for the coupling kernel's time."""
     E, D = synth.system_arrays(S_HE_TEST, seed=synth.HE_SEED + 7)
     sysg = mpci.System(E, D, gauge="v")
@@ -322,7 +323,7 @@ def run_c1(mpci, synth, c1):
         t += dt
     x0 = synth.ground_state(g.N)
     rates = {}
-    for mode in (-1, 0):  # the default (fused small-system path), the tiles
+    for mode in (-1, 0):  # the default (persistent row form), the tiles
         prop = make_prop(mpci, g)
         on = prop.set_small_path(mode)
         prop.set_state(x0)
@@ -336,7 +337,7 @@ def run_c1(mpci, synth, c1):
     return {"steps": steps,
             "steps_per_s": round(rates["small_path"], 1),
             "tile_path_steps_per_s": round(rates["tile_path"], 1),
-            "path": "fused small-system stage kernel (one launch per stage)",
+            "path": "persistent row form (whole attempts in one launch)",
             "bound": "launch/latency: 0.94 MB of dipoles stay in cache, so "
                      "no HBM roofline applies"}
 
