@@ -138,6 +138,7 @@ struct mpci_prop {
   int rows_kq = 1;       // quads per computing wave
   int wait_limit_ms = 0; // time limit of one wait inside the launch
   bool coop_refused = false;  // another process holds cooperative launching
+  bool persistent = false;    // the pending attempts are such a launch
   DevBuf<RowWg> rwg;
   // the same for larger systems (k_tiles_run)
   bool tiles = false;
@@ -1818,10 +1819,12 @@ static bool run_attempts_persistent(mpci_prop *pr) {
 }
 
 static int run_attempts(mpci_prop *pr, int n) {
+  pr->persistent = false;
   if (pr->instrument) return run_attempts_instrumented(pr, n);
   if ((pr->rows || pr->tiles) && pr->use_graph && !pr->store.xs &&
       !pr->store.xn && !pr->store.nrm && !pr->store.ckpt) {
-    if (run_attempts_persistent(pr)) return MPCI_OK;
+    pr->persistent = run_attempts_persistent(pr);
+    if (pr->persistent) return MPCI_OK;
     pr->rows = pr->tiles = false;
   }
   if (pr->use_graph) {
@@ -1835,7 +1838,10 @@ static int run_attempts(mpci_prop *pr, int n) {
 
 static int read_ctl(mpci_prop *pr, std::vector<Ctl> &c) {
   const int P = pr->P;
-  const bool persistent = pr->rows || pr->tiles;
+  // (the give-up flag of an earlier launch stays behind the records until
+  // the next one clears it)
+  const bool persistent = pr->persistent;
+  pr->persistent = false;
   c.resize(persistent ? 2 * P + 1 : P);
   HIPCHK(hipStreamSynchronize(pr->stream));
   TRY(d2h(pr, c.data(), pr->ctl.p, sizeof(Ctl) * c.size()));

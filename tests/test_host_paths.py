@@ -1,0 +1,61 @@
+"""The engine's host code on a runtime of host memory (no GPU): what it
+launches, keeps and gives back, and what it reads after a launch."""
+import pytest
+
+from host_runtime import host_runtime  # noqa: F401
+
+
+@pytest.mark.parametrize("s,P", [([60, 75, 33], 1), ([1777, 2401], 1),
+                                 ([60, 75, 33], 3)])
+def test_old_give_up_does_not_undo_later_runs(host_runtime, s, P):  # noqa
+    """A persistent launch that gave up leaves its flag on the device; with
+    the persistent forms switched on again, runs that go by launches
+    (eager, instrumented, the adjoint, grouped) keep what they computed."""
+    host_runtime(f"""
+    g, P = system({s}), {P}
+    p = mpci.Propagator(g, P=P)
+    x0 = np.arange(2.0 * g.N)
+    for i in range(P):
+        p.set_state(x0, i)
+        p.set_pulse(mpci.Pulse.pwl(np.full(4, 0.01), 0.7, 100.0), i)
+    F = np.full((P, 30), 0.02)
+    n = 0
+
+    def ran(k):
+        global n
+        n += k
+        for i in range(P):
+            assert np.array_equal(p.get_state(i), x0 + n), (n, i)
+
+    def adaptive(run):
+        st = run()
+        assert all(q.accepted == 8 and q.t == 2.0 for q in st)
+        ran(8)
+
+    p.set_wait_limit(-1)
+    p.prop_fixed(0.0, 0.1, F)
+    ran(30)
+    assert launches("k_apply") == 30  # it gave up
+    p.set_wait_limit(0)
+    p.set_small_path(-1)
+    p.set_graph(False)
+    p.prop_fixed(0.0, 0.1, F[:, :7])
+    ran(7)
+    one = lambda: p.prop_adaptive(0.0, 2.0, 0.25, 1e-9, 1e-9)[0]
+    adaptive(one)
+    p.set_graph(True)
+    p.set_instrument(True)
+    adaptive(one)
+    p.set_instrument(False)
+    W = np.ones(g.N)
+    assert p.adjoint(0.0, 2.0, 0.25, W)[2].tolist() == [8] * P
+    ran(8)
+    if P > 1:
+        p.set_graph(False)
+        adaptive(lambda: mpci.multi_adaptive([p], [0.0], [2.0], [0.25], 1e-9,
+                                             1e-9, grouped=True)[0])
+        p.set_graph(True)
+    rt.rt_clear()
+    adaptive(one)
+    assert launches("_run") == 1 and launches("k_apply") == 0
+    """)
