@@ -1070,6 +1070,11 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
       g.nlds = (int)std::min<long long>(std::max(nch - reg, 0),
                                         (room - base) / (nq * 2048LL));
       *lds = std::max<size_t>(*lds, base + g.nlds * nq * 2048LL);
+      // the kernel reads the second copy of the stage input a group of four
+      // chunks ahead of those it holds in registers
+      const int nchp = (nch + 3) / 4 * 4;
+      *lds = std::max<size_t>(
+          *lds, (nchp + std::min(nchp, reg) + 4LL) * 64 * sizeof(double2));
       wg.push_back(g);
     }
   }

@@ -520,7 +520,7 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
             if (q >= nq) continue;  // uniform over the wave
             double2 acc[4] = {};
             // every x is read a group of four chunks ahead (past the last
-            // group that stays inside the LDS buffer and is not used)
+            // group that is not used; the launch's LDS reaches there)
             double2 xn[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) xn[u] = xs[u * 64];

@@ -29,6 +29,7 @@ size_t fail_above = ~(size_t)0, alloc_us = 0;
 int abort_after = -1;                        // persistent launches give up
 std::vector<std::string> launched;
 std::vector<int> attempts;                   // of each persistent launch
+size_t lds = 0;                              // dynamic LDS of the last one
 long long stored = 0;                        // stages that kept their input
 struct Cost {
   std::string what;
@@ -131,10 +132,12 @@ hipError_t launch(const void *fn, void **args) {
   } else if (is("k_rows_run")) {
     const auto a = arg<RowRun>(args, 0);
     attempts.push_back(a.attempts);
+    lds = config.back().lds;
     f = [=] { persistent(a, a.P); };
   } else if (is("k_tiles_run")) {
     const auto a = arg<TileRun>(args, 0);
     attempts.push_back(a.attempts);
+    lds = config.back().lds;
     f = [=] { persistent(a, 1); };
   } else if (is("k_finalize_g") || is("k_apply_g")) {
     const auto m = arg<const GroupMember *>(args, 0);
@@ -230,6 +233,7 @@ int rt_attempts(int *out, int cap) {
   return (int)attempts.size();
 }
 long long rt_stored() { return stored; }
+size_t rt_lds() { return lds; }
 
 // ---- the runtime ----------------------------------------------------------
 void **__hipRegisterFatBinary(const void *) {

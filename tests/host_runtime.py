@@ -17,6 +17,7 @@ sys.path.insert(0, %r)
 rt = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
 rt.rt_fail_above.argtypes = rt.rt_alloc_us.argtypes = [ctypes.c_size_t]
 rt.rt_live_bytes.restype = rt.rt_live.restype = ctypes.c_size_t
+rt.rt_lds.restype = ctypes.c_size_t
 rt.rt_stored.restype = ctypes.c_longlong
 rt.rt_cost.argtypes = [ctypes.c_char_p, ctypes.c_double, ctypes.c_double,
                        ctypes.c_int]

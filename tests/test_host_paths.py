@@ -59,3 +59,26 @@ def test_old_give_up_does_not_undo_later_runs(host_runtime, s, P):  # noqa
     adaptive(one)
     assert launches("_run") == 1 and launches("k_apply") == 0
     """)
+
+
+def test_row_kernel_reads_ahead_inside_its_lds(host_runtime):  # noqa: F811
+    """k_rows_run reads the second copy of the neighbours' stage input one
+    group of four 64-row chunks of 16-byte elements ahead while it works on
+    chunks held in registers (16): its LDS has to reach there also where
+    little else follows the copies."""
+    host_runtime("""
+    for s, P in (([1, 1], 1), ([198] * 4, 1), ([300] * 6, 1), ([64, 65], 1),
+                 ([500, 500], 1), ([512, 512, 512], 1), ([513, 512, 512], 1),
+                 ([1, 1], 3), ([198] * 4, 5), ([1025, 30, 1100], 1)):
+        g = system(s)
+        p = mpci.Propagator(g, P=P)
+        p.prop_fixed(0.0, 0.1, np.full((P, 1), 0.02))
+        assert launches("k_rows_run") == 1
+        rt.rt_clear()
+        ch = lambda n: (n + 63) // 64
+        nch = [(ch(s[L - 1]) if L else 0) +
+               (ch(s[L + 1]) if L + 1 < len(s) else 0) for L in range(len(s))]
+        whole = [(n + 3) // 4 * 4 for n in nch]
+        last = max(w + min(w, 16) + 4 for w in whole)
+        assert rt.rt_lds() >= last * 64 * 16, (s, P, rt.rt_lds(), last)
+    """)
