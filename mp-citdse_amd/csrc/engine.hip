@@ -57,9 +57,10 @@ struct DevBuf {
       (void)hipFree(p);
       p = nullptr;
     }
-    n = count;
+    n = 0;  // until the memory is there
     if (count == 0) return MPCI_OK;
     HIPCHK(hipMalloc(&p, sizeof(T) * count));
+    n = count;
     return MPCI_OK;
   }
   void swap(DevBuf &o) {

@@ -82,3 +82,58 @@ def test_row_kernel_reads_ahead_inside_its_lds(host_runtime):  # noqa: F811
         last = max(w + min(w, 16) + 4 for w in whole)
         assert rt.rt_lds() >= last * 64 * 16, (s, P, rt.rt_lds(), last)
     """)
+
+
+REFUSED = """
+def refused(f, code=-2):
+    try:
+        f()
+    except mpci.MpciError as e:
+        assert e.code == code, e
+        return
+    assert False, "accepted"
+"""
+
+
+def test_tables_grow_again_after_a_failed_allocation(host_runtime):  # noqa
+    """A table that could not grow is allocated again by a smaller call."""
+    host_runtime(REFUSED + """
+g = system([60, 75, 33])
+p = mpci.Propagator(g)
+x0 = np.arange(2.0 * g.N)
+p.set_state(x0)
+huge = 1 << 18
+rt.rt_fail_above(1 << 20)
+refused(lambda: p.prop_fixed(0.0, 0.1, np.full((1, huge), 0.02)))
+refused(lambda: p.prop_schedule(0.0, np.full((1, huge), 0.1)))
+p.prop_fixed(0.0, 0.1, np.full((1, 5), 0.02))
+p.prop_schedule(0.0, np.full((1, 6), 0.1))
+assert np.array_equal(p.get_state(), x0 + 11)
+""")
+
+
+CANDIDATES = REFUSED + """
+g = system([300, 280, 310])
+p = mpci.Propagator(g, P=4)
+held = {}
+for k in range(p.gemm_candidates()):
+    p.set_gemm_candidate(k)
+    held[k] = rt.rt_live_bytes()
+big, small = max(held, key=held.get), min(held, key=held.get)
+mid = [k for k in held if held[small] < held[k] < held[big]][0]
+split = (300 + 2 * 280 + 310) * 4 * 16   # partials of one K split
+p.set_gemm_candidate(small)
+rt.rt_fail_above(split)
+refused(lambda: p.set_gemm_candidate(big))
+"""
+
+
+def test_tiles_after_one_that_did_not_fit(host_runtime):  # noqa: F811
+    """After a candidate tile whose buffers did not fit, a smaller one gets
+    its own (it was timed on no buffer at all)."""
+    host_runtime(CANDIDATES + """
+rt.rt_fail_above(1 << 40)
+p.set_gemm_candidate(mid)
+assert rt.rt_live_bytes() == held[mid]
+p.prop_fixed(0.0, 0.1, np.full((4, 2), 0.02))
+""")
