@@ -695,11 +695,20 @@ static int build_gemm_jobs(mpci_prop *pr, int kind, int wm, int wn, int fm,
   return MPCI_OK;
 }
 
+// A tile change that ran out of memory leaves neither its own nor the last
+// tile's buffers.
+static int have_tile(const mpci_prop *pr) {
+  if (pr->part.p && pr->dgjobs.p) return MPCI_OK;
+  return fail(MPCI_ERR_STATE, "no coupling buffers: the last tile change "
+                              "failed (set another one)");
+}
+
 // e0 / e1 (may be null): HIP events attached to the kernel's own dispatch,
 // so their interval is the kernel's execution alone.
 static int launch_gemm(mpci_prop *pr, const double2 *xin,
                        hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   mpci_system *sys = pr->sys;
+  TRY(have_tile(pr));
   const dim3 grid((unsigned)pr->gjobs.size());
   const double *X = reinterpret_cast<const double *>(xin);
   double *part = reinterpret_cast<double *>(pr->part.p);
@@ -2320,6 +2329,7 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
     if (pr->sys->device != props[0]->sys->device)
       return fail(MPCI_ERR_NOTSUP, "mpci_multi_adaptive_grouped: members on "
                                    "different devices");
+    TRY(have_tile(pr));
   }
   // members whose batch runs in one persistent launch run it, beside each
   // other, and the group is made of the others

@@ -137,3 +137,19 @@ p.set_gemm_candidate(mid)
 assert rt.rt_live_bytes() == held[mid]
 p.prop_fixed(0.0, 0.1, np.full((4, 2), 0.02))
 """)
+
+
+def test_no_launch_without_coupling_buffers(host_runtime):  # noqa: F811
+    """A propagator left without its coupling buffers by a tile that did not
+    fit refuses to run until it has a tile again."""
+    host_runtime(CANDIDATES + """
+rt.rt_clear()
+refused(lambda: p.prop_fixed(0.0, 0.1, np.full((4, 2), 0.02)), -3)
+refused(lambda: p.rhs(0.02, np.ones(8 * g.N)), -3)
+refused(lambda: mpci.multi_adaptive([p], [0.0], [2.0], [0.25], 1e-9, 1e-9,
+                                    grouped=True), -3)
+assert launches("k_gemm") == launches("7k_stage") == launches("k_apply") == 0
+p.set_gemm_candidate(small)
+p.prop_fixed(0.0, 0.1, np.full((4, 2), 0.02))
+p.rhs(0.02, np.ones(8 * g.N))
+""")
