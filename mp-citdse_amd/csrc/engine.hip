@@ -2331,6 +2331,12 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
                                    "different devices");
     TRY(have_tile(pr));
   }
+  for (int i = 0; i < n; ++i) {  // every argument, before any member runs
+    std::vector<Ctl> c;
+    std::vector<std::vector<LogEnt>> acc;
+    TRY(setup_adaptive(props[i], t0[i], t1[i], h0[i], atol, rtol,
+                       max_attempts, 0, c, acc));
+  }
   // members whose batch runs in one persistent launch run it, beside each
   // other, and the group is made of the others
   std::vector<int> alone, rest;

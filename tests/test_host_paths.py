@@ -153,3 +153,32 @@ p.set_gemm_candidate(small)
 p.prop_fixed(0.0, 0.1, np.full((4, 2), 0.02))
 p.rhs(0.02, np.ones(8 * g.N))
 """)
+
+
+@pytest.mark.parametrize("grouped", [True, False])
+def test_bad_argument_of_one_member_runs_none(host_runtime, grouped):  # noqa
+    """An argument error of any member is found before a member runs, also
+    where some run in persistent launches and the others grouped."""
+    host_runtime(REFUSED + f"""
+ps, xs = [], []
+for i, s in enumerate(([60, 75, 33], [300, 280], [40, 41])):
+    p = mpci.Propagator(system(s), P=2)
+    if i == 1:
+        p.set_small_path(0)
+    x = np.arange(2.0 * sum(s))
+    for k in range(2):
+        p.set_state(x, k)
+    ps.append(p)
+    xs.append(x)
+for bad in range(3):
+    h = [0.25] * 3
+    h[bad] = 0.0
+    refused(lambda: mpci.multi_adaptive(ps, [0.0] * 3, [2.0] * 3, h, 1e-9,
+                                        1e-9, grouped={grouped}), -1)
+    for p, x in zip(ps, xs):
+        assert np.array_equal(p.get_state(0), x)
+mpci.multi_adaptive(ps, [0.0] * 3, [2.0] * 3, [0.25] * 3, 1e-9, 1e-9,
+                    grouped={grouped})
+for p, x in zip(ps, xs):
+    assert np.array_equal(p.get_state(1), x + 8)
+""")
