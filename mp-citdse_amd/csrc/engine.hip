@@ -175,6 +175,7 @@ struct mpci_prop {
   int gm_kind = 0, gm_wm = 2, gm_wn = 2, gm_fm = 2, gm_fn = 2, gm_tk = 32,
       gm_ks = 1;
   double gemm_ms = 0.0;  // autotuned time of one coupling evaluation
+  bool pinned = false;   // the tile was set (mpci_prop_set_gemm_candidate)
   std::vector<GemmJob> gjobs;
   DevBuf<GemmJob> dgjobs;
   // pes observable weights on the device (mpci_prop_observables)
@@ -1293,7 +1294,8 @@ static int apply_small_path(mpci_prop *pr, int mode) {
     rows = mode == 1 || (mode < 0 && row_groups(sys) <= sys->ncu);
     tiles = mode < 0 && !rows;
   }
-  if (pr->P > 1 && sys->nb > 1 && mode != 0) rows = rows_pay(pr);
+  if (pr->P > 1 && sys->nb > 1 && mode != 0 && !pr->pinned)
+    rows = rows_pay(pr);
   if (on || rows) {
     TRY(ensure_rows(sys));
     pr->nblk_small = sys->hrow.quad0[sys->nb];
@@ -3086,7 +3088,8 @@ extern "C" int mpci_prop_set_gemm_candidate(mpci_prop *pr, int index) {
   // are reallocated here
   HIPCHK(hipStreamSynchronize(pr->stream));
   drop_graph(pr);
-  if (pr->P > 1) pr->rows = false;  // the pinned tile is what runs
+  pr->pinned = true;  // the tile is what runs
+  pr->rows = false;
   return tune_gemm(pr, &kGemmCands[index]);
 }
 

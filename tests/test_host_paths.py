@@ -182,3 +182,21 @@ mpci.multi_adaptive(ps, [0.0] * 3, [2.0] * 3, [0.25] * 3, 1e-9, 1e-9,
 for p, x in zip(ps, xs):
     assert np.array_equal(p.get_state(1), x + 8)
 """)
+
+
+def test_pinned_tile_stays(host_runtime):  # noqa: F811
+    """A pinned tile is what a batch runs, also after the small-system path
+    has been chosen anew."""
+    host_runtime("""
+    g = system([60, 75, 33])
+    p = mpci.Propagator(g, P=5)
+    F = np.full((5, 4), 0.02)
+    p.prop_fixed(0.0, 0.1, F)
+    assert launches("k_rows_run") == 1
+    p.set_gemm_candidate(2)
+    for mode in (-1, 1, 0):
+        p.set_small_path(mode)
+        rt.rt_clear()
+        p.prop_fixed(0.0, 0.1, F)
+        assert launches("k_rows_run") == 0 and launches("k_gemm") == 4 * 13
+    """)
