@@ -115,6 +115,9 @@ struct mpci_system {
     double ms;
   };
   std::map<int, Tuned> tuned;
+  // what propagators share and the first of them builds (Dr, Dq, tuned):
+  // several threads may create propagators of one system
+  std::mutex mu;
 };
 
 struct mpci_prop {
@@ -555,6 +558,7 @@ static int init_desc_kind(mpci_prop *pr, int kind, int ks) {
 // column, when there is one, holds zeros), so the batched kernels can load
 // 16-byte pairs from any even column.
 static int ensure_rowmajor(mpci_system *sys) {
+  std::lock_guard<std::mutex> lk(sys->mu);
   if (sys->Dr.p || sys->nb < 2) return MPCI_OK;
   std::vector<long long> off(sys->nb - 1);
   sys->dr_ld.assign(sys->nb - 1, 0);
@@ -588,6 +592,7 @@ static int row_chunks(const mpci_system *sys, int L) {
 
 // The row store (RowDesc), built on the device from the GEMV store.
 static int ensure_rows(mpci_system *sys) {
+  std::lock_guard<std::mutex> lk(sys->mu);
   if (sys->Dq.p || sys->nb < 2) return MPCI_OK;
   RowDesc r{};
   long long tot = 0;
@@ -979,6 +984,7 @@ static int tune_gemm(mpci_prop *pr, const GemmCand *only) {
 // and pulse count and keeps the fastest; later propagators of the same
 // system and pulse count reuse the choice.
 static int autotune_gemm(mpci_prop *pr) {
+  std::lock_guard<std::mutex> lk(pr->sys->mu);
   auto it = pr->sys->tuned.find(pr->P);
   if (it != pr->sys->tuned.end()) {
     const auto &t = it->second;

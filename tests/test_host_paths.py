@@ -200,3 +200,32 @@ def test_pinned_tile_stays(host_runtime):  # noqa: F811
         p.prop_fixed(0.0, 0.1, F)
         assert launches("k_rows_run") == 0 and launches("k_gemm") == 4 * 13
     """)
+
+
+@pytest.mark.parametrize("s,P,kernel", [([1201, 1333, 997], 1, "k_relayout_r"),
+                                        ([300, 280, 310], 40, "k_gemm_db")])
+def test_propagators_created_in_threads(host_runtime, s, P, kernel):  # noqa
+    """Several threads create propagators of one system: its row store is
+    built once, and its tile searched once, as one after the other."""
+    host_runtime(f"""
+    import threading
+    counts = []
+    for n in (1, 6):
+        g = system({s})
+        rt.rt_clear()
+        rt.rt_alloc_us(2000)
+        ps = [None] * n
+
+        def make(i):
+            ps[i] = mpci.Propagator(g, P={P})
+
+        ts = [threading.Thread(target=make, args=(i,)) for i in range(n)]
+        [t.start() for t in ts]
+        [t.join() for t in ts]
+        counts.append(launches("{kernel}"))
+        rt.rt_alloc_us(0)
+        [p.close() for p in ps]
+        g.close()
+        assert rt.rt_live() == 0
+    assert counts[0] == counts[1] > 0, counts
+    """)
