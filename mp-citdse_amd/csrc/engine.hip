@@ -590,11 +590,9 @@ static int row_chunks(const mpci_system *sys, int L) {
   return (n0 + 63) / 64 + (n1 + 63) / 64;
 }
 
-// The row store (RowDesc), built on the device from the GEMV store.
-static int ensure_rows(mpci_system *sys) {
-  std::lock_guard<std::mutex> lk(sys->mu);
-  if (sys->Dq.p || sys->nb < 2) return MPCI_OK;
-  RowDesc r{};
+// The layout of the row store; returns its size in doubles.
+static long long row_layout(const mpci_system *sys, RowDesc &r) {
+  r = RowDesc{};
   long long tot = 0;
   for (int L = 0; L < sys->nb; ++L) {
     const int nq = (sys->s[L] + kRwQuad - 1) / kRwQuad;
@@ -602,6 +600,15 @@ static int ensure_rows(mpci_system *sys) {
     r.quad0[L + 1] = r.quad0[L] + nq;
     tot += (long long)nq * row_chunks(sys, L) * 64 * kRwQuad;
   }
+  return tot;
+}
+
+// The row store (RowDesc), built on the device from the GEMV store.
+static int ensure_rows(mpci_system *sys) {
+  std::lock_guard<std::mutex> lk(sys->mu);
+  if (sys->Dq.p || sys->nb < 2) return MPCI_OK;
+  RowDesc r;
+  const long long tot = row_layout(sys, r);
   DevBuf<RowDesc> dr;
   DevBuf<double> q;
   TRY(dr.alloc(1));
@@ -1071,6 +1078,8 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
   const int rmax = *std::max_element(rpw.begin(), rpw.end());
   *kq = rmax <= 16 ? 1 : rmax <= 32 ? 2 : 4;
   const int reg = *kq == 1 ? kRwReg : 0;
+  RowDesc rd;
+  (void)row_layout(sys, rd);
   *lds = 0;
   for (int L = 0; L < sys->nb; ++L) {
     const int nch = row_chunks(sys, L);
@@ -1079,7 +1088,7 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
       g.L = L;
       g.row0 = r;
       g.nrows = std::min(rpw[L], sys->s[L] - r);
-      g.quad0 = sys->hrow.quad0[L] + r / kRwQuad;
+      g.quad0 = rd.quad0[L] + r / kRwQuad;
       const int nq = (g.nrows + kRwQuad - 1) / kRwQuad;
       const long long base = 2LL * ((nch + 3) / 4 * 4) * 64 * 16 +
                              nslot * (kStages + 2LL) * nq * kRwQuad * 16;
@@ -1263,11 +1272,20 @@ static bool plan_tiles(const mpci_prop *pr, TilePlan &pl) {
   return true;
 }
 
+// The two persistent forms share the exchange buffers: each drops the other's
+// tables when it is set up, and all of it when it cannot be.
+static void drop_persistent(mpci_prop *pr) {
+  for (auto *b : {&pr->xb, &pr->pb, &pr->rb}) (void)b->alloc(0);
+  (void)pr->rwg.alloc(0);
+  (void)pr->twg.alloc(0);
+}
+
 static int setup_tiles(mpci_prop *pr, bool *ok) {
   TilePlan pl;
   *ok = plan_tiles(pr, pl);
   if (!*ok) return MPCI_OK;
   const int N = pr->sys->N, W = (int)pl.wg.size();
+  drop_persistent(pr);
   TRY(pr->xb.alloc(3 * (size_t)N));
   TRY(pr->pb.alloc(3 * (size_t)pl.desc.part_n));
   TRY(pr->rb.alloc(3 * (size_t)W));
@@ -1288,10 +1306,38 @@ static int setup_tiles(mpci_prop *pr, bool *ok) {
   return MPCI_OK;
 }
 
+// (the row store, which stays with the system, comes last)
+static int setup_rows(mpci_prop *pr, bool *ok) {
+  mpci_system *sys = pr->sys;
+  std::vector<RowWg> wg;
+  *ok = plan_rows(pr, 1, wg, &pr->rows_lds, &pr->rows_kq);
+  pr->rows_grp = pr->rows_slots = 1;
+  if (*ok && pr->P > 1) {
+    pr->rows_grp = std::min(pr->P, sys->ncu / (int)wg.size());
+    pr->rows_slots = std::min(
+        (pr->P + pr->rows_grp - 1) / pr->rows_grp, kRwSlots);
+    *ok = plan_rows(pr, pr->rows_slots, wg, &pr->rows_lds, &pr->rows_kq);
+  }
+  if (!*ok) return MPCI_OK;
+  const size_t ns = (size_t)pr->rows_grp * pr->rows_slots;
+  RowDesc rd;
+  (void)row_layout(sys, rd);
+  drop_persistent(pr);
+  TRY(pr->xb.alloc(ns * 4 * sys->N));
+  TRY(pr->rb.alloc(ns * 3 * rd.quad0[sys->nb]));
+  TRY(pr->rwg.alloc(wg.size()));
+  TRY(h2d(pr, pr->rwg.p, wg.data(), sizeof(RowWg) * wg.size()));
+  TRY(ensure_rows(sys));
+  pr->rows_wg = (int)wg.size();
+  return MPCI_OK;
+}
+
 // The forms of one pulse on more than one block: fused stages from the row
 // store (small), and the persistent launches (rows, tiles).  mode -1:
 // automatic; 0: none of them; 1: the row store wherever it applies.  A batch
-// has the persistent row form, where it pays, unless mode is 0.
+// has the persistent row form, where it pays, unless mode is 0 or its tile
+// was pinned.  A form whose buffers do not fit is left out: the launches of
+// single stages need none of them.
 static int apply_small_path(mpci_prop *pr, int mode) {
   mpci_system *sys = pr->sys;
   bool on = false, rows = false, tiles = false;
@@ -1302,33 +1348,18 @@ static int apply_small_path(mpci_prop *pr, int mode) {
   }
   if (pr->P > 1 && sys->nb > 1 && mode != 0 && !pr->pinned)
     rows = rows_pay(pr);
-  if (on || rows) {
-    TRY(ensure_rows(sys));
+  auto fits = [](int rc) {
+    if (rc != MPCI_OK) (void)hipGetLastError();
+    return rc == MPCI_OK;
+  };
+  if (on) {
+    on = fits(ensure_rows(sys)) && (pr->Xs2.p || fits(pr->Xs2.alloc(pr->NP)));
     pr->nblk_small = sys->hrow.quad0[sys->nb];
   }
-  if (on && !pr->Xs2.p) TRY(pr->Xs2.alloc(pr->NP));
-  if (rows && !pr->rwg.p) {
-    std::vector<RowWg> wg;
-    rows = plan_rows(pr, 1, wg, &pr->rows_lds, &pr->rows_kq);
-    pr->rows_grp = pr->rows_slots = 1;
-    if (rows && pr->P > 1) {
-      pr->rows_grp = std::min(pr->P, sys->ncu / (int)wg.size());
-      pr->rows_slots = std::min(
-          (pr->P + pr->rows_grp - 1) / pr->rows_grp, kRwSlots);
-      rows = plan_rows(pr, pr->rows_slots, wg, &pr->rows_lds, &pr->rows_kq);
-    }
-    if (rows) {
-      const size_t ns = (size_t)pr->rows_slots;
-      TRY(pr->xb.alloc((size_t)pr->rows_grp * ns * 4 * sys->N));
-      TRY(pr->rb.alloc((size_t)pr->rows_grp * ns * 3 * sys->hrow.quad0[sys->nb]));
-      DevBuf<RowWg> d;
-      TRY(d.alloc(wg.size()));
-      TRY(h2d(pr, d.p, wg.data(), sizeof(RowWg) * wg.size()));
-      pr->rwg.swap(d);
-      pr->rows_wg = (int)wg.size();
-    }
-  }
-  if (tiles && !pr->twg.p) TRY(setup_tiles(pr, &tiles));
+  bool ok = true;
+  if (rows && !pr->rwg.p) rows = fits(setup_rows(pr, &ok)) && ok;
+  if (tiles && !pr->twg.p) tiles = fits(setup_tiles(pr, &ok)) && ok;
+  if (!rows && !tiles && mode != 0) drop_persistent(pr);
   pr->small = on;
   pr->rows = rows;
   pr->tiles = tiles;

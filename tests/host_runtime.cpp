@@ -25,7 +25,7 @@ namespace {
 std::recursive_mutex mu;
 std::map<const void *, std::string> names;   // kernel stubs
 std::map<void *, size_t> live;               // allocations
-size_t fail_above = ~(size_t)0, alloc_us = 0;
+size_t fail_above = ~(size_t)0, fail_from = 1, fail_to = 0, alloc_us = 0;
 int abort_after = -1;                        // persistent launches give up
 std::vector<std::string> launched;
 std::vector<int> attempts;                   // of each persistent launch
@@ -206,6 +206,10 @@ hipError_t launch(const void *fn, void **args) {
 extern "C" {
 // ---- controls for the tests ---------------------------------------------
 void rt_fail_above(size_t bytes) { fail_above = bytes; }
+void rt_fail_at(size_t from, size_t to) {
+  fail_from = from;
+  fail_to = to;
+}
 void rt_alloc_us(size_t us) { alloc_us = us; }
 void rt_abort_after(int n) { abort_after = n; }
 size_t rt_live() { return live.size(); }
@@ -283,7 +287,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     std::this_thread::sleep_for(std::chrono::microseconds(alloc_us));
   std::lock_guard<std::recursive_mutex> lk(mu);
   *p = nullptr;
-  if (n > fail_above) return hipErrorOutOfMemory;
+  if (n > fail_above || (n >= fail_from && n <= fail_to)) return hipErrorOutOfMemory;
   *p = std::calloc(n, 1);
   live[*p] = n;
   return hipSuccess;

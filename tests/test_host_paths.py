@@ -229,3 +229,50 @@ def test_propagators_created_in_threads(host_runtime, s, P, kernel):  # noqa
         assert rt.rt_live() == 0
     assert counts[0] == counts[1] > 0, counts
     """)
+
+
+@pytest.mark.parametrize("s,P,first", [
+    ([198] * 4, 1, "row store"), ([1201, 1333, 997], 1, "row store"),
+    ([1201, 1333, 997], 1, "exchange"), ([1777, 2401], 1, "exchange"),
+    ([300, 280, 310], 5, "row store"), ([300, 280, 310], 5, "exchange")])
+def test_persistent_form_without_room(host_runtime, s, P, first):  # noqa
+    """Where the row store or the exchange buffers do not fit, a propagator
+    is created all the same, runs by launches and holds nothing of the form;
+    it has the form when it is asked for again and there is room."""
+    n16 = sum(-(-n // 16) for n in s)
+    ch = [-(-n // 64) for n in s]
+    store = 4 * 64 * 8 * sum(
+        -(-n // 4) * (sum(ch[max(L - 1, 0):L]) + sum(ch[L + 1:L + 2]))
+        for L, n in enumerate(s))
+    groups = min(P, max(256 // n16, 1))
+    copies = 3 if n16 > 256 else 4 * groups * -(-P // groups)
+    size = store if first == "row store" else 16 * sum(s) * copies
+    host_runtime(f"""
+    s, P = {s}, {P}
+    F, x0 = np.full((P, 2), 0.02), np.arange(2.0 * sum(s))
+
+    def run(p, persistent):
+        p.set_state(x0)
+        rt.rt_clear()
+        p.prop_fixed(0.0, 0.1, F)
+        assert np.array_equal(p.get_state(), x0 + 2)
+        assert launches("_run") == persistent
+        assert launches("k_apply") == (0 if persistent else 2)
+        return rt.rt_live_bytes()
+
+    rt.rt_fail_at.argtypes = [ctypes.c_size_t] * 2
+    g = system(s)
+    p = mpci.Propagator(g, P=P)
+    held = run(p, True)
+    p.close(), g.close()
+    rt.rt_fail_at({size}, {size})
+    g = system(s)
+    p = mpci.Propagator(g, P=P)
+    assert run(p, False) <= held - {size if n16 > 256 else store}
+    p.rhs(0.02, np.ones(2 * g.N * P))
+    rt.rt_fail_at(1, 0)
+    p.set_small_path(-1)
+    assert run(p, True) == held
+    p.close(), g.close()
+    assert rt.rt_live() == 0
+    """)
