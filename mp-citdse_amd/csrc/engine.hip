@@ -1773,11 +1773,26 @@ static int run_attempts_instrumented(mpci_prop *pr, int n) {
   return MPCI_OK;
 }
 
-// Attempts until the pulse has finished (or the log is full) in one
+// Attempts of one persistent launch.  It holds the compute units it runs on,
+// so that the work of other propagators, streams and processes waits for its
+// end: about 100 ms, 20 ms beside other members of a multi run.  A launch of
+// its own costs about 0.1 ms.  An attempt is taken for 13 sweeps of the dipoles at
+// 5.5 TB/s, 100 us at least (a row form's is 28 to 120 us for the pulses that
+// it holds at a time, however many these are).
+static int persistent_attempts(const mpci_prop *pr, bool shared) {
+  const double us = std::max(100.0, pr->rows ? 0.0 : 13 * 8e-6 / 5.5 *
+                                                         (double)pr->sys->S);
+  const int held = pr->rows_grp * pr->rows_slots;
+  const int passes = pr->rows ? (pr->P + held - 1) / held : 1;
+  const double n = (shared ? 20e3 : 100e3) / (us * passes);
+  return std::min(pr->logcap, std::max(16, (int)n));
+}
+
+// Attempts until the pulse has finished, `attempts` of them at most, in one
 // cooperative launch (k_rows_run, k_tiles_run); read_ctl undoes and switches
 // off a launch that gave up.  Returns false when the device does not take
 // the launch.
-static bool run_attempts_persistent(mpci_prop *pr) {
+static bool run_attempts_persistent(mpci_prop *pr, int attempts) {
   mpci_system *sys = pr->sys;
   const int nxb = pr->rows ? (int)pr->xb.n : 3 * sys->N;
   const int npb = pr->rows ? 0 : 3 * pr->tiles_part;
@@ -1805,7 +1820,7 @@ static bool run_attempts_persistent(mpci_prop *pr) {
     a.logcap = pr->logcap;
     a.track = pr->track;
     a.N = sys->N;
-    a.attempts = pr->logcap;
+    a.attempts = attempts;
     a.limit_ms = pr->wait_limit_ms;
     a.arrived = arrived;
     a.start_ms = pr->coop_refused ? kStartLimitMs : 0;
@@ -1872,12 +1887,15 @@ static bool run_attempts_persistent(mpci_prop *pr) {
   return false;
 }
 
-static int run_attempts(mpci_prop *pr, int n) {
+// n attempts as launches of their own, or a persistent launch; shared: others
+// run beside it.
+static int run_attempts(mpci_prop *pr, int n, bool shared = false) {
   pr->persistent = false;
   if (pr->instrument) return run_attempts_instrumented(pr, n);
   if ((pr->rows || pr->tiles) && pr->use_graph && !pr->store.xs &&
       !pr->store.xn && !pr->store.nrm && !pr->store.ckpt) {
-    pr->persistent = run_attempts_persistent(pr);
+    pr->persistent =
+        run_attempts_persistent(pr, persistent_attempts(pr, shared));
     if (pr->persistent) return MPCI_OK;
     pr->rows = pr->tiles = false;
   }
@@ -2236,8 +2254,11 @@ extern "C" int mpci_prop_adaptive(mpci_prop *pr, const double *t0,
 // Several propagators (instances: different systems, different P) stepped
 // concurrently.  Each member runs on its own stream; whenever a member's
 // chunk has drained, its log is collected and its next chunk is enqueued at
-// once, so a small instance never waits for a large one and the device
-// always has the work of every unfinished member queued.
+// once, so the device always has the work of every unfinished member queued.
+// Chunks of single launches overlap with the other members' work; a
+// persistent launch takes the device for itself, so it is kept short
+// (persistent_attempts): a small instance waits for the others' launches, not
+// for their runs.
 extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
                                    const double *const *t0,
                                    const double *const *t1,
@@ -2268,7 +2289,8 @@ extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
     TRY(start_ctl(props[i], m[i].c));
   }
   for (;;) {
-    int live = 0;
+    int live = 0, unfinished = 0;
+    for (auto &x : m) unfinished += !x.finished;
     for (auto &x : m) {
       if (x.finished || x.busy) {
         live += !x.finished;
@@ -2279,7 +2301,7 @@ extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
         x.finished = true;
         continue;
       }
-      TRY(run_attempts(x.pr, k));
+      TRY(run_attempts(x.pr, k, unfinished > 1));
       x.busy = true;
       ++live;
     }

@@ -276,3 +276,42 @@ def test_persistent_form_without_room(host_runtime, s, P, first):  # noqa
     p.close(), g.close()
     assert rt.rt_live() == 0
     """)
+
+
+def test_persistent_launches_are_bounded(host_runtime):  # noqa: F811
+    """A persistent launch holds the device, so it takes a stated time at
+    most: by the time of its attempts 100 ms alone, 20 ms beside others (a
+    row attempt at least 30 us and a pass, a tile attempt at least 13 sweeps
+    of the dipoles at 7 TB/s)."""
+    host_runtime("""
+    def run(members, together):
+        ps = []
+        for s, P in members:
+            p = mpci.Propagator(system(s), P=P)
+            p.set_state(np.zeros(2 * sum(s)))
+            ps.append(p)
+        rt.rt_clear()
+        for q in [ps] if together else [[p] for p in ps]:
+            n = len(q)
+            st = mpci.multi_adaptive(q, [0.0] * n, [1024.0] * n, [0.25] * n,
+                                     1e-9, 1e-9)
+            assert all(x[0].accepted == 4096 for x in st)
+        a = attempts()
+        for p in ps:
+            assert np.array_equal(p.get_state(), np.full(2 * p.sys.N, 4096.0))
+        assert sum(a) >= 4096 * len(members)
+        return a
+
+    small, tiles, batch = ([198] * 4, 1), ([1500] * 4, 1), ([60] * 8, 5)
+    one = 13 * 8 * 3 * 1500 ** 2 / 7e6  # us
+    assert max(run([small], False)) * 30.0 <= 100e3
+    assert max(run([tiles], False)) * one <= 100e3
+    a = run([small, batch], True)
+    assert max(a) * 30.0 <= 20e3 and min(a) >= 16
+    a = run([tiles, small], True)
+    assert min(a) * one <= 20e3 and min(a) >= 16
+    p = mpci.Propagator(system([1500] * 4))
+    rt.rt_clear()
+    p.prop_fixed(0.0, 0.1, np.full((1, 4500), 0.02))
+    assert max(attempts()) * one <= 100e3
+    """)
