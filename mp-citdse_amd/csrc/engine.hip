@@ -2697,8 +2697,14 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
   // What the sweep needs of a segment's K steps.  The forward pass keeps it
   // too, so the steps of the last segment are not propagated again (all of
   // them, for a run of up to K steps: 16 pulses on 4000 x 4, 7 steps, 44.5 ->
-  // 31.7 ms); without room for it beside the checkpoints they are.
-  bool kept = false;
+  // 31.7 ms); without room for it beside the checkpoints they are.  Keeping
+  // a step's stage inputs costs 5 % of its time there, and which segment is the
+  // last is not known: the forward pass keeps the first K steps and those
+  // from where at most kKeepSegments segments' steps seem to be left.
+  constexpr int kKeepSegments = 4;
+  bool kept = false;       // the buffers are there
+  bool keeping = false;    // the steps of the coming chunk go to them
+  std::vector<int> since(P, 0);  // steps of each pulse from which it does
   auto alloc_segment = [&]() -> int {
     TRY(xs_store.alloc((size_t)K * (kStages - 1) * NP));
     TRY(xn_store.alloc((size_t)(K + 1) * NP));
@@ -2770,11 +2776,7 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
   pr->store.cap = K;
   TRY(grow_ckpt(2));
   kept = alloc_segment() == MPCI_OK;
-  if (kept) {
-    pr->store.xs = xs_store.p;
-    pr->store.xn = xn_store.p;
-    pr->store.nrm = nrm_store.p;
-  } else {
+  if (!kept) {
     (void)hipGetLastError();
     drop_segment();
   }
@@ -2791,7 +2793,20 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
     if (done_max > max_steps)
       return fail(MPCI_ERR_LIMIT, "adjoint forward took more than max_steps "
                                   "accepted steps");
+    double left = 0.0;  // steps still expected
+    for (const Ctl &x : c)
+      if (!x.done)
+        left = std::max(left, (x.t_end - x.t) / std::max(x.h, 1e-300));
+    const bool end = left <= (double)kKeepSegments * K;
     TRY(grow_ckpt((done_max + n) / K + 2));
+    if (done_max < K && !end) n = std::min(n, K - done_max);
+    const bool keep = kept && (done_max < K || end);
+    if (keep && !keeping)
+      for (int p = 0; p < P; ++p) since[p] = c[p].accepted;
+    keeping = keep;
+    pr->store.xs = keep ? xs_store.p : nullptr;
+    pr->store.xn = keep ? xn_store.p : nullptr;
+    pr->store.nrm = keep ? nrm_store.p : nullptr;
     TRY(run_attempts(pr, n));
     TRY(read_ctl(pr, c));
     TRY(drain_log(pr, c, acc));
@@ -2857,6 +2872,10 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
     for (int k = 0; k < grad_stride; ++k) grad[(size_t)p * grad_stride + k] = 0;
 
   const int nseg = (nmax + K - 1) / K;
+  // whether the forward pass kept all steps of the last segment
+  bool last_kept = keeping;
+  for (int p = 0; p < P; ++p)
+    if (nst[p] > (nseg - 1) * K && since[p] > (nseg - 1) * K) last_kept = false;
   std::vector<double> hs((size_t)P * K), tn((size_t)K * P), hn((size_t)K * P),
       g((size_t)K * kStages * P), ts(P);
   std::vector<int> nloc(P);
@@ -2869,7 +2888,7 @@ extern "C" int mpci_prop_adjoint(mpci_prop *pr, const double *t0,
     if (kmax == 0) continue;
     // recompute the segment from checkpoint j, storing what the sweep needs
     // (the last one's is there from the forward pass)
-    const bool stored = kept && j == nseg - 1;
+    const bool stored = last_kept && j == nseg - 1;
     HIPCHK(hipMemcpyAsync(xn_store.p, ckpt.p + (size_t)j * NP,
                           sizeof(double2) * NP, hipMemcpyDeviceToDevice,
                           pr->stream));

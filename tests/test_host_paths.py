@@ -315,3 +315,28 @@ def test_persistent_launches_are_bounded(host_runtime):  # noqa: F811
     p.prop_fixed(0.0, 0.1, np.full((1, 4500), 0.02))
     assert max(attempts()) * one <= 100e3
     """)
+
+
+@pytest.mark.parametrize("s,P", [([60, 75, 33], 1), ([30, 20], 3)])
+@pytest.mark.parametrize("steps,K", [(1000, 32), (1000, 8), (992, 32),
+                                     (20, 32), (32, 32), (33, 32), (5, 1)])
+def test_adjoint_keeps_little_more_than_it_uses(host_runtime, s, P, steps, K):  # noqa
+    """The adjoint's forward pass keeps the stage inputs of its last segment,
+    and of few steps besides: the first segment's (a short run has no other)
+    and those of the last four segments.  The last segment is not propagated
+    again."""
+    host_runtime(f"""
+    g, P, steps, K = system({s}), {P}, {steps}, {K}
+    p = mpci.Propagator(g, P=P)
+    for i in range(P):
+        p.set_state(np.arange(2.0 * g.N), i)
+        p.set_pulse(mpci.Pulse.pwl(np.full(4, 0.01), 0.7, 2000.0), i)
+    nst, st = p.adjoint(0.0, 0.25 * steps, 0.25, np.ones(g.N),
+                        ckpt_every=K)[2::2]
+    assert nst.tolist() == [steps] * P
+    again = (steps - 1) // K * K   # all but the last segment
+    kept = rt.rt_stored() - 13 * again
+    assert kept % 13 == 0 and steps - again <= kept // 13 <= 6 * K, kept
+    if steps <= K:
+        assert kept == 13 * steps
+    """)
