@@ -899,16 +899,21 @@ static int time_gemm_cand(mpci_prop *pr, const GemmCand &cd, hipEvent_t e0,
     a.xs_store = nullptr;  // leave any adjoint stage store alone
     return launch_stage(pr, a);
   };
-  // two warm evaluations, then the twelve stages timed unless the second is
-  // three times slower than the best so far
+  // two warm evaluations, then the twelve stages timed unless the second and,
+  // as other work may have slowed it, a third are three times slower than the
+  // best so far
   constexpr int kReps = kStages - 1;
   TRY(eval(0));
-  HIPCHK(hipEventRecord(e0, pr->stream));
-  TRY(eval(1));
-  HIPCHK(hipEventRecord(e1, pr->stream));
-  HIPCHK(hipEventSynchronize(e1));
-  HIPCHK(hipEventElapsedTime(ms, e0, e1));
-  if (*ms > 3.f * best + 0.02f) return MPCI_OK;
+  bool slow = true;
+  for (int look = 0; slow && look < 2; ++look) {
+    HIPCHK(hipEventRecord(e0, pr->stream));
+    TRY(eval(1));
+    HIPCHK(hipEventRecord(e1, pr->stream));
+    HIPCHK(hipEventSynchronize(e1));
+    HIPCHK(hipEventElapsedTime(ms, e0, e1));
+    slow = *ms > 3.f * best + 0.02f;
+  }
+  if (slow) return MPCI_OK;
   HIPCHK(hipEventRecord(e0, pr->stream));
   for (int s = 0; s < kReps; ++s) TRY(eval(s));
   HIPCHK(hipEventRecord(e1, pr->stream));

@@ -340,3 +340,24 @@ def test_adjoint_keeps_little_more_than_it_uses(host_runtime, s, P, steps, K):  
     if steps <= K:
         assert kept == 13 * steps
     """)
+
+
+def test_one_slow_launch_does_not_drop_a_tile(host_runtime):  # noqa: F811
+    """The tile search leaves a candidate after a slow evaluation only when a
+    second one is slow as well."""
+    host_runtime("""
+    g = system([300, 280, 310])
+    # k_gemm_lds of 4 x 1 waves and 2 x 1 blocks: the fastest, but slow once
+    rt.rt_cost(b"k_gemm", 100.0, 100.0, 0)
+    rt.rt_cost(b"k_gemm_ldsILi4ELi1ELi2ELi1E", 1.0, 1e5, 2)
+    c = mpci.Propagator(g, P=40).gemm_config()
+    assert (c["kernel"], c["wm"], c["wn"], c["fm"], c["fn"]) == (
+        "k_gemm_lds", 4, 1, 2, 1), c
+    assert c["ms"] < 0.02
+    # always slow ones are left after two looks
+    rt.rt_cost(b"k_gemm_pair", 1e5, 1e5, 0)
+    rt.rt_clear()
+    g = system([300, 280, 310])
+    assert mpci.Propagator(g, P=40).gemm_config() == c
+    assert launches("k_gemm_pair") == 2 * 3
+    """)
