@@ -735,10 +735,11 @@ static int launch_gemm(mpci_prop *pr, const double2 *xin,
                         pr->dgjobs.p, sys->Dr.p, sys->dr_off.p, X, part,    \
                         pr->ddesc.p, pr->ctl.p)
 #define MPCI_GEMM_LDS(WM, WN, FM, FN)                                        \
-  hipExtLaunchKernelGGL((k_gemm_lds<WM, WN, FM, FN>), grid,                  \
-                        dim3(64 * WM * WN), 0,                               \
-                        pr->stream, e0, e1, 0, pr->dgjobs.p, sys->Dr.p,      \
-                        sys->dr_off.p, X, part, pr->ddesc.p, pr->ctl.p)
+  if (wm == WM && wn == WN && pr->gm_fm == FM && pr->gm_fn == FN)            \
+    hipExtLaunchKernelGGL((k_gemm_lds<WM, WN, FM, FN>), grid,                \
+                          dim3(64 * WM * WN), 0, pr->stream, e0, e1, 0,      \
+                          pr->dgjobs.p, sys->Dr.p, sys->dr_off.p, X, part,   \
+                          pr->ddesc.p, pr->ctl.p);
   const int wm = pr->gm_wm, wn = pr->gm_wn, tk = pr->gm_tk;
   const int f = pr->gm_fm * 10 + pr->gm_fn;
   if (pr->gm_kind == 3) {
@@ -746,32 +747,7 @@ static int launch_gemm(mpci_prop *pr, const double2 *xin,
                           0, pr->dgjobs.p, sys->Dr.p, sys->dr_off.p, X, part,
                           pr->ddesc.p, pr->ctl.p);
   } else if (pr->gm_kind == 2) {
-    const int w = wm * 10 + wn;
-    if (f == 11) {
-      if (w == 22)
-        MPCI_GEMM_LDS(2, 2, 1, 1);
-      else if (w == 42)
-        MPCI_GEMM_LDS(4, 2, 1, 1);
-      else
-        MPCI_GEMM_LDS(4, 1, 1, 1);
-    } else if (f == 21) {
-      if (w == 22)
-        MPCI_GEMM_LDS(2, 2, 2, 1);
-      else
-        MPCI_GEMM_LDS(4, 1, 2, 1);
-    } else if (w == 21) {
-      MPCI_GEMM_LDS(2, 1, 2, 2);
-    } else if (w == 41) {
-      MPCI_GEMM_LDS(4, 1, 2, 2);
-    } else if (w == 22) {
-      MPCI_GEMM_LDS(2, 2, 2, 2);
-    } else if (w == 42) {
-      MPCI_GEMM_LDS(4, 2, 2, 2);
-    } else if (w == 24) {
-      MPCI_GEMM_LDS(2, 4, 2, 2);
-    } else {
-      MPCI_GEMM_LDS(4, 4, 2, 2);
-    }
+    MPCI_LDS_TILES(MPCI_GEMM_LDS)
   } else if (pr->gm_kind == 0) {
     if (wm == 2 && wn == 2)
       MPCI_GEMM(2, 2);
@@ -2346,23 +2322,14 @@ extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
 // The attempt is captured once into a graph on the first member's stream.
 // ---------------------------------------------------------------------
 namespace {
-int launch_gemm_group(hipStream_t st, int wm, int wn, unsigned njobs,
-                      const GemmJob *jobs, const GroupGemm &m, int s) {
-#define MPCI_GEMM_G(WM, WN)                                                  \
-  hipLaunchKernelGGL((k_gemm_lds_g<WM, WN>), dim3(njobs), dim3(64 * WM * WN), \
-                     0, st, jobs, m, s)
-  if (wm == 2 && wn == 1)
-    MPCI_GEMM_G(2, 1);
-  else if (wm == 4 && wn == 1)
-    MPCI_GEMM_G(4, 1);
-  else if (wm == 2 && wn == 2)
-    MPCI_GEMM_G(2, 2);
-  else if (wm == 4 && wn == 2)
-    MPCI_GEMM_G(4, 2);
-  else if (wm == 2 && wn == 4)
-    MPCI_GEMM_G(2, 4);
-  else
-    MPCI_GEMM_G(4, 4);
+int launch_gemm_group(hipStream_t st, int wm, int wn, int fm, int fn,
+                      unsigned njobs, const GemmJob *jobs, const GroupGemm &m,
+                      int s) {
+#define MPCI_GEMM_G(WM, WN, FM, FN)                                     \
+  if (wm == WM && wn == WN && fm == FM && fn == FN)                     \
+    hipLaunchKernelGGL((k_gemm_lds_g<WM, WN, FM, FN>), dim3(njobs),     \
+                       dim3(64 * WM * WN), 0, st, jobs, m, s);
+  MPCI_LDS_TILES(MPCI_GEMM_G)
 #undef MPCI_GEMM_G
   HIPCHK(hipGetLastError());
   return MPCI_OK;
@@ -2430,7 +2397,7 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
     return rc2 != MPCI_OK ? rc2 : rc;
   }
   // the group's tile: that of the member with the most coupling work when
-  // it is a direct-to-LDS tile, else 4 x 2 waves
+  // it is a direct-to-LDS tile, else 4 x 2 waves of 2 x 2 blocks
   int lead = 0;
   double most = -1.0;
   for (int i = 0; i < n; ++i) {
@@ -2440,10 +2407,12 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
       lead = i;
     }
   }
-  int wm = 4, wn = 2;
+  int wm = 4, wn = 2, fm = 2, fn = 2;
   if (props[lead]->gm_kind == 2) {
     wm = props[lead]->gm_wm;
     wn = props[lead]->gm_wn;
+    fm = props[lead]->gm_fm;
+    fn = props[lead]->gm_fn;
   }
   for (int i = 0; i < n; ++i) HIPCHK(hipStreamSynchronize(props[i]->stream));
   hipStream_t st = props[0]->stream;
@@ -2491,7 +2460,7 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
     // a member tuned to k_gemm_pair keeps its own launch (its sums run in
     // another order than the direct-to-LDS kernel's)
     if (pr->gm_kind == 3) continue;
-    jl[i] = gemm_job_list(pr, wm, wn, 2, 2, pr->gm_ks, i);
+    jl[i] = gemm_job_list(pr, wm, wn, fm, fn, pr->gm_ks, i);
     njobs += jl[i].size();
   }
   // shortest K range first: the short panels of small-block members run
@@ -2537,7 +2506,8 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
   HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   for (int s = 0; s < kStages && rc == MPCI_OK; ++s) {
     if (!jobs.empty())
-      rc = launch_gemm_group(st, wm, wn, (unsigned)jobs.size(), djobs.p, gg, s);
+      rc = launch_gemm_group(st, wm, wn, fm, fn, (unsigned)jobs.size(),
+                             djobs.p, gg, s);
     if (rc != MPCI_OK) break;
     for (int i = 0; i < n; ++i) {
       mpci_prop *pr = props[i];

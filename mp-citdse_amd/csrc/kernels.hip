@@ -838,36 +838,24 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((
 
 // Grouped form: one launch over the panels of several members (each job
 // names its member), every member's stage input X (stage 0) or Xs.
-template <int WM, int WN>
+template <int WM, int WN, int FM, int FN>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((
     amdgpu_waves_per_eu(WM * WN == 8 ? 6 : 1))) void k_gemm_lds_g(
     const GemmJob *__restrict__ jobs, GroupGemm g, int s) {
   const GemmJob jb = jobs[blockIdx.x];
   const int i = jb.member;
-  gemm_lds_panel<WM, WN, 2, 2>(jb, g.Dr[i], g.dr_off[i], s == 0 ? g.X[i] : g.Xs[i],
-                         g.part[i], *g.d[i], g.ctl[i]);
+  gemm_lds_panel<WM, WN, FM, FN>(jb, g.Dr[i], g.dr_off[i],
+                                 s == 0 ? g.X[i] : g.Xs[i], g.part[i],
+                                 *g.d[i], g.ctl[i]);
 }
 
 #define MPCI_GEMM_LDS(WM, WN, FM, FN)                                      \
   template __global__ void k_gemm_lds<WM, WN, FM, FN>(                    \
       const GemmJob *, const double *, const long long *, const double *, \
-      double *, const SysDesc *, const Ctl *);
-#define MPCI_GEMM_LDS_G(WM, WN)                                             \
-  MPCI_GEMM_LDS(WM, WN, 2, 2)                                               \
-  template __global__ void k_gemm_lds_g<WM, WN>(const GemmJob *, GroupGemm, \
-                                                int);
-MPCI_GEMM_LDS_G(2, 1)
-MPCI_GEMM_LDS_G(4, 1)
-MPCI_GEMM_LDS_G(2, 2)
-MPCI_GEMM_LDS_G(4, 2)
-MPCI_GEMM_LDS_G(2, 4)
-MPCI_GEMM_LDS_G(4, 4)
-MPCI_GEMM_LDS(2, 2, 1, 1)
-MPCI_GEMM_LDS(4, 2, 1, 1)
-MPCI_GEMM_LDS(2, 2, 2, 1)
-MPCI_GEMM_LDS(4, 1, 1, 1)
-MPCI_GEMM_LDS(4, 1, 2, 1)
-#undef MPCI_GEMM_LDS_G
+      double *, const SysDesc *, const Ctl *);                            \
+  template __global__ void k_gemm_lds_g<WM, WN, FM, FN>(const GemmJob *,  \
+                                                        GroupGemm, int);
+MPCI_LDS_TILES(MPCI_GEMM_LDS)
 #undef MPCI_GEMM_LDS
 
 // ---------------------------------------------------------------------

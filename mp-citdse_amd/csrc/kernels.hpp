@@ -148,7 +148,12 @@ template <int WM, int WN, int FM, int FN>
 __global__ void k_gemm_lds(const GemmJob *jobs, const double *Dr,
                            const long long *dr_off, const double *X,
                            double *part, const SysDesc *d, const Ctl *ctl);
-template <int WM, int WN>
+// its tiles: wm x wn waves, each fm x fn blocks of 16 x 16
+#define MPCI_LDS_TILES(T)                                                   \
+  T(2, 1, 2, 2) T(4, 1, 2, 2) T(2, 2, 2, 2) T(4, 2, 2, 2) T(2, 4, 2, 2)     \
+  T(4, 4, 2, 2) T(2, 2, 1, 1) T(4, 2, 1, 1) T(2, 2, 2, 1) T(4, 1, 1, 1)     \
+  T(4, 1, 2, 1)
+template <int WM, int WN, int FM, int FN>
 __global__ void k_gemm_lds_g(const GemmJob *jobs, GroupGemm g, int s);
 __global__ void k_gemm_pair(const GemmJob *jobs, const double *Dr,
                             const long long *dr_off, const double *X,

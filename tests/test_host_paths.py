@@ -361,3 +361,40 @@ def test_one_slow_launch_does_not_drop_a_tile(host_runtime):  # noqa: F811
     assert mpci.Propagator(g, P=40).gemm_config() == c
     assert launches("k_gemm_pair") == 2 * 3
     """)
+
+
+@pytest.mark.parametrize("wm,wn,fm,fn", [(2, 2, 1, 1), (4, 2, 1, 1),
+                                         (2, 2, 2, 1), (4, 1, 1, 1),
+                                         (4, 1, 2, 1), (4, 2, 2, 2)])
+def test_group_runs_the_tile_of_its_largest_member(host_runtime, wm, wn, fm,  # noqa
+                                                   fn):
+    """The grouped launches take the tile that was timed for the member with
+    the most coupling work, its blocks a wave as well as its waves."""
+    host_runtime(f"""
+    want = dict(kernel="k_gemm_lds", wm={wm}, wn={wn}, fm={fm}, fn={fn})
+    ps = [mpci.Propagator(system(s), P=20) for s in ([300, 280], [70, 60, 50])]
+    for k in range(ps[0].gemm_candidates()):
+        c = ps[0].set_gemm_candidate(k)
+        if all(c[q] == v for q, v in want.items()):
+            break
+    else:
+        assert False, "no such candidate"
+    ps[1].set_small_path(0)
+    rt.rt_clear()
+    mpci.multi_adaptive(ps, [0.0] * 2, [2.0] * 2, [0.25] * 2, 1e-9, 1e-9,
+                        grouped=True)
+    name = "k_gemm_lds_gILi{wm}ELi{wn}ELi{fm}ELi{fn}E"
+    assert launches(name) == launches("k_gemm") >= 8 * 13
+    assert launches("k_apply_g") >= 8 and launches("_run") == 0
+    """)
+
+
+def test_every_candidate_tile_is_launched(host_runtime):  # noqa: F811
+    host_runtime("""
+    p = mpci.Propagator(system([300, 280]), P=3)
+    for k in range(p.gemm_candidates()):
+        c = p.set_gemm_candidate(k)
+        rt.rt_clear()
+        p.prop_fixed(0.0, 0.1, np.full((3, 1), 0.02))
+        assert launches(c["kernel"]) == launches("k_gemm") == 13, c
+    """)
