@@ -1099,19 +1099,23 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
 // 149, P = 20 196 / 175; 800 x 5, P = 3 93 / 210, P = 5 164 / 218; 2000 x 2, P
 // = 2 103 / 261, P = 4 196 / 265, P = 5 275 / 264; 1500, 1000, 1500, P = 2
 // 175 / 234; 80 x 32, P = 5 92 / 144.
+static double row_pulse_us(const mpci_system *sys) {
+  int chunks = 0;
+  for (int L = 0; L < sys->nb; ++L)
+    chunks = std::max(chunks, row_chunks(sys, L));
+  const int c = std::max(chunks - kRwReg, 0);
+  return 20.0 + 1.2 * c + 0.045 * c * c;
+}
+
 static bool rows_pay(const mpci_prop *pr) {
   const mpci_system *sys = pr->sys;
   const int n16 = row_groups(sys);
-  int chunks = 0, smax = 0;
-  for (int L = 0; L < sys->nb; ++L) {
-    chunks = std::max(chunks, row_chunks(sys, L));
-    smax = std::max(smax, sys->s[L]);
-  }
+  int smax = 0;
+  for (int L = 0; L < sys->nb; ++L) smax = std::max(smax, sys->s[L]);
   if (n16 > sys->ncu) return false;
   const int groups = std::min(pr->P, sys->ncu / n16);
   const int each = (pr->P + groups - 1) / groups;
-  const int c = std::max(chunks - kRwReg, 0);
-  const double pulse = 20.0 + 1.2 * c + 0.045 * c * c;
+  const double pulse = row_pulse_us(sys);
   const double batched = 100.0 + 0.075 * std::min(smax, 1500) + 1.1 * sys->nb +
                          2e-6 * (double)sys->S * pr->P;
   return each * pulse < 0.97 * batched;
@@ -1773,40 +1777,66 @@ static int persistent_attempts(const mpci_prop *pr, bool shared) {
 // cooperative launch (k_rows_run, k_tiles_run); read_ctl undoes and switches
 // off a launch that gave up.  Returns false when the device does not take
 // the launch.
+static int *give_up_flag(mpci_prop *pr) { return &pr->ctl.p[2 * pr->P].status; }
+
+// What both persistent kernels are told of the propagator's run.
+template <class A>
+static void fill_run(mpci_prop *pr, int attempts, A &a) {
+  a.X = pr->X.p;
+  a.E = pr->sys->E.p;
+  a.xb = pr->xb.p;
+  a.rb = pr->rb.p;
+  a.ctl = pr->ctl.p;
+  a.abort_flag = give_up_flag(pr);
+  a.hs = pr->hs.p;
+  a.Ftab = pr->Ftab.p;
+  a.pulses = pr->pulses.p;
+  a.env = pr->env.p;
+  a.log = pr->log.p;
+  a.logcap = pr->logcap;
+  a.track = pr->track;
+  a.N = pr->sys->N;
+  a.attempts = attempts;
+  a.limit_ms = pr->wait_limit_ms;
+  a.arrived = &pr->ctl.p[2 * pr->P].nlog;
+  a.start_ms = pr->coop_refused ? kStartLimitMs : 0;
+}
+
+static RowRun row_run(mpci_prop *pr, int attempts) {
+  const mpci_system *sys = pr->sys;
+  RowRun a{};
+  fill_run(pr, attempts, a);
+  a.d = pr->ddesc.p;
+  a.rows = sys->drow.p;
+  a.Dq = sys->Dq.p;
+  a.wg = pr->rwg.p;
+  a.P = pr->P;
+  a.ngrp = pr->rows_grp;
+  a.nwg = pr->rows_wg;
+  a.nslot = pr->rows_slots;
+  a.nquad = sys->hrow.quad0[sys->nb];
+  return a;
+}
+
+// Before a persistent launch: the exchange buffers (nx, np, nr elements)
+// unset, the state and the control records saved.
+static bool begin_persistent(mpci_prop *pr, hipStream_t st, double2 *xb,
+                             int nx, double2 *pb, int np, double2 *rb, int nr) {
+  const int NP = (int)pr->NP;
+  const unsigned nb = (unsigned)((std::max({nx, np, nr, NP}) + 255) / 256);
+  hipLaunchKernelGGL(k_rows_begin, dim3(nb), dim3(256), 0, st, xb, nx, pb, np,
+                     rb, nr, pr->X.p, NP, pr->Y.p, pr->ctl.p, pr->P,
+                     give_up_flag(pr), &pr->ctl.p[2 * pr->P].nlog);
+  return hipGetLastError() == hipSuccess;
+}
+
 static bool run_attempts_persistent(mpci_prop *pr, int attempts) {
   mpci_system *sys = pr->sys;
-  const int nxb = pr->rows ? (int)pr->xb.n : 3 * sys->N;
-  const int npb = pr->rows ? 0 : 3 * pr->tiles_part;
-  const int nrb = pr->rows ? (int)pr->rb.n : 3 * pr->tiles_wg;
-  int *flag = &pr->ctl.p[2 * pr->P].status;
-  int *arrived = &pr->ctl.p[2 * pr->P].nlog;
-  const int NP = (int)pr->NP;
-  const unsigned nb = (unsigned)((std::max({nxb, npb, NP}) + 255) / 256);
-  hipLaunchKernelGGL(k_rows_begin, dim3(nb), dim3(256), 0, pr->stream,
-                     pr->xb.p, nxb, pr->pb.p, npb, pr->rb.p, nrb, pr->X.p,
-                     NP, pr->Y.p, pr->ctl.p, pr->P, flag, arrived);
-  if (hipGetLastError() != hipSuccess) return false;
-  auto common = [&](auto &a) {
-    a.X = pr->X.p;
-    a.E = sys->E.p;
-    a.xb = pr->xb.p;
-    a.rb = pr->rb.p;
-    a.ctl = pr->ctl.p;
-    a.abort_flag = flag;
-    a.hs = pr->hs.p;
-    a.Ftab = pr->Ftab.p;
-    a.pulses = pr->pulses.p;
-    a.env = pr->env.p;
-    a.log = pr->log.p;
-    a.logcap = pr->logcap;
-    a.track = pr->track;
-    a.N = sys->N;
-    a.attempts = attempts;
-    a.limit_ms = pr->wait_limit_ms;
-    a.arrived = arrived;
-    a.start_ms = pr->coop_refused ? kStartLimitMs : 0;
-  };
-  const SysDesc *d = pr->ddesc.p;
+  if (!begin_persistent(pr, pr->stream, pr->xb.p,
+                        pr->rows ? (int)pr->xb.n : 3 * sys->N, pr->pb.p,
+                        pr->rows ? 0 : 3 * pr->tiles_part, pr->rb.p,
+                        pr->rows ? (int)pr->rb.n : 3 * pr->tiles_wg))
+    return false;
   // A second process on the device is refused cooperative launches
   // (hipErrorIllegalState) for as long as the first holds them.  It launches
   // the ordinary way: on an idle device every workgroup is resident all the
@@ -1826,17 +1856,11 @@ static bool run_attempts_persistent(mpci_prop *pr, int attempts) {
   };
   hipError_t e;
   if (pr->rows) {
-    RowRun a{};
-    common(a);
-    a.wg = pr->rwg.p;
-    a.P = pr->P;
-    a.ngrp = pr->rows_grp;
-    a.nwg = pr->rows_wg;
-    a.nslot = pr->rows_slots;
-    a.nquad = sys->hrow.quad0[sys->nb];
-    const RowDesc *rd = sys->drow.p;
-    const double *dq = sys->Dq.p;
-    void *args[] = {&a, &d, &rd, &dq};
+    RowRuns m{};
+    m.n = 1;
+    RowRun &a = m.run[0];
+    a = row_run(pr, attempts);
+    void *one[] = {&a}, *many[] = {&m};
     const void *fn =
         pr->P > 1 ? reinterpret_cast<const void *>(k_rows_run<1, true>)
         : pr->rows_kq == 1
@@ -1844,10 +1868,11 @@ static bool run_attempts_persistent(mpci_prop *pr, int attempts) {
         : pr->rows_kq == 2
             ? reinterpret_cast<const void *>(k_rows_run<2, false>)
             : reinterpret_cast<const void *>(k_rows_run<4, false>);
-    e = launch(fn, pr->rows_wg * pr->rows_grp, kRwThreads, args, &a.start_ms, pr->rows_lds);
+    e = launch(fn, pr->rows_wg * pr->rows_grp, kRwThreads,
+               pr->P > 1 ? many : one, &a.start_ms, pr->rows_lds);
   } else {
     TileRun a{};
-    common(a);
+    fill_run(pr, attempts, a);
     a.wg = pr->twg.p;
     a.seg = pr->tseg.p;
     a.nslot = pr->tslot.p;
@@ -1858,6 +1883,7 @@ static bool run_attempts_persistent(mpci_prop *pr, int attempts) {
     a.xs_rows = pr->tiles_xrows;
     a.xs_segs = pr->tiles_xsegs;
     a.xs_pieces = pr->tiles_xpieces;
+    const SysDesc *d = pr->ddesc.p;
     const TileDesc *td = pr->tdesc.p;
     void *args[] = {&a, &d, &td};
     e = launch(reinterpret_cast<const void *>(k_tiles_run), pr->tiles_wg,
@@ -2232,6 +2258,27 @@ extern "C" int mpci_prop_adaptive(mpci_prop *pr, const double *t0,
   return rc;
 }
 
+namespace {
+// One propagator of a multi run.
+struct Member {
+  mpci_prop *pr = nullptr;
+  std::vector<Ctl> c;
+  std::vector<std::vector<LogEnt>> acc;
+  bool busy = false, finished = false;
+};
+
+// The members' statistics; MPCI_ERR_LIMIT where a pulse hit its limit.
+int report(const std::vector<Member> &m, mpci_stats *const *stats) {
+  int rc = MPCI_OK;
+  for (size_t i = 0; i < m.size(); ++i) {
+    if (stats && stats[i]) fill_stats(m[i].c, stats[i]);
+    for (auto &x : m[i].c)
+      if (x.status) rc = fail(MPCI_ERR_LIMIT, "adaptive: max_attempts hit");
+  }
+  return rc;
+}
+}  // namespace
+
 // Several propagators (instances: different systems, different P) stepped
 // concurrently.  Each member runs on its own stream; whenever a member's
 // chunk has drained, its log is collected and its next chunk is enqueued at
@@ -2240,35 +2287,7 @@ extern "C" int mpci_prop_adaptive(mpci_prop *pr, const double *t0,
 // persistent launch takes the device for itself, so it is kept short
 // (persistent_attempts): a small instance waits for the others' launches, not
 // for their runs.
-extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
-                                   const double *const *t0,
-                                   const double *const *t1,
-                                   const double *const *h0, double atol,
-                                   double rtol, int max_attempts,
-                                   mpci_stats *const *stats) {
-  if (n < 1 || !props || !t0 || !t1 || !h0)
-    return fail(MPCI_ERR_ARG, "mpci_multi_adaptive: bad argument");
-  for (int i = 0; i < n; ++i) {
-    if (!props[i] || !t0[i] || !t1[i] || !h0[i])
-      return fail(MPCI_ERR_ARG, "mpci_multi_adaptive: NULL member");
-    for (int j = 0; j < i; ++j)
-      if (props[j] == props[i])
-        return fail(MPCI_ERR_ARG, "mpci_multi_adaptive: a propagator is "
-                                  "listed twice");
-  }
-  struct Member {
-    mpci_prop *pr;
-    std::vector<Ctl> c;
-    std::vector<std::vector<LogEnt>> acc;
-    bool busy = false, finished = false;
-  };
-  std::vector<Member> m(n);
-  for (int i = 0; i < n; ++i) {
-    m[i].pr = props[i];
-    TRY(setup_adaptive(props[i], t0[i], t1[i], h0[i], atol, rtol,
-                       max_attempts, 0, m[i].c, m[i].acc));
-    TRY(start_ctl(props[i], m[i].c));
-  }
+static int run_members(std::vector<Member> &m) {
   for (;;) {
     int live = 0, unfinished = 0;
     for (auto &x : m) unfinished += !x.finished;
@@ -2304,13 +2323,147 @@ extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
       if (!got) std::this_thread::yield();
     }
   }
-  int rc = MPCI_OK;
+  return MPCI_OK;
+}
+
+// Batches in the row form, several in one launch: k_rows_run's runs share
+// the compute units out, each with fewer groups and so more pulses a group.
+// One launch after the other costs the sum of their attempts, together the
+// slowest one's: 8 members of 5 pulses on 60 x 8 205 us an attempt of all
+// members one after the other, 160 us as one batched group, 92 us together.
+// Runs nothing where that is no gain or there is no room, and stops where a
+// launch gives up; run_members goes on.
+static int rows_together(std::vector<Member> &m) {
+  const int n = (int)m.size();
+  if (n < 2 || n > kRowRuns) return MPCI_OK;
+  const int ncu = m[0].pr->sys->ncu;
+  std::vector<int> wgs(n), grp(n, 1);
+  int used = 0;
+  auto us = [&](int i, int g) {
+    return ((m[i].pr->P + g - 1) / g) * row_pulse_us(m[i].pr->sys);
+  };
+  double apart = 0.0;
   for (int i = 0; i < n; ++i) {
-    if (stats && stats[i]) fill_stats(m[i].c, stats[i]);
-    for (auto &x : m[i].c)
-      if (x.status) rc = fail(MPCI_ERR_LIMIT, "adaptive: max_attempts hit");
+    const mpci_prop *pr = m[i].pr;
+    if (pr->instrument || pr->coop_refused) return MPCI_OK;
+    used += wgs[i] = row_groups(pr->sys);
+    apart += us(i, pr->rows_grp);
   }
-  return rc;
+  if (used > ncu) return MPCI_OK;
+  // one group each, then one more for the slowest while there is room
+  double slowest = 0.0;
+  for (;;) {
+    int k = 0;
+    for (int i = 1; i < n; ++i)
+      if (us(i, grp[i]) > us(k, grp[k])) k = i;
+    slowest = us(k, grp[k]);
+    if (grp[k] >= m[k].pr->P || used + wgs[k] > ncu) break;
+    used += wgs[k];
+    ++grp[k];
+  }
+  if (slowest >= apart) return MPCI_OK;
+  struct Share {
+    DevBuf<RowWg> wg;
+    DevBuf<double2> xb, rb;
+    int slots = 1;
+    size_t lds = 0;
+  };
+  std::vector<Share> sh(n);
+  for (int i = 0; i < n; ++i) {
+    mpci_prop *pr = m[i].pr;
+    Share &q = sh[i];
+    q.slots = std::min((pr->P + grp[i] - 1) / grp[i], kRwSlots);
+    std::vector<RowWg> wg;
+    int kq = 1;
+    if (!plan_rows(pr, q.slots, wg, &q.lds, &kq)) return MPCI_OK;
+    const size_t held = (size_t)grp[i] * q.slots;
+    if (q.xb.alloc(held * 4 * pr->sys->N) != MPCI_OK ||
+        q.rb.alloc(held * 3 * pr->sys->hrow.quad0[pr->sys->nb]) != MPCI_OK ||
+        q.wg.alloc(wg.size()) != MPCI_OK) {
+      (void)hipGetLastError();
+      return MPCI_OK;
+    }
+    TRY(h2d(pr, q.wg.p, wg.data(), sizeof(RowWg) * wg.size()));
+  }
+  hipStream_t st = m[0].pr->stream;
+  const int attempts =
+      std::max(16, (int)(100e3 / std::max(100.0, slowest)));
+  for (bool gave_up = false; !gave_up;) {
+    RowRuns r{};
+    std::vector<Member *> live;
+    unsigned blocks = 0;
+    size_t lds = 0;
+    bool ok = true;
+    for (int i = 0; i < n; ++i) {
+      mpci_prop *pr = m[i].pr;
+      if (plan_chunk(pr, m[i].c) == 0) continue;
+      live.push_back(&m[i]);
+      RowRun &a = r.run[r.n++];
+      a = row_run(pr, std::min(attempts, pr->logcap));
+      a.wg = sh[i].wg.p;
+      a.xb = sh[i].xb.p;
+      a.rb = sh[i].rb.p;
+      a.ngrp = grp[i];
+      a.nslot = sh[i].slots;
+      blocks += (unsigned)(a.nwg * a.ngrp);
+      lds = std::max(lds, sh[i].lds);
+      ok = ok && begin_persistent(pr, st, a.xb, (int)sh[i].xb.n, nullptr, 0,
+                                  a.rb, (int)sh[i].rb.n);
+    }
+    if (live.empty()) break;
+    void *args[] = {&r};
+    ok = ok && hipLaunchCooperativeKernel(
+                   reinterpret_cast<const void *>(k_rows_run<1, true>),
+                   dim3(blocks), dim3(kRwThreads), args, (unsigned)lds,
+                   st) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    HIPCHK(hipStreamSynchronize(st));
+    if (!ok) break;
+    for (Member *x : live) {
+      x->pr->persistent = true;
+      TRY(read_ctl(x->pr, x->c));
+      TRY(drain_log(x->pr, x->c, x->acc));
+      gave_up = gave_up || !x->pr->rows;
+    }
+  }
+  return MPCI_OK;
+}
+
+// n checked members; together: those in the row form may share a launch.
+static int run_multi(int n, mpci_prop *const *props, const double *const *t0,
+                     const double *const *t1, const double *const *h0,
+                     double atol, double rtol, int max_attempts,
+                     mpci_stats *const *stats, bool together) {
+  std::vector<Member> m(n);
+  for (int i = 0; i < n; ++i) {
+    m[i].pr = props[i];
+    TRY(setup_adaptive(props[i], t0[i], t1[i], h0[i], atol, rtol,
+                       max_attempts, 0, m[i].c, m[i].acc));
+    TRY(start_ctl(props[i], m[i].c));
+  }
+  if (together) TRY(rows_together(m));
+  TRY(run_members(m));
+  return report(m, stats);
+}
+
+extern "C" int mpci_multi_adaptive(int n, mpci_prop *const *props,
+                                   const double *const *t0,
+                                   const double *const *t1,
+                                   const double *const *h0, double atol,
+                                   double rtol, int max_attempts,
+                                   mpci_stats *const *stats) {
+  if (n < 1 || !props || !t0 || !t1 || !h0)
+    return fail(MPCI_ERR_ARG, "mpci_multi_adaptive: bad argument");
+  for (int i = 0; i < n; ++i) {
+    if (!props[i] || !t0[i] || !t1[i] || !h0[i])
+      return fail(MPCI_ERR_ARG, "mpci_multi_adaptive: NULL member");
+    for (int j = 0; j < i; ++j)
+      if (props[j] == props[i])
+        return fail(MPCI_ERR_ARG, "mpci_multi_adaptive: a propagator is "
+                                  "listed twice");
+  }
+  return run_multi(n, props, t0, t1, h0, atol, rtol, max_attempts, stats,
+                   false);
 }
 
 // ---------------------------------------------------------------------
@@ -2370,8 +2523,8 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
     TRY(setup_adaptive(props[i], t0[i], t1[i], h0[i], atol, rtol,
                        max_attempts, 0, c, acc));
   }
-  // members whose batch runs in one persistent launch run it, beside each
-  // other, and the group is made of the others
+  // members whose batch runs in a persistent launch run in one, together
+  // where that is faster, and the group is made of the others
   std::vector<int> alone, rest;
   for (int i = 0; i < n; ++i)
     (props[i]->rows && props[i]->use_graph ? alone : rest).push_back(i);
@@ -2387,9 +2540,12 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
         h.push_back(h0[i]);
         st.push_back(stats ? stats[i] : nullptr);
       }
-      return (grouped ? mpci_multi_adaptive_grouped : mpci_multi_adaptive)(
-          (int)idx.size(), p.data(), a.data(), b.data(), h.data(), atol, rtol,
-          max_attempts, st.data());
+      const int k = (int)idx.size();
+      return grouped ? mpci_multi_adaptive_grouped(
+                           k, p.data(), a.data(), b.data(), h.data(), atol,
+                           rtol, max_attempts, st.data())
+                     : run_multi(k, p.data(), a.data(), b.data(), h.data(),
+                                 atol, rtol, max_attempts, st.data(), true);
     };
     const int rc = part(alone, false);
     if ((rc != MPCI_OK && rc != MPCI_ERR_LIMIT) || rest.empty()) return rc;
@@ -2489,10 +2645,6 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
   TRY(h2d(props[0], dtab.p, tab.data(), sizeof(GroupMember) * n));
   TRY(h2d(props[0], djobs.p, jobs.data(), sizeof(GemmJob) * jobs.size()));
   // per-member set-up, as mpci_prop_adaptive does it
-  struct Member {
-    std::vector<Ctl> c;
-    std::vector<std::vector<LogEnt>> acc;
-  };
   std::vector<Member> m(n);
   for (int i = 0; i < n; ++i) {
     TRY(setup_adaptive(props[i], t0[i], t1[i], h0[i], atol, rtol,
@@ -2565,12 +2717,7 @@ extern "C" int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
   (void)hipGraphExecDestroy(gexec);
   (void)hipGraphDestroy(graph);
   TRY(rc);
-  for (int i = 0; i < n; ++i) {
-    if (stats && stats[i]) fill_stats(m[i].c, stats[i]);
-    for (auto &x : m[i].c)
-      if (x.status) rc = fail(MPCI_ERR_LIMIT, "adaptive: max_attempts hit");
-  }
-  return rc;
+  return report(m, stats);
 }
 
 // Schedule replay with per-pulse step counts n[p] (<= stride); hs is

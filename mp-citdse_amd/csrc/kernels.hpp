@@ -53,6 +53,9 @@ struct AdjArgs {
 // cooperative launch: ngrp groups of nwg workgroups, nslot pulses at a time
 // in each.
 struct RowRun {
+  const SysDesc *d;
+  const RowDesc *rows;
+  const double *Dq;      // row store
   const RowWg *wg;
   double2 *X;            // committed states (N x P)
   const double *E;
@@ -70,6 +73,21 @@ struct RowRun {
   int limit_ms;          // time limit of one wait
   int start_ms;          // > 0: not cooperative, wait for all workgroups
   int *arrived;          // workgroups that run
+};
+
+// The batches of one launch: each has nwg ngrp workgroups of the grid.
+constexpr int kRowRuns = 8;
+struct RowRuns {
+  int n, pad;
+  RowRun run[kRowRuns];
+};
+template <bool kMany>
+struct RowArgs {
+  using type = RowRun;
+};
+template <>
+struct RowArgs<true> {
+  using type = RowRuns;
 };
 
 // The persistent tile kernel, likewise.
@@ -187,8 +205,7 @@ __global__ void k_rows_begin(double2 *xb, int nxb, double2 *pb, int npb,
                              int *abort_flag, int *arrived);
 __global__ void k_tiles_run(TileRun a, const SysDesc *d, const TileDesc *td);
 template <int kQ, bool kMany>
-__global__ void k_rows_run(RowRun a, const SysDesc *d, const RowDesc *rd,
-                           const double *Dq);
+__global__ void k_rows_run(typename RowArgs<kMany>::type args);
 __global__ void k_finalize(Ctl *ctl, const double *red, int nblk, int P,
                            const double *hs, const double *Ftab,
                            const PulseDev *pulses, const double *env);

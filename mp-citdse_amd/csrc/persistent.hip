@@ -41,7 +41,8 @@ namespace mpci {
 // control (a polling wave each) and its attempts.  Per attempt of all pulses,
 // against the batched launches (13 GEMM and 13 stage launches of 5 to 14 us
 // each whatever they hold): 300 x 6, P = 5 164 -> 62 us; 198 x 4, P = 16 145
-// -> 78 us; 60 x 8, P = 5 128 -> 28 us.  A further pulse of a group costs
+// -> 78 us; 60 x 8, P = 5 128 -> 28 us.  One launch may hold several batches
+// (RowRuns), each with workgroups of its own.  A further pulse of a group costs
 // about 20 us, 1.5 us a stage: the computing waves' tableau sums, coupling
 // sums and stage algebra.  Fewer, larger groups (32 to 64 rows a workgroup)
 // were slower from P = 2 on (300 x 6, P = 5: 98 to 141 us).
@@ -153,10 +154,12 @@ __device__ __forceinline__ bool all_started(int *arrived, int *abort_flag,
   return true;
 }
 
+// Workgroup blk of run a.
 template <int kQ, bool kMany>
-__global__ __launch_bounds__(kRwThreads) void k_rows_run(
-    RowRun a, const SysDesc *__restrict__ dp, const RowDesc *__restrict__ rp,
-    const double *__restrict__ Dq) {
+__device__ __forceinline__ void rows_run(const RowRun &a, int blk) {
+  const SysDesc *__restrict__ dp = a.d;
+  const RowDesc *__restrict__ rp = a.rows;
+  const double *__restrict__ Dq = a.Dq;
   // chunks of a quad kept in registers: one quad a wave leaves room for them
   constexpr int kReg = kQ == 1 ? kRwReg : 0;
   static_assert(!kMany || kQ == 1, "several slots: a quad a wave");
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
   const SysDesc &d = *dp;
   // group grp of nwg workgroups runs pulses grp, grp + ngrp, .., nslot of
   // them at a time, a stage of each in turn
-  const int grp = blockIdx.x / a.nwg, wgi = blockIdx.x - grp * a.nwg;
+  const int grp = blk / a.nwg, wgi = blk - grp * a.nwg;
   const RowWg g = a.wg[wgi];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -645,15 +648,27 @@ __global__ __launch_bounds__(kRwThreads) void k_rows_run(
   }
 }
 
-#define MPCI_ROWS(Q, MANY)                                          \
-  template __global__ void k_rows_run<Q, MANY>(RowRun, const SysDesc *, \
-                                               const RowDesc *,     \
-                                               const double *)
-MPCI_ROWS(1, false);
-MPCI_ROWS(2, false);
-MPCI_ROWS(4, false);
-MPCI_ROWS(1, true);
-#undef MPCI_ROWS
+template <int kQ, bool kMany>
+__global__ __launch_bounds__(kRwThreads) void k_rows_run(
+    typename RowArgs<kMany>::type args) {
+  int blk = blockIdx.x;
+  if constexpr (kMany) {
+    int i = 0;
+    for (; i + 1 < args.n; ++i) {
+      const int n = args.run[i].nwg * args.run[i].ngrp;
+      if (blk < n) break;
+      blk -= n;
+    }
+    rows_run<kQ, kMany>(args.run[i], blk);
+  } else {
+    rows_run<kQ, kMany>(args, blk);
+  }
+}
+
+template __global__ void k_rows_run<1, false>(RowRun);
+template __global__ void k_rows_run<2, false>(RowRun);
+template __global__ void k_rows_run<4, false>(RowRun);
+template __global__ void k_rows_run<1, true>(RowRuns);
 
 // ---------------------------------------------------------------------
 // Persistent tile kernel: whole attempts of one pulse on a larger system in

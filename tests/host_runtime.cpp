@@ -130,10 +130,19 @@ hipError_t launch(const void *fn, void **args) {
       *flag = 0;
     };
   } else if (is("k_rows_run")) {
-    const auto a = arg<RowRun>(args, 0);
-    attempts.push_back(a.attempts);
+    // of several batches, or of one
+    RowRuns r{};
+    if (is("ELb1E")) {
+      r = arg<RowRuns>(args, 0);
+    } else {
+      r.n = 1;
+      r.run[0] = arg<RowRun>(args, 0);
+    }
+    attempts.push_back(r.run[0].attempts);
     lds = config.back().lds;
-    f = [=] { persistent(a, a.P); };
+    f = [=] {
+      for (int i = 0; i < r.n; ++i) persistent(r.run[i], r.run[i].P);
+    };
   } else if (is("k_tiles_run")) {
     const auto a = arg<TileRun>(args, 0);
     attempts.push_back(a.attempts);

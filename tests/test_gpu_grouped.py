@@ -94,3 +94,12 @@ def test_persistent_members_beside_a_group(mpci, members):
     """The first two members run persistently, the third by launches."""
     check(mpci, members, [{}, {}, {}], [False, False, True])
     check(mpci, members, [{}, {}, {}], [False, True, True])
+
+
+def test_persistent_members_in_one_launch(mpci, members):
+    """Small batches that run persistently by themselves: grouped, their
+    workgroups share one launch, with fewer groups and more pulses a group,
+    and slots that take one pulse after another."""
+    m = members
+    check(mpci, [m[0], m[1]], [{}] * 2, [False] * 2)
+    check(mpci, [m[0]] * 4 + [m[1], m[2]] + [m[0]] * 2, [{}] * 8, [False] * 8)

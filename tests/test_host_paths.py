@@ -398,3 +398,42 @@ def test_every_candidate_tile_is_launched(host_runtime):  # noqa: F811
         p.prop_fixed(0.0, 0.1, np.full((3, 1), 0.02))
         assert launches(c["kernel"]) == launches("k_gemm") == 13, c
     """)
+
+
+def test_grouped_row_members_share_launches(host_runtime):  # noqa: F811
+    """Grouped members in the row form run in launches for all of them; one
+    that gives up goes on by launches of single stages; too many rows for the
+    device together run one after the other."""
+    host_runtime("""
+    def run(shapes, quits=()):
+        ps = []
+        for i, (s, P) in enumerate(shapes):
+            p = mpci.Propagator(system(s), P=P)
+            for k in range(P):
+                p.set_state(np.arange(2.0 * sum(s)), k)
+            if i in quits:
+                p.set_wait_limit(-1)
+            ps.append(p)
+        n = len(ps)
+        t1 = [2.0 + i + np.arange(p.P) for i, p in enumerate(ps)]
+        rt.rt_clear()
+        before = rt.rt_live()
+        st = mpci.multi_adaptive(ps, [0.0] * n, t1, [0.25] * n, 1e-9, 1e-9,
+                                 grouped=True)
+        assert rt.rt_live() <= before
+        for i, p in enumerate(ps):
+            for k in range(p.P):
+                steps = int(t1[i][k] / 0.25)
+                assert st[i][k].accepted == steps and st[i][k].t == t1[i][k]
+                assert np.array_equal(p.get_state(k),
+                                      np.arange(2.0 * p.sys.N) + steps)
+        return launches("k_rows_run"), launches("k_apply")
+
+    assert run([([60] * 8, 5)] * 8) == (1, 0)
+    assert run([([60] * 8, 5), ([40, 30], 3), ([198] * 4, 9)]) == (1, 0)
+    n, apply = run([([60] * 8, 5), ([40, 30], 3), ([198] * 4, 2)], [1])
+    assert n == 1 and 20 <= apply < 40     # (plus what was planned past the end)
+    assert run([([300] * 6, 5)] * 3) == (3, 0)
+    # no gain (two pulses a group each), and a third in grouped launches
+    assert run([([60] * 8, 5)] * 2 + [([300, 280], 200)])[0] == 2
+    """)
