@@ -263,10 +263,11 @@ int mpci_prop_observables(mpci_prop *prop, int electrons, double threshold,
  * another one on the device holds them, makes an ordinary launch of it. */
 int mpci_prop_set_graph(mpci_prop *prop, int enable);
 /* The workgroups of that launch wait for one another; a wait is given up
- * after `ms` milliseconds (0: the default of 20000; negative: at once), for
- * instance when other work holds part of the device for that long.  The run
- * then goes back to where the launch began and goes on with one launch per
- * stage. */
+ * after `ms` milliseconds (0: the default of 20000; -1: at once; -2 - n: after
+ * 100 ms, while one workgroup leaves the launch after n attempts), for instance
+ * when other work holds part of the device for that long.  The run then goes
+ * back to where the launch began and goes on with one launch per stage, and so
+ * do later ones.  Negative limits serve tests. */
 int mpci_prop_set_wait_limit(mpci_prop *prop, int ms);
 /* One pulse on a small system: each stage as one fused launch (coupling
  * from row-major copies of D_L and D_L^T, one wave per row, then the stage

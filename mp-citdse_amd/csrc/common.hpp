@@ -89,9 +89,10 @@ struct RowDesc {
 
 // One workgroup of the persistent row kernel: rows row0 .. row0 + nrows - 1
 // of block L, its first quad's number, and how many chunks of each quad it
-// keeps in LDS.
+// keeps in LDS.  quit > 0: it leaves the last group after quit - 1 attempts,
+// so that the others wait in vain.
 struct RowWg {
-  int L, row0, nrows, quad0, nlds, pad;
+  int L, row0, nrows, quad0, nlds, quit;
 };
 
 // ---- persistent tile form (one pulse, larger systems) ------------------
@@ -113,7 +114,7 @@ struct TileWg {
   int ngroups, nlds;   // groups in all, groups kept in LDS
   int L, row0, nrows;  // its rows: of block L (nrows may be 0)
   int nrs, ncs;        // partials per row: D x_{L+1}, D^T x_{L-1} (at most)
-  int pad;
+  int quit;            // as RowWg's
 };
 struct TileDesc {
   int part_n;                  // partials of one exchange copy

@@ -1009,6 +1009,7 @@ constexpr long long kSmallPathBytes = 12LL << 20;
 // tile form takes 127, 355 and 763 us there.
 constexpr size_t kPinnedStates = 8u << 20;  // bound of the pinned buffer
 constexpr int kWaitLimitMs = 20000;  // time limit of one wait in them
+constexpr int kQuitLimitMs = 100;    // where a workgroup quits (tests)
 // Time limit of the start of an ordinary launch: two processes' launches
 // that hold half the device each let go of it after this.
 constexpr int kStartLimitMs = 200;
@@ -1797,7 +1798,7 @@ static void fill_run(mpci_prop *pr, int attempts, A &a) {
   a.track = pr->track;
   a.N = pr->sys->N;
   a.attempts = attempts;
-  a.limit_ms = pr->wait_limit_ms;
+  a.limit_ms = pr->wait_limit_ms < -1 ? kQuitLimitMs : pr->wait_limit_ms;
   a.arrived = &pr->ctl.p[2 * pr->P].nlog;
   a.start_ms = pr->coop_refused ? kStartLimitMs : 0;
 }
@@ -3305,8 +3306,21 @@ extern "C" int mpci_prop_set_small_path(mpci_prop *pr, int mode,
   return MPCI_OK;
 }
 
+// Has the last workgroup of a table leave early (RowWg::quit), or no longer.
+template <class W>
+static int set_quit(mpci_prop *pr, DevBuf<W> &table, int quit) {
+  if (!table.p) return MPCI_OK;
+  W w;
+  TRY(d2h(pr, &w, table.p + table.n - 1, sizeof(W)));
+  w.quit = quit;
+  return h2d(pr, table.p + table.n - 1, &w, sizeof(W));
+}
+
 extern "C" int mpci_prop_set_wait_limit(mpci_prop *pr, int ms) {
   if (!pr) return fail(MPCI_ERR_ARG, "NULL argument");
+  const int quit = ms < -1 ? -1 - std::max(ms, -(1 << 30)) : 0;
+  TRY(set_quit(pr, pr->rwg, quit));
+  TRY(set_quit(pr, pr->twg, quit));
   pr->wait_limit_ms = ms == 0 ? kWaitLimitMs : ms;
   return MPCI_OK;
 }

@@ -169,6 +169,8 @@ __device__ __forceinline__ void rows_run(const RowRun &a, int blk) {
   // them at a time, a stage of each in turn
   const int grp = blk / a.nwg, wgi = blk - grp * a.nwg;
   const RowWg g = a.wg[wgi];
+  const int attempts =
+      g.quit > 0 && grp == a.ngrp - 1 ? g.quit - 1 : a.attempts;
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int L = g.L, gauge = d.gauge;
@@ -317,7 +319,7 @@ __device__ __forceinline__ void rows_run(const RowRun &a, int blk) {
           kMany ? min((int)nslot, (a.P - 1 - grp) / a.ngrp - base + 1) : 1;
       __syncthreads();  // the last pulses' records have been read
       __syncthreads();  // these are there
-      for (int n = 0; n < a.attempts; ++n) {
+      for (int n = 0; n < attempts; ++n) {
         const unsigned act = live_slots(ns);
         if (act == 0) break;
         for (int s = 0; s < kStages; ++s) {
@@ -450,7 +452,7 @@ __device__ __forceinline__ void rows_run(const RowRun &a, int blk) {
           if (kMany) own_rows[b * slot_n + kStages * nr4 + lr[m]] = x[m];
         }
     __syncthreads();
-    for (int n = 0; n < a.attempts; ++n) {
+    for (int n = 0; n < attempts; ++n) {
       const unsigned act = live_slots(ns);
       if (act == 0) break;
       for (unsigned mb = act; mb; mb &= mb - 1) {
@@ -739,6 +741,7 @@ __global__ __launch_bounds__(kGvThreads) void k_tiles_run(
   const int tr = t & 15, cg = t >> 4;
   constexpr int kWv = kGvThreads / 64;
   const int gauge = d.gauge, ngroups = g.ngroups;
+  const int attempts = g.quit > 0 ? g.quit - 1 : a.attempts;
   const int nown = g.nrows;
   const int nitems = g.nrs + g.ncs;
 
@@ -950,7 +953,7 @@ __global__ __launch_bounds__(kGvThreads) void k_tiles_run(
     if (nstr > 0) load_group(streamed(m, 0, 1), S[m]);
   }
   int ph = 0;  // which of them comes next
-  for (int n = 0; n < a.attempts && !cl.done; ++n) {
+  for (int n = 0; n < attempts && !cl.done; ++n) {
     const double h = cl.hc;
     const unsigned rnext = rbuf == 2 ? 0 : rbuf + 1;
     double2 xin = x, v = x;

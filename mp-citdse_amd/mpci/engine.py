@@ -233,7 +233,8 @@ class Propagator:
         check(_lib.tdse_lib().mpci_prop_set_graph(self.h, int(on)))
 
     def set_wait_limit(self, ms: int = 0):
-        """Time limit of one wait inside a persistent launch (0: default)."""
+        """Time limit of one wait inside a persistent launch (0: default;
+        negative: see mpci_prop_set_wait_limit)."""
         check(_lib.tdse_lib().mpci_prop_set_wait_limit(self.h, int(ms)))
 
     def set_instrument(self, on: bool):

@@ -437,3 +437,27 @@ def test_grouped_row_members_share_launches(host_runtime):  # noqa: F811
     # no gain (two pulses a group each), and a third in grouped launches
     assert run([([60] * 8, 5)] * 2 + [([300, 280], 200)])[0] == 2
     """)
+
+
+@pytest.mark.parametrize("s,P", [([60, 75, 33], 1), ([1777, 2401], 1),
+                                 ([60, 75, 33], 3)])
+def test_work_of_a_launch_that_gave_up_is_undone(host_runtime, s, P):  # noqa
+    """States, control records and log entries written before a launch gave
+    up are put back; the run counts every step once."""
+    host_runtime(f"""
+    g, P = system({s}), {P}
+    for n in (0, 3, 8):
+        rt.rt_abort_after(n)
+        p = mpci.Propagator(g, P=P)
+        x0 = np.arange(2.0 * g.N)
+        for i in range(P):
+            p.set_state(x0 + i, i)
+        rt.rt_clear()
+        st, log = p.prop_adaptive(0.0, 2.0, 0.25, 1e-9, 1e-9, log_cap=20)
+        assert launches("_run") == 1 and launches("k_apply") >= 8
+        for i in range(P):
+            assert (st[i].accepted, st[i].attempts, st[i].t) == (8, 8, 2.0)
+            assert np.array_equal(p.get_state(i), x0 + i + 8)
+            assert log[i, :8, 0].tolist() == [0.25 * (k + 1) for k in range(8)]
+        p.close()
+    """)
