@@ -945,6 +945,11 @@ static int tune_gemm(mpci_prop *pr, const GemmCand *only) {
           continue;
         float ms = 0.f;
         rc = time_gemm_cand(pr, cd, e0, e1, &ms, best);
+        if (rc != MPCI_OK && !(pr->part.p && pr->dgjobs.p)) {
+          (void)hipGetLastError();  // no room for its buffers
+          rc = MPCI_OK;
+          continue;
+        }
         if (rc != MPCI_OK) break;
         if (ms < best) {
           best = ms;

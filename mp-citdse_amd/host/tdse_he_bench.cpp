@@ -1,14 +1,16 @@
 // Stand-alone driver of the single-pulse hot path over the C ABI, for
 // hardware-counter runs that need a plain process (no Python runtime).
 //
-//   tdse_he_bench [attempts] [copy_mib] [batch_pulses] [he|h]
+//   tdse_he_bench [attempts] [copy_mib] [batch_pulses] [he|h|NxB] [default]
 //
 // Builds the seeded synthetic He system (4 blocks of 4000 states, velocity
 // gauge; with `h`, the H-shaped system of 21 blocks of 998 states that the
-// multi-instance bench leg uses), propagates one sin^2 pulse (w = 0.7, E0 = 0.03, 10 cycles) from the
-// ground state with the adaptive RKF78 (atol = rtol = 1e-10) for `attempts`
-// attempts, launched individually (no graph), then copies copy_mib MiB
-// device to device three times.  The copy reads and writes exactly
+// multi-instance bench leg uses; with NxB, B blocks of N states), propagates
+// one sin^2 pulse (w = 0.7, E0 = 0.03, 10 cycles) from the ground state with the
+// adaptive RKF78 (atol = rtol = 1e-10) for `attempts` attempts, launched
+// individually (no graph; with `default`, in the form that the library
+// chooses: persistent launches for one pulse, and for small batches), then
+// copies copy_mib MiB device to device three times.  The copy reads and writes exactly
 // copy_mib MiB per launch, which scales byte counters (FETCH_SIZE,
 // WRITE_SIZE) measured for the coupling kernel in the same run.
 //
@@ -40,9 +42,13 @@ int main(int argc, char **argv) {
   const long long copy_mib = argc > 2 ? std::atoll(argv[2]) : 1024;
   const int batch = argc > 3 ? std::atoi(argv[3]) : 0;
   const bool hshape = argc > 4 && argv[4][0] == 'h' && argv[4][1] == 0;
+  const int chosen = argc > 5 && argv[5][0] == 'd';
   // the seeds and energy ranges of mpci/synth.py as bench.py uses them
-  const int nb = hshape ? 21 : 4;
-  const std::vector<int> s(nb, hshape ? 998 : 4000);
+  int nb = hshape ? 21 : 4, size = hshape ? 998 : 4000;
+  if (argc > 4 && std::sscanf(argv[4], "%dx%d", &size, &nb) == 2 &&
+      (size < 1 || nb < 2 || nb > 32))
+    return 1;
+  const std::vector<int> s(nb, size);
   const unsigned long long seed = hshape ? 20261203ULL : 20261202ULL;
   const double e_lo = hshape ? -0.5 : -2.9;
   std::vector<std::vector<double>> E(nb), D(nb - 1);
@@ -63,7 +69,7 @@ int main(int argc, char **argv) {
         "mpci_system_create");
   mpci_prop *prop = nullptr;
   check(mpci_prop_create(sys, 1, &prop), "mpci_prop_create");
-  check(mpci_prop_set_graph(prop, 0), "mpci_prop_set_graph");
+  check(mpci_prop_set_graph(prop, chosen), "mpci_prop_set_graph");
   mpci_pulse pl;
   const double w = 0.7, e0 = 0.03;
   check(mpci_pulse_sine(e0 * e0, w, 0.0, 10, 'v', &pl), "mpci_pulse_sine");
@@ -103,7 +109,7 @@ int main(int argc, char **argv) {
     const int P = batch;
     mpci_prop *bp = nullptr;
     check(mpci_prop_create(sys, P, &bp), "mpci_prop_create (batch)");
-    check(mpci_prop_set_graph(bp, 0), "mpci_prop_set_graph");
+    check(mpci_prop_set_graph(bp, chosen), "mpci_prop_set_graph");
     // the pulse batch of mpci/synth.py pulse_batch (seed + 3, stream 1000)
     std::vector<double> u(3 * (size_t)P);
     mpci_synth_uniform(20261202ULL + 3, 1000, 3LL * P, 0.0, 1.0, u.data());

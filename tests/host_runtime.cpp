@@ -25,7 +25,8 @@ namespace {
 std::recursive_mutex mu;
 std::map<const void *, std::string> names;   // kernel stubs
 std::map<void *, size_t> live;               // allocations
-size_t fail_above = ~(size_t)0, fail_from = 1, fail_to = 0, alloc_us = 0;
+size_t fail_above = ~(size_t)0, fail_from = 1, fail_to = 0, alloc_us = 0,
+       fail_unit = 0, fail_most = 0;
 int abort_after = -1;                        // persistent launches give up
 std::vector<std::string> launched;
 std::vector<int> attempts;                   // of each persistent launch
@@ -219,6 +220,11 @@ void rt_fail_at(size_t from, size_t to) {
   fail_from = from;
   fail_to = to;
 }
+// multiples of unit, more than `most` of it
+void rt_fail_multiples(size_t unit, size_t most) {
+  fail_unit = unit;
+  fail_most = most;
+}
 void rt_alloc_us(size_t us) { alloc_us = us; }
 void rt_abort_after(int n) { abort_after = n; }
 size_t rt_live() { return live.size(); }
@@ -296,7 +302,9 @@ hipError_t hipMalloc(void **p, size_t n) {
     std::this_thread::sleep_for(std::chrono::microseconds(alloc_us));
   std::lock_guard<std::recursive_mutex> lk(mu);
   *p = nullptr;
-  if (n > fail_above || (n >= fail_from && n <= fail_to)) return hipErrorOutOfMemory;
+  if (n > fail_above || (n >= fail_from && n <= fail_to) ||
+      (fail_unit && n % fail_unit == 0 && n / fail_unit > fail_most))
+    return hipErrorOutOfMemory;
   *p = std::calloc(n, 1);
   live[*p] = n;
   return hipSuccess;

@@ -461,3 +461,24 @@ def test_work_of_a_launch_that_gave_up_is_undone(host_runtime, s, P):  # noqa
             assert log[i, :8, 0].tolist() == [0.25 * (k + 1) for k in range(8)]
         p.close()
     """)
+
+
+def test_tile_search_leaves_out_what_does_not_fit(host_runtime):  # noqa: F811
+    """Creating a batch needs room for the tile it runs: candidates with finer
+    K splits, whose partials do not fit, are left out."""
+    split = (300 + 2 * 280 + 310) * 40 * 16   # partials of one K split
+    host_runtime(REFUSED + f"""
+rt.rt_cost(b"k_gemm", 100.0, 100.0, 0)
+rt.rt_fail_multiples.argtypes = [ctypes.c_size_t] * 2
+for most in (8, 4, 2, 1):
+    rt.rt_fail_multiples({split}, most)
+    g = system([300, 280, 310])
+    p = mpci.Propagator(g, P=40)
+    assert p.gemm_config()["ksplit"] <= most
+    p.prop_fixed(0.0, 0.1, np.full((40, 2), 0.02))
+    p.close(), g.close()
+    assert rt.rt_live() == 0
+rt.rt_fail_multiples({split}, 0)   # no tile fits
+g = system([300, 280, 310])
+refused(lambda: mpci.Propagator(g, P=40))
+""")
