@@ -173,7 +173,9 @@ int mpci_prop_adaptive(mpci_prop *prop, const double *t0, const double *t1,
  * max_attempts, track 0, stats[i], no log) for n distinct propagators, which
  * may hold different systems and batch sizes, concurrently on one device:
  * each member keeps its own stream and its next chunk is launched as soon
- * as its previous one drains.  Results equal n separate calls.  stats[i] may
+ * as its previous one drains.  A member that runs in cooperative launches has
+ * the device for about 20 ms at a time while others are unfinished.  Results
+ * equal n separate calls.  stats[i] may
  * be NULL.  Returns MPCI_ERR_LIMIT when any pulse hit max_attempts. */
 int mpci_multi_adaptive(int n, mpci_prop *const *props,
                         const double *const *t0, const double *const *t1,
@@ -185,7 +187,9 @@ int mpci_multi_adaptive(int n, mpci_prop *const *props,
  * of all members' panels, one stage launch over all members' rows, one
  * step-control and one apply launch over all their pulses, captured once
  * as a graph.  Each member keeps its own K split, so its results equal a
- * separate mpci_prop_adaptive call bit for bit.  1 <= n <= 8; every
+ * separate mpci_prop_adaptive call bit for bit.  Members whose batch runs in
+ * cooperative launches (mpci_prop_set_graph) run in those, before the group
+ * and, where that is faster, several in one.  1 <= n <= 8; every
  * member must be a batched propagator (P >= 2) with two or more blocks on
  * the same device, otherwise MPCI_ERR_NOTSUP (use mpci_multi_adaptive). */
 int mpci_multi_adaptive_grouped(int n, mpci_prop *const *props,
@@ -259,7 +263,7 @@ int mpci_prop_observables(mpci_prop *prop, int electrons, double threshold,
  * small-system stages (below), otherwise with the coupling sums in an order
  * of its own (equal to rounding, and the same from run to run).  So does a
  * batch of few pulses on such a small system, every pulse with the bits of
- * its run alone. A process that is refused cooperative launches, because
+ * its run alone.  Such a launch takes about 100 ms at most.  A process that is refused cooperative launches, because
  * another one on the device holds them, makes an ordinary launch of it. */
 int mpci_prop_set_graph(mpci_prop *prop, int enable);
 /* The workgroups of that launch wait for one another; a wait is given up
@@ -270,8 +274,9 @@ int mpci_prop_set_graph(mpci_prop *prop, int enable);
  * do later ones.  Negative limits serve tests. */
 int mpci_prop_set_wait_limit(mpci_prop *prop, int ms);
 /* One pulse on a small system: each stage as one fused launch (coupling
- * from row-major copies of D_L and D_L^T, one wave per row, then the stage
- * algebra) instead of the GEMV tile kernel and the stage kernel.  mode -1
+ * from a store of both dipole blocks of every four rows, one wave per four
+ * rows, then the stage algebra) instead of the GEMV tile kernel and the stage
+ * kernel.  mode -1
  * (default): on when P = 1, the system has more than one block and its
  * dipoles take at most 12 MiB; 0: off; 1: on whenever P = 1 and there is
  * more than one block (also inside the cooperative launch, whatever the

@@ -997,10 +997,15 @@ static int autotune_gemm(mpci_prop *pr) {
 }
 
 // Dipole bytes (8 S) up to which one pulse takes the small-system path by
-// default: there every stage is a handful of microseconds of launch and
-// latency, and the fused kernel halves the launches per attempt.  Measured
-// on four equal blocks: 1.95x the tile path at 0.9 MB of dipoles, 1.30x at
-// 8.6 MB, even at 15 MB, 0.85x at 24 MB.
+// default where it goes by launches (eager and instrumented runs, the adjoint,
+// single right-hand sides, after a persistent launch gave up): there every
+// stage is a handful of microseconds of launch and latency, and the fused
+// kernel halves the launches per attempt.  Tile path against fused stages, us
+// an attempt: 4 x 198 (0.9 MB) 159 / 76, 4 x 600 (8.6 MB) 161 / 106, 8 x 500 (14
+// MB) 164 / 112, 4 x 800 (15 MB) 160 / 135, 4 x 900 (19 MB) 161 / 164, 1201,
+// 1333, 997 (23 MB) 163 / 184, 2 x 2000 (32 MB) 174 / 205.  The two are even at
+// about 19 MB; the line stays at the 12 MiB that the interface states, as the
+// order of the sums, and with it the bits, changes at it.
 constexpr long long kSmallPathBytes = 12LL << 20;
 // The same for whole runs in one persistent launch: the row form
 // (k_rows_run) while a compute unit's share is at most 16 rows (a quad a
@@ -1094,6 +1099,16 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
   return (int)wg.size() <= sys->ncu;
 }
 
+// What a pulse costs its group of workgroups in the persistent row form, in us
+// an attempt (see rows_pay).
+static double row_pulse_us(const mpci_system *sys) {
+  int chunks = 0;
+  for (int L = 0; L < sys->nb; ++L)
+    chunks = std::max(chunks, row_chunks(sys, L));
+  const int c = std::max(chunks - kRwReg, 0);
+  return 20.0 + 1.2 * c + 0.045 * c * c;
+}
+
 // Whether a batch runs in the persistent row form: pulses are independent, so
 // groups of workgroups take some each and a group runs a stage of each of its
 // pulses in turn, which hides one's exchange behind the others'.  A pulse
@@ -1105,14 +1120,6 @@ static bool plan_rows(const mpci_prop *pr, int nslot, std::vector<RowWg> &wg,
 // 149, P = 20 196 / 175; 800 x 5, P = 3 93 / 210, P = 5 164 / 218; 2000 x 2, P
 // = 2 103 / 261, P = 4 196 / 265, P = 5 275 / 264; 1500, 1000, 1500, P = 2
 // 175 / 234; 80 x 32, P = 5 92 / 144.
-static double row_pulse_us(const mpci_system *sys) {
-  int chunks = 0;
-  for (int L = 0; L < sys->nb; ++L)
-    chunks = std::max(chunks, row_chunks(sys, L));
-  const int c = std::max(chunks - kRwReg, 0);
-  return 20.0 + 1.2 * c + 0.045 * c * c;
-}
-
 static bool rows_pay(const mpci_prop *pr) {
   const mpci_system *sys = pr->sys;
   const int n16 = row_groups(sys);
@@ -1766,8 +1773,8 @@ static int run_attempts_instrumented(mpci_prop *pr, int n) {
 
 // Attempts of one persistent launch.  It holds the compute units it runs on,
 // so that the work of other propagators, streams and processes waits for its
-// end: about 100 ms, 20 ms beside other members of a multi run.  A launch of
-// its own costs about 0.1 ms.  An attempt is taken for 13 sweeps of the dipoles at
+// end: about 100 ms, 20 ms beside other members of a multi run.  A launch
+// costs about 0.1 ms more.  An attempt is taken for 13 sweeps of the dipoles at
 // 5.5 TB/s, 100 us at least (a row form's is 28 to 120 us for the pulses that
 // it holds at a time, however many these are).
 static int persistent_attempts(const mpci_prop *pr, bool shared) {
@@ -1779,10 +1786,6 @@ static int persistent_attempts(const mpci_prop *pr, bool shared) {
   return std::min(pr->logcap, std::max(16, (int)n));
 }
 
-// Attempts until the pulse has finished, `attempts` of them at most, in one
-// cooperative launch (k_rows_run, k_tiles_run); read_ctl undoes and switches
-// off a launch that gave up.  Returns false when the device does not take
-// the launch.
 static int *give_up_flag(mpci_prop *pr) { return &pr->ctl.p[2 * pr->P].status; }
 
 // What both persistent kernels are told of the propagator's run.
@@ -1836,6 +1839,10 @@ static bool begin_persistent(mpci_prop *pr, hipStream_t st, double2 *xb,
   return hipGetLastError() == hipSuccess;
 }
 
+// Attempts until the pulse has finished, `attempts` of them at most, in one
+// cooperative launch (k_rows_run, k_tiles_run); read_ctl undoes and switches
+// off a launch that gave up.  Returns false when the device does not take
+// the launch.
 static bool run_attempts_persistent(mpci_prop *pr, int attempts) {
   mpci_system *sys = pr->sys;
   if (!begin_persistent(pr, pr->stream, pr->xb.p,

@@ -695,11 +695,13 @@ template __global__ void k_rows_run<1, true>(RowRuns);
 // one stage after its readers have passed it) and of the step control's
 // per-workgroup maxima rb.
 //
-// What bounds it: up to about 80 MB, where nothing or little is streamed,
+// What bounds it: up to about 60 MB, where nothing or little is streamed,
 // the two exchanges and the polls (about 8 us a stage); past that the
-// streamed bytes, at 5.5 to 6 TB/s of the 6.9 TB/s that long reads reach
-// (the copies in registers and LDS, 76 MB over the device, are not read
-// again; the fill and drain of the ring and the exchanges are the rest).
+// streamed bytes, at 5.3 to 5.7 TB/s of the 6.9 TB/s that long reads reach
+// over the whole stage (the copies in registers and LDS, 50 to 59 MB over the
+// device, are not read again; the fill and drain of the ring and the exchanges
+// are the rest).  4000 x 4: 50.3 of 393.2 MB kept, 323 MB a stage fetched past
+// L2 by the counters.
 // Per attempt, against launches of k_gemv_tile and k_stage1: blocks 1500 x 4
 // (54 MB) 225 -> 127 us, 2000 x 4 (96 MB) 306 -> 181 us, blocks 2200, 2600,
 // 1800, 2400, 2000 355 against 482 us, 998 x 21 (159 MB) 473 -> 312 us,
