@@ -1773,16 +1773,19 @@ static int run_attempts_instrumented(mpci_prop *pr, int n) {
 
 // Attempts of one persistent launch.  It holds the compute units it runs on,
 // so that the work of other propagators, streams and processes waits for its
-// end: about 100 ms, 20 ms beside other members of a multi run.  A launch
-// costs about 0.1 ms more.  An attempt is taken for 13 sweeps of the dipoles at
-// 5.5 TB/s, 100 us at least (a row form's is 28 to 120 us for the pulses that
-// it holds at a time, however many these are).
+// end: about 100 ms, 20 ms beside other members of a multi run.  A further
+// launch costs 0.15 ms at most.  An attempt is taken for what the pulses of a
+// group cost it in turn (30 us at least: 30 for 198 x 4, 60 for 5 pulses on 300
+// x 6), however many sets of them there are, in tiles for 13 sweeps of the
+// dipoles at 5.5 TB/s (100 us at least: 127 for 1500 x 4, 763 for 4000 x 4).
 static int persistent_attempts(const mpci_prop *pr, bool shared) {
-  const double us = std::max(100.0, pr->rows ? 0.0 : 13 * 8e-6 / 5.5 *
-                                                         (double)pr->sys->S);
-  const int held = pr->rows_grp * pr->rows_slots;
-  const int passes = pr->rows ? (pr->P + held - 1) / held : 1;
-  const double n = (shared ? 20e3 : 100e3) / (us * passes);
+  double us = std::max(100.0, 13 * 8e-6 / 5.5 * (double)pr->sys->S);
+  if (pr->rows) {
+    const int held = pr->rows_grp * pr->rows_slots;
+    us = std::max(30.0, pr->rows_slots * row_pulse_us(pr->sys)) *
+         ((pr->P + held - 1) / held);
+  }
+  const double n = (shared ? 20e3 : 100e3) / us;
   return std::min(pr->logcap, std::max(16, (int)n));
 }
 
@@ -2400,7 +2403,7 @@ static int rows_together(std::vector<Member> &m) {
   }
   hipStream_t st = m[0].pr->stream;
   const int attempts =
-      std::max(16, (int)(100e3 / std::max(100.0, slowest)));
+      std::max(16, (int)(100e3 / std::max(30.0, slowest)));
   for (bool gave_up = false; !gave_up;) {
     RowRuns r{};
     std::vector<Member *> live;
